@@ -16,7 +16,8 @@
 //    valid samples cover every pixel of every frame exactly once;
 //  * the active-list chunks of both iterate kernels (every run length) for a
 //    range of list lengths: every entry read below the length, each entry taken
-//    once, and the claim ranges partitioning the chunks.
+//    once, the waves' own first chunks each taken once, and the claim ranges
+//    partitioning the chunks.
 // Test support, not part of the render path: built as its own library and called
 // from the CPU tests.
 #include <cstdarg>
@@ -346,6 +347,24 @@ long long nm_index_check(int nr, int nc, int nframes, int tile, int num_cu, int 
       next = hi;
     }
     if (next != nch) R.fail("claim ranges end at %u of %u chunks", next, nch);
+    // a launch's waves: their own first chunks and the claimed rest, each chunk once
+    for (const uint32_t grid : {1u, 2u, 7u, (uint32_t)num_cu * 4u})
+      for (const uint32_t wpw : {4u, 8u}) {
+        const uint32_t waves = grid * wpw, base = nch < waves ? nch : waves;
+        std::vector<uint8_t> first(nch, 0);
+        for (uint32_t b = 0; b < grid; b++)
+          for (uint32_t w = 0; w < wpw; w++) {
+            const uint32_t c = first_chunk(w, b, grid);
+            if (c < base && first[c]++) R.fail("chunk %u of %u is the first of two waves (grid %u)", c, nch, grid);
+            if (c < base && b >= base) R.fail("workgroup %u of %u leaves before its chunk %u", b, grid, c);
+          }
+        for (uint32_t c = 0; c < base; c++)
+          if (!first[c]) {
+            R.fail("chunk %u of %u is no wave's first (grid %u)", c, nch, grid);
+            break;
+          }
+        R.checked += base;
+      }
     // interleaved chunks: runs of 1 (plain), runs of 1 .. 64 (series: 64 is 64
     // consecutive entries); plant 3 interleaves the plain chunks with one too few
     for (uint32_t shift = 0; shift <= 7; shift++) {  // 7: the plain kernel's own chunk_pos

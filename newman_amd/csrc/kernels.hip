@@ -12,7 +12,6 @@
 //   hand[]          u64 per 64 samples: bit l = sample handed to the iteration
 //                   kernel (one word per wave and sample slot of the start kernels)
 //   state[]         per sample: delta (or z) and epsilon (or c), 4 x f64; it, m
-//   r2[]            |Y|^2 at the escape of iterated samples (smoothing input)
 //   active[]        u32 sample ids that iterate, compacted in sample order
 //   reference block Zd (the orbit as f64 pairs, Zd[0] = 0, padded past its end),
 //                   Xlo, A, B, C and the stop-search tables
@@ -36,8 +35,8 @@
 //               popcount ranks) from 64-sample chunks of active[], which waves
 //               claim from 8 claim ranges, with the next chunk prefetched (plain:
 //               its states; series: its ids); the series kernel keeps the orbit's head and
-//               tail windows in LDS
-//   finalize    smoothing of the iterated samples from r2
+//               tail windows in LDS; escaped samples wait in a queue per wave until 64
+//               are smoothed and stored together
 //   emit        tiled sample orders only: results into the row-major grids
 // Counters go to per-workgroup partial slots reduced on the device.
 // This file is compiled with -ffp-contract=off: the plain path must reproduce the
@@ -85,12 +84,11 @@ constexpr int kLdsHead = 1024, kLdsTail = 1024;
 // what the registers allow (8 per SIMD at 64 VGPRs: four workgroups, 128 KB).
 constexpr int kSeriesIterThreads = 512;
 static_assert(kLdsTail >= 64 && kLdsHead >= 64, "a block of up to 64 steps reads inside one window");
-constexpr int kPartSlots = 10240;       // per-workgroup partial counter slots
+constexpr int kPartSlots = 6144;        // per-workgroup partial counter slots
 
 // partial-slot ranges of the kernels of one render
 constexpr int kSlotStart = 0;
 constexpr int kSlotIter = 4096;
-constexpr int kSlotFinal = 6144;
 
 struct Common {
   const DevFrame* frames;
@@ -99,7 +97,6 @@ struct Common {
   double inv_frame;     // 1.0 / frame_size
   uint32_t total;
   EscapeValue* out;
-  double* r2;  // |z|^2 at the escape of iterated samples (per sample)
   double4* state;  // per sample: plain (x, y, cx, cy); series: (dr, di) as double2[]
   int2* state_i;   // per sample, series path: (it, m)
   uint64_t* hand;  // hand-on bits (hand_word)
@@ -805,6 +802,41 @@ __global__ __launch_bounds__(kThreads) void k_scatter(const uint64_t* hand, cons
   }
 }
 
+// ---- retirement -------------------------------------------------------------
+// An escaped sample's result waits in its wave's LDS queue until 64 have come
+// together; then every lane smooths and stores one.  The two logarithms (some 45
+// instructions) so run with all lanes busy, where at the escape itself they would
+// run for one or two lanes, and |z|^2 never goes through HBM (a pass of its own
+// over the iterated samples took 0.20-0.23 ms of the 33 M-sample frames).
+struct RetireEntry {
+  uint32_t pix;
+  int32_t it;
+  double r2;
+};
+constexpr int kRetireCap = 128;  // per wave: up to 63 waiting, 64 more pushed
+__device__ __forceinline__ void retire_flush(const Common& c, const RetireEntry* q, int from, int n,
+                                             unsigned long long& credited) {
+  __builtin_amdgcn_wave_barrier();
+  if (lane_id() < n) {
+    const RetireEntry e = q[from + lane_id()];
+    c.out[e.pix] = EscapeValue{e.it, smooth_of(e.r2, c)};
+    credited += (unsigned long long)e.it;
+  }
+  __builtin_amdgcn_wave_barrier();
+}
+// every lane calls it; qn (wave-uniform): entries waiting
+__device__ __forceinline__ void retire_push(const Common& c, RetireEntry* q, int& qn, bool esc, uint32_t pix, int it,
+                                            double r2, unsigned long long& credited) {
+  const unsigned long long w = __ballot(esc);
+  if (w == 0) return;
+  if (esc) q[qn + __popcll(w & ((1ull << lane_id()) - 1ull))] = RetireEntry{pix, it, r2};
+  qn += __popcll(w);
+  if (qn >= 64) {  // the last 64; the rest stay in front
+    qn -= 64;
+    retire_flush(c, q, qn, 64, credited);
+  }
+}
+
 // ---- work pipeline of a persistent wave -------------------------------------
 // A wave takes chunks of 64 entries of active[] (ChunkMap) by claims
 // (ChunkClaim).  Each lane holds one entry of the chunks in flight: CUR
@@ -833,17 +865,30 @@ __host__ __device__ inline uint32_t* scan_group_sums(unsigned long long* part) {
 constexpr uint32_t kNoChunk = 0xffffffffu;
 struct ChunkClaim {
   uint32_t* ctr;  // kQueues claim counters, kQueueStride apart
-  uint32_t nch;   // chunks
+  uint32_t nch;   // chunks left to claims: those past the waves' first
+  uint32_t base;  // the first of them
   uint32_t home;  // wave-uniform: the range claimed from
   uint32_t done;  // wave-uniform: ranges found empty
+  // every wave's first chunk is its own (first()); the claims share the rest.  When
+  // there are no more chunks than waves no wave touches a counter: 4096 waves that
+  // each asked 8 empty ranges had taken most of a small frame's 56 us here.
   __device__ void init(unsigned long long* part, uint32_t chunks) {
     ctr = (uint32_t*)(part + (size_t)kPartSlots * C_COUNT);
-    nch = chunks;
+    const uint32_t waves = gridDim.x * (blockDim.x >> 6);
+    base = min(chunks, waves);
+    nch = chunks - base;
     home = blockIdx.x & (kQueues - 1);
-    done = 0;
+    done = nch ? 0u : (1u << kQueues) - 1u;
+  }
+  // the wave's own chunk: a launch with fewer chunks than waves spreads them over
+  // its workgroups (base is then the chunk count)
+  __device__ __forceinline__ uint32_t first() const {
+    const uint32_t w = first_chunk(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6), blockIdx.x, gridDim.x);
+    return w < base ? w : kNoChunk;
   }
   // the next chunk, or kNoChunk when every range is empty
   __device__ __forceinline__ uint32_t next() {
+    if (done == (1u << kQueues) - 1u) return kNoChunk;
     for (int t = 0; t < kQueues; t++) {
       const uint32_t h = (home + (uint32_t)t) & (kQueues - 1);
       if (done & (1u << h)) continue;
@@ -853,7 +898,7 @@ struct ChunkClaim {
       v = __builtin_amdgcn_readfirstlane(v);
       if (v < hi - lo) {
         home = h;
-        return lo + v;
+        return base + lo + v;
       }
       done |= 1u << h;
     }
@@ -926,7 +971,7 @@ __device__ __forceinline__ void plain_block(PlainLane& L, const double b2) {
 }
 
 template <int K, bool FMA2, bool GROUPED>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_plain_iterate(
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_plain_iterate(
     PlainArgs a) {
   const Common& c = a.c;
   const uint32_t total = *c.nactive;
@@ -934,7 +979,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(8, 8))
   cm.init(total);
   ChunkClaim q;
   q.init(c.part, cm.nch);
-  const uint32_t c0 = q.next(), c1 = q.next(), c2 = q.next();
+  __shared__ RetireEntry retire[kThreads / 64][kRetireCap];
+  RetireEntry* const rq = retire[threadIdx.x >> 6];
+  int rn = 0;
+  unsigned long long credited = 0;
+  const uint32_t c0 = q.first(), c1 = q.next(), c2 = q.next();
   uint32_t ncur = cm.items(c0), nnext = cm.items(c1), nfar = cm.items(c2);
   uint32_t cur_pix = cm.pix(c.active, c0, ncur), nxt_pix = cm.pix(c.active, c1, nnext);
   uint32_t far_pix = cm.pix(c.active, c2, nfar);
@@ -991,24 +1040,28 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(8, 8))
     double mgesc = 0.0;
     PlainLane L{x, y, r2, i2, cx, cy, act, jesc, mgesc};
     plain_block<0, K, GROUPED ? kIterGroup : 1, FMA2>(L, c.b2);
+    bool esc = false;
     if (was) {
       // the reference tests k >= N before each update: an escape at k0 + j
       // counts only below N, and a sample that reaches N in the block ends there
       const int ran = jesc >= 0 ? jesc + 1 : K;
       if (k0 + ran > N || (jesc < 0 && k0 + K == N)) {
         c.out[pix] = EscapeValue{N, 0.0f};
+        credited += (unsigned long long)N;
         act = false;
         park(x, y, r2, i2, cx, cy);
-      } else if (jesc >= 0) {
-        c.out[pix] = EscapeValue{k0 + jesc, 0.0f};
-        c.r2[pix] = mgesc;  // smoothing: k_finalize
+      } else {
+        esc = jesc >= 0;
       }
       executed += (unsigned long long)min(ran, N - k0);
       k = k0 + K;
     }
+    retire_push(c, rq, rn, esc, pix, k0 + jesc, mgesc, credited);
   }
-  const int idx[1] = {C_EXECUTED};
-  block_partial(c.part, kSlotIter + blockIdx.x, &executed, idx, 1);
+  retire_flush(c, rq, 0, rn, credited);
+  const unsigned long long v[2] = {executed, credited};
+  const int idx[2] = {C_EXECUTED, C_CREDITED};
+  block_partial(c.part, kSlotIter + blockIdx.x, v, idx, 2);
 }
 
 // =============================================================== series path
@@ -1651,12 +1704,21 @@ __device__ __forceinline__ void pert_block_fx(float& wr, float& wi, int& ex, flo
 // their objects in scratch and spilled the LDS head pointer, reloaded in the
 // step loop's rebase branch): no scratch at all.
 template <int K, bool FX>
-__global__ __launch_bounds__(kSeriesIterThreads) __attribute__((amdgpu_waves_per_eu(FX || K < 16 ? 1 : 8, 8)))
+__global__ __launch_bounds__(kSeriesIterThreads) __attribute__((amdgpu_waves_per_eu(4, 8)))
 void k_series_iterate(SeriesArgs a) {
   const Common& c = a.c;
   const uint32_t total = *c.nactive;
   uint32_t executed = 0, rebased = 0;  // per lane (< 2^32 steps per lane per launch)
   const int N = c.N, mend = a.mend;
+  ChunkMap cm;
+  cm.init(total, a.run_shift);
+  ChunkClaim q;
+  q.init(c.part, cm.nch);
+  if (blockIdx.x >= q.base) return;  // no chunk for any wave of the workgroup
+  __shared__ RetireEntry retire[kSeriesIterThreads / 64][kRetireCap];
+  RetireEntry* const rq = retire[threadIdx.x >> 6];
+  int rn = 0;
+  unsigned long long credited = 0;
   // the orbit's tail and head windows (zlds[t] = Zd[tail_lo + t],
   // zlds[kLdsTail + h] = Zd[h] for h < kLdsHead); entries past Zd's allocation
   // read 0.  The head sits above 16 K positions so that a rebased lane's base
@@ -1670,11 +1732,7 @@ void k_series_iterate(SeriesArgs a) {
   }
   __syncthreads();
   const double2* zhead = zlds + kLdsTail;  // rebased lanes read the orbit from its start
-  ChunkMap cm;
-  cm.init(total, a.run_shift);
-  ChunkClaim q;
-  q.init(c.part, cm.nch);
-  const uint32_t c0 = q.next(), c1 = q.next();
+  const uint32_t c0 = q.first(), c1 = q.next();
   uint32_t ncur = cm.items(c0), nnext = cm.items(c1);
   uint32_t cur_pix = cm.pix(c.active, c0, ncur), nxt_pix = cm.pix(c.active, c1, nnext);
   const double2* dstate = (const double2*)c.state;  // the series start's deltas
@@ -1813,25 +1871,26 @@ void k_series_iterate(SeriesArgs a) {
         kdone = pert_block<K, false>(dr, di, er, ei, m, it, fz, fhead, 0, mend, c.b2, !act, can_refill, esc,
                                      esc_r2, rb);
     }
+    bool escaped = false;
     if (act) {
       it = it0 + kdone;
-      const bool escaped = esc >= 0 && esc <= N - 1;
+      escaped = esc >= 0 && esc <= N - 1;
       executed += escaped ? (unsigned)(esc - it0 + 1) : (unsigned)min(kdone, N - it0);
       rebased += rb;
-      if (escaped || it >= N) {  // tops up to N-1 decided
-        c.out[pix] = EscapeValue{escaped ? esc : N, 0.0f};
-        if (escaped) c.r2[pix] = esc_r2;  // smoothing: k_finalize
-        act = false;
+      if (!escaped && it >= N) {  // tops up to N-1 decided
+        c.out[pix] = EscapeValue{N, 0.0f};
+        credited += (unsigned long long)N;
       }
+      act = !escaped && it < N;
     }
+    retire_push(c, rq, rn, escaped, pix, esc, esc_r2, credited);
   }
-  const unsigned long long v[2] = {executed, rebased};
-  const int idx[2] = {C_EXECUTED, C_REBASED};
-  block_partial(c.part, kSlotIter + blockIdx.x, v, idx, 2);
+  retire_flush(c, rq, 0, rn, credited);
+  const unsigned long long v[3] = {executed, rebased, credited};
+  const int idx[3] = {C_EXECUTED, C_REBASED, C_CREDITED};
+  block_partial(c.part, kSlotIter + blockIdx.x, v, idx, 3);
 }
 
-// smoothing of the iterated samples (mandelbrot.cpp:133-136), converged: one
-// thread per entry of active[]
 // tiled sample order: results (sample order) -> the row-major grids
 __global__ __launch_bounds__(kThreads) void k_emit(Common c, EscapeValue* grid) {
   // 64-bit loop index: a total near 2^32 must not wrap the stride
@@ -1841,38 +1900,6 @@ __global__ __launch_bounds__(kThreads) void k_emit(Common c, EscapeValue* grid) 
     const Loc lc = locate(f, gid - f.sample_base);
     if (lc.valid) grid[f.out_base + (uint64_t)lc.r * f.nc + lc.c] = c.out[gid];
   }
-}
-
-constexpr int kFinalizePer = 8;
-__global__ __launch_bounds__(kThreads) void k_finalize(Common c) {
-  const uint32_t total = *c.nactive;
-  const uint32_t stride = gridDim.x * blockDim.x;
-  unsigned long long credited = 0;  // the iterated samples' counts (the start kernel adds the rest)
-  // kFinalizePer samples per thread per round, their loads issued together
-  // (64-bit entry indices: a total near 2^32 must not wrap the stride)
-  for (uint64_t i = blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (uint64_t)kFinalizePer * stride) {
-    uint32_t pix[kFinalizePer];
-    int it[kFinalizePer];
-    double r2[kFinalizePer];
-#pragma unroll
-    for (int k = 0; k < kFinalizePer; k++) {
-      const uint64_t e = i + (uint64_t)k * stride;
-      pix[k] = e < total ? c.active[e] : c.total;
-    }
-#pragma unroll
-    for (int k = 0; k < kFinalizePer; k++) {
-      it[k] = pix[k] < c.total ? c.out[pix[k]].iterations : c.N;
-      r2[k] = pix[k] < c.total ? c.r2[pix[k]] : 0.0;
-    }
-#pragma unroll
-    for (int k = 0; k < kFinalizePer; k++) {
-      if (pix[k] >= c.total) continue;
-      credited += (unsigned long long)it[k];
-      if (it[k] < c.N) c.out[pix[k]].smoothing = smooth_of(r2[k], c);
-    }
-  }
-  const int idx[1] = {C_CREDITED};
-  block_partial(c.part, kSlotFinal + blockIdx.x, &credited, idx, 1);
 }
 
 // ============================================================ grid utilities
@@ -1939,14 +1966,13 @@ constexpr int iter_threads() { return kThreads; }
 template <>
 constexpr int iter_threads<SeriesArgs>() { return kSeriesIterThreads; }
 
-// workgroups of the tile kernels (start, scatter, finalize, emit)
+// workgroups of the tile kernels (start, scatter, emit)
 static int tile_grid(uint64_t total, int num_cu) {
   return start_grid(total, num_cu, (uint64_t)(kSlotIter - kSlotStart));
 }
 
 // The kernels of one pass on `stream`: zero the counters (part: kPartWords
-// words), start, scan, scatter, iterate, finalize (and emit for tiled sample
-// orders).  evs != nullptr records an event before each stage (eager timing);
+// words), start, scan, scatter, iterate (and emit for tiled sample orders).  evs != nullptr records an event before each stage (eager timing);
 // under stream capture it is null.  Returns the first launch error.
 template <class Args, class StartFn, class IterFn>
 static hipError_t launch_pass_on(hipStream_t stream, int num_cu, unsigned long long* part, uint32_t* nactive,
@@ -1957,7 +1983,7 @@ static hipError_t launch_pass_on(hipStream_t stream, int num_cu, unsigned long l
   const int gtile = tile_grid(c.total, num_cu);
   // waves = persistent waves per SIMD: 4 per CU for each 256 threads
   const int ti = iter_threads<Args>();
-  const int giter = std::max(1, std::min(num_cu * waves * 256 / ti, kSlotFinal - kSlotIter));
+  const int giter = std::max(1, std::min(num_cu * waves * 256 / ti, kPartSlots - kSlotIter));
   hipError_t e;
 #define NM_LAUNCH_OK(expr)                   \
   do {                                       \
@@ -1979,8 +2005,6 @@ static hipError_t launch_pass_on(hipStream_t stream, int num_cu, unsigned long l
   if (evs && (e = hipEventRecord(evs[2], stream)) != hipSuccess) return e;
   NM_LAUNCH_OK(hipLaunchKernelGGL(iter, dim3(giter), dim3(ti), 0, stream, args));
   if (evs && (e = hipEventRecord(evs[3], stream)) != hipSuccess) return e;
-  static_assert(kPartSlots - kSlotFinal >= kSlotIter - kSlotStart, "finalize runs on the start grid");
-  NM_LAUNCH_OK(hipLaunchKernelGGL(k_finalize, dim3(gtile), dim3(kThreads), 0, stream, c));
   if (emit_to) NM_LAUNCH_OK(hipLaunchKernelGGL(k_emit, dim3(gtile), dim3(kThreads), 0, stream, c, emit_to));
   if (evs && (e = hipEventRecord(evs[4], stream)) != hipSuccess) return e;
 #undef NM_LAUNCH_OK
@@ -2012,7 +2036,6 @@ class EngineImpl : public Engine {
   void* d_mask = nullptr; size_t n_mask_bytes = 0;
   void* d_out = nullptr; size_t n_out_bytes = 0;
   void* d_hand = nullptr; size_t n_hand_bytes = 0;
-  void* d_r2 = nullptr; size_t n_r2_bytes = 0;
   void* d_tiles = nullptr; size_t n_tiles_bytes = 0;
   void* d_active = nullptr; size_t n_active_bytes = 0;
   void* d_state = nullptr; size_t n_state_bytes = 0;
@@ -2185,7 +2208,6 @@ class EngineImpl : public Engine {
     int st;
     if ((st = grow(&d_out, &n_out_bytes, total * sizeof(EscapeValue)))) return st;
     if ((st = grow(&d_hand, &n_hand_bytes, (uint64_t)hand_words((uint32_t)total) * 8))) return st;
-    if ((st = grow(&d_r2, &n_r2_bytes, total * 8))) return st;
     if ((st = grow(&d_state, &n_state_bytes, total * sizeof(double4)))) return st;
     if ((st = grow(&d_state_i, &n_state_i_bytes, total * sizeof(int2)))) return st;
     if ((st = grow(&d_tiles, &n_tiles_bytes, ntiles * 4))) return st;
@@ -2193,7 +2215,6 @@ class EngineImpl : public Engine {
     c.frames = (const DevFrame*)d_frames;
     c.total = (uint32_t)total;
     c.out = (EscapeValue*)d_out;
-    c.r2 = (double*)d_r2;
     c.state = (double4*)d_state;
     c.state_i = (int2*)d_state_i;
     c.hand = (uint64_t*)d_hand;
@@ -2779,7 +2800,7 @@ constexpr size_t na_align(size_t b) { return (b + 255) & ~(size_t)255; }
 // bytes of the layout for n samples on an nr x nc frame (noalloc_layout)
 constexpr size_t na_bytes(uint64_t n, uint64_t nr, uint64_t nc) {
   return na_align((2 * nc + 2 * nr) * sizeof(double)) + na_align(sizeof(DevFrame)) +
-         na_align(n * sizeof(EscapeValue)) + na_align(n * sizeof(double)) + na_align(n * sizeof(double4)) +
+         na_align(n * sizeof(EscapeValue)) + na_align(n * sizeof(double4)) +
          na_align((n + kTile - 1) / kTile * kHandWordsPerTile * 8) + na_align((n + kTile - 1) / kTile * 4) +
          na_align(n * 4) +
          na_align((size_t)kPartWords * sizeof(unsigned long long)) + na_align(4);
@@ -2861,7 +2882,6 @@ int render_hw_noalloc(const HwFrameView& f, int N, double bailout, EscapeValue* 
   double* tabs = (double*)take((2 * (size_t)f.nc + 2 * (size_t)f.nr) * sizeof(double));
   DevFrame* frame = (DevFrame*)take(sizeof(DevFrame));
   EscapeValue* out = (EscapeValue*)take(n * sizeof(EscapeValue));
-  double* r2 = (double*)take(n * sizeof(double));
   double4* state = (double4*)take(n * sizeof(double4));
   uint64_t* hand = (uint64_t*)take((size_t)hand_words((uint32_t)n) * 8);
   uint32_t* tiles = (uint32_t*)take((n + kTile - 1) / kTile * 4);
@@ -2896,7 +2916,6 @@ int render_hw_noalloc(const HwFrameView& f, int N, double bailout, EscapeValue* 
   c.inv_frame = 1.0 / (double)n;
   c.total = (uint32_t)n;
   c.out = out;
-  c.r2 = r2;
   c.state = state;
   c.state_i = nullptr;  // the plain path keeps no per-sample count
   c.hand = hand;

@@ -149,7 +149,12 @@ __host__ __device__ inline uint32_t chunk_pos_run(uint32_t lane, uint32_t c, uin
 __host__ __device__ inline uint32_t chunk_pos(uint32_t lane, uint32_t c, uint32_t nch) {
   return chunk_pos_run(lane, c, nch, 0);
 }
-// the chunks of claim range h: [claim_lo(nch, h), claim_lo(nch, h + 1))
+// The first chunks are the waves' own: wave w of workgroup b (grid workgroups)
+// takes chunk w grid + b when that is below min(nch, waves), so that a launch with
+// fewer chunks than waves spreads them over its workgroups; the chunks from
+// min(nch, waves) on are claimed, in kQueues ranges.
+__host__ __device__ inline uint32_t first_chunk(uint32_t w, uint32_t b, uint32_t grid) { return w * grid + b; }
+// the claimed chunks of range h, of `nch` in all: [claim_lo(nch, h), claim_lo(nch, h + 1))
 __host__ __device__ inline uint32_t claim_lo(uint32_t nch, uint32_t h) {
   return (uint32_t)((uint64_t)nch * h / kQueues);
 }

@@ -1,0 +1,38 @@
+"""Escaped samples leave the iterate kernels through a queue per wave that is
+smoothed 64 at a time: list lengths around a wave and a queue, on both paths,
+against the oracle.  At the plain view every sample outlives the start kernel."""
+import json
+import os
+
+import numpy as np
+import pytest
+
+import oracle_lib as O
+
+pytestmark = pytest.mark.gpu
+
+_T13 = json.load(open(os.path.join(os.path.dirname(__file__), "golden", "views.json")))["t13"]
+
+
+def _check(g, want):
+    assert np.array_equal(g["iterations"], want["iterations"])
+    a, b = g["smoothing"].astype(np.float64), want["smoothing"].astype(np.float64)
+    assert (np.abs(a - b) <= 1e-6 * np.maximum(np.abs(b), 1.0)).all()
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 127, 128, 129, 4097])
+@pytest.mark.parametrize("deep", [False, True])
+def test_queue_lengths(gpu, n, deep):
+    m, o = gpu.Mandelbrot(1, n), O.OView(1, n)
+    view = (_T13["N"], _T13["re"], _T13["im"], "1e-24") if deep else (900, "-0.7453", "0.1127", "0.01")
+    m.set_view(*view)
+    o.set_view(*view)
+    if deep:
+        m.precompute()
+        o.precompute_at(*m.reference_point())
+    st = m.render()
+    rc = np.array([(0, c) for c in range(n)], dtype=np.int32)
+    want = o.render_samples(rc, pert=True) if deep else o.render_rows(np.zeros(1, dtype=np.int32))[0]
+    _check(m.grid()[0], want)
+    # cardioid and bulb samples are counted apart from credited work
+    assert st["credited"] == int(want["iterations"].astype(np.int64).sum()) - st["n_cardioid"] * view[0]
