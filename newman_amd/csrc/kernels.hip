@@ -24,7 +24,8 @@
 //   *_start     tiles of 1024 samples: cardioid/bulb test and up to pre_iter
 //               updates (plain path), or the reference's per-sample series start
 //               (series path: stop index, series skip, escape inside the skip,
-//               first step); resolves what it can, marks the rest (one ballot
+//               first step, and with FP64 deltas the steps a wave's samples can do
+//               together); resolves what it can, marks the rest (one ballot
 //               word per wave), counts per tile
 //   scan        exclusive scan of the tile counts (range totals, then each
 //               range's scan from the earlier ranges' sum; up to 64 workgroups)
@@ -75,10 +76,10 @@ enum CounterIdx {
 
 constexpr int kHead = 64;               // orbit padding past its end (>= max K)
 // orbit windows each iterate workgroup keeps in LDS: the head (where rebased
-// lanes live) and the tail (where samples that never rebased run out the
+// lanes live) and the tail (where samples that have not rebased yet run out the
 // reference); lanes whose block fits a window read it from LDS, the others
 // gather from global memory, whose cache tag lookups bound the gathers
-constexpr int kLdsHead = 1024, kLdsTail = 1024;
+constexpr int kLdsTail = 1024, kLdsHead = 3040;
 // The series iterate kernel runs 8 waves per workgroup: the 32 KB of LDS orbit
 // windows is shared by 8 waves, so LDS does not cap the waves a CU holds below
 // what the registers allow (8 per SIMD at 64 VGPRs: four workgroups, 128 KB).
@@ -158,6 +159,8 @@ struct SeriesArgs {
   const int2 *Ae, *Be, *Ce;
   int fxs;
   uint32_t run_shift;  // active-list chunks (ChunkMap): runs of 2^run_shift entries
+  double* safe;        // safe radius per orbit index (safe_radius); null: no coherent phase (FP32X deltas)
+  double emax, radius;  // what the radii hold for: |e| of every sample, the bailout
 };
 
 // ------------------------------------------------------------ device helpers
@@ -1379,15 +1382,173 @@ __global__ __launch_bounds__(64) void k_tile_skip(SeriesArgs a, const int2* prob
   }
 }
 
+// ---- the coherent phase -----------------------------------------------------
+// Until a sample first rebases it sits at the orbit index its skip left it at plus
+// the steps done since, so the 64 neighbours of a wave read one and the same orbit
+// entry, and its delta is far below the orbit's magnitude on most steps: no rebase
+// (|Z + d| < |d|) and no escape can happen there, which a bound on the growth of
+// |d| proves ahead for kCoh steps at a time.  Such a step is its 8 FP64
+// instructions (Z + d, Z + Y, d W + e) with the orbit entry in scalar registers,
+// where a step of the iterate kernel is 15 and the handlers of the lanes around
+// it, with the entry loaded per lane.  54% of the continuation steps of the 1e-30
+// view lie before the sample's first rebase, 75% of the 1e-40 view's, 91% of a
+// 1e-25 view's, 19% of the 1e-100 view's.
+constexpr int kCoh = 8;  // steps per block
+// Leave the phase when fewer lanes than this still take part: a wave-step costs
+// the same for any number of lanes, about 9 instruction slots with the proof and 16
+// without, against some 20 per lane-step / 64 in the iterate kernel.
+constexpr int kCohQuiet = 20, kCohChecked = 36;
+constexpr int kCohSpread = 64;  // lanes whose skip ended further back than this are handed on at once
+
+// safe[i]: with max(|dr|, |di|) <= safe[i] and |e| <= emax, none of the steps at
+// orbit indices i .. i + kCoh - 1 can rebase, escape or meet the orbit's end.  A
+// step at index k is sure of that for |d| <= rho(k) = min(0.49 |Z_k|, 0.99 R -
+// |Z_k|): then |Y| >= |Z_k| - |d| > 1.04 |d| and |Y| < 0.99 R, far beyond the
+// rounding of the computed tests (|Z_k| >= 2^-400 keeps their squares normal).  From |d|
+// <= r the next delta is at most r (2 |Z_k| + r) + emax, so r is sure of the rest
+// of the block when that is at most the next index's radius t + emax: r = t /
+// (|Z_k| + sqrt(|Z_k|^2 + t)), taken backwards from the block's last step.  The
+// table is in the max norm (a factor sqrt 2, rounded down).
+__device__ __forceinline__ double safe_rho(const double2* Zd, int k, int mend, double radius, double* az) {
+  const double2 z = Zd[k];
+  const double q = sqrt(z.x * z.x + z.y * z.y);
+  *az = q;
+  if (k >= mend || !(q >= 0x1p-400)) return 0.0;
+  return fmax(0.0, fmin(0.49 * q, 0.99 * radius - q));
+}
+__device__ __forceinline__ void safe_radius(const double2* Zd, int mend, double radius, double emax, double* safe,
+                                            int i) {
+  double s = 0.0;
+  if (i + kCoh <= mend) {
+    double az;
+    double rho = safe_rho(Zd, i + kCoh - 1, mend, radius, &az);
+    for (int j = kCoh - 2; j >= 0; j--) {
+      const double own = safe_rho(Zd, i + j, mend, radius, &az);
+      const double t = rho - emax;
+      rho = t > 0.0 ? fmin(own, t / (az + sqrt(az * az + t)) * (1.0 - 1e-9)) : 0.0;
+    }
+    s = rho * 0.7071067;
+  }
+  safe[i] = s;
+}
+
+// an orbit entry at a wave-uniform index, through the constant address space (the
+// orbit is written before the launch): scalar loads
+__device__ __forceinline__ double2 uniform_orbit(const double2* Zd, int i) {
+#if __HIP_DEVICE_COMPILE__
+  typedef __attribute__((address_space(4))) const double ConstDouble;
+  const ConstDouble* p = (const ConstDouble*)(Zd + i);
+  return make_double2(p[0], p[1]);
+#else
+  return Zd[i];
+#endif
+}
+__device__ __forceinline__ double uniform_safe(const double* safe, int i) {
+#if __HIP_DEVICE_COMPILE__
+  typedef __attribute__((address_space(4))) const double ConstDouble;
+  return ((const ConstDouble*)safe)[i];
+#else
+  return safe[i];
+#endif
+}
+
+// The coherent phase of a wave's 64 samples (every lane calls it): lanes with
+// `want` hold a state (d, it, m) to be handed on, and those that have not rebased
+// (m = it + 1) step along the orbit together.  A lane whose rebase test holds does
+// that step and leaves with the state behind it (m = 1); one whose escape test
+// holds leaves with the state before it, and the iterate kernel decides it.  Every
+// step done is the iterate kernel's, operation for operation.  (Going on with the
+// lanes of a common rebase from the orbit's start was slower: 3.2 -> 3.4 ms a pass
+// of the 1e-30 view, 5.2 -> 6.0 ms of the 1e-100 view, whose lanes part too soon.)
+__device__ __forceinline__ void coherent_phase(const SeriesArgs& a, const bool want, double& dr, double& di,
+                                               const double2 e, int& it, int& m) {
+  const Common& c = a.c;
+  bool act = want && m == it + 1;
+  if (__popcll(__ballot(act)) < kCohChecked) return;
+  int top = act ? m : 0;  // the largest index of the wave: the others step up to it
+  for (int off = 32; off > 0; off >>= 1) top = max(top, __shfl_xor(top, off));
+  int mu = __builtin_amdgcn_readfirstlane(top);
+  act = act && mu - m <= kCohSpread;
+  while (__ballot(act && m < mu) != 0) {
+    if (act && m < mu) {
+      const double2 z = a.Zd[m];
+      const double yr = z.x + dr, yi = z.y + di;
+      const double r2 = yr * yr + yi * yi;
+      const double dmag = fma(dr, dr, di * di);
+      if (r2 < dmag || r2 > c.b2) {
+        act = false;
+      } else {
+        const double wr = z.x + yr, wi = z.y + yi;
+        const double nr = fma(dr, wr, fma(-di, wi, e.x));
+        di = fma(dr, wi, fma(di, wr, e.y));
+        dr = nr;
+        m++;
+        it++;
+      }
+    }
+  }
+  double xr = dr, xi = di;  // the walking lanes' delta; dr, di keep what a lane left with
+  unsigned long long live = __ballot(act);
+  for (;;) {
+    const int n = __popcll(live);
+    // it = m - 1 on every walking lane: the block must end below N
+    if (n < kCohQuiet || mu + kCoh > a.mend || mu - 1 + kCoh >= c.N) break;
+    const double s = uniform_safe(a.safe, mu);
+    double2 zs[kCoh];
+#pragma unroll
+    for (int j = 0; j < kCoh; j++) zs[j] = uniform_orbit(a.Zd, mu + j);
+    if (((__ballot(!(fabs(xr) <= s)) | __ballot(!(fabs(xi) <= s))) & live) == 0) {
+#pragma unroll
+      for (int j = 0; j < kCoh; j++) {
+        const double2 z = zs[j];
+        const double wr = z.x + (z.x + xr), wi = z.y + (z.y + xi);
+        const double nr = fma(xr, wr, fma(-xi, wi, e.x));
+        xi = fma(xr, wi, fma(xi, wr, e.y));
+        xr = nr;
+      }
+    } else {
+      if (n < kCohChecked) break;
+#pragma unroll
+      for (int j = 0; j < kCoh; j++) {
+        const double2 z = zs[j];
+        const double yr = z.x + xr, yi = z.y + xi;
+        const double r2 = yr * yr + yi * yi;
+        const double dmag = fma(xr, xr, xi * xi);
+        const unsigned long long out = __ballot(r2 > c.b2) & live, reb = __ballot(r2 < dmag) & live & ~out;
+        if (__builtin_expect((out | reb) != 0, 0)) {
+          live &= ~(out | reb);
+          if (((out | reb) >> lane_id()) & 1ull) {
+            const bool r = (reb >> lane_id()) & 1ull;
+            dr = r ? fma(yr, yr, fma(-yi, yi, e.x)) : xr;
+            di = r ? fma(yr, yi, fma(yi, yr, e.y)) : xi;
+            m = r ? 1 : mu + j;
+            it = mu + j - (r ? 0 : 1);
+          }
+        }
+        const double wr = z.x + yr, wi = z.y + yi;
+        const double nr = fma(xr, wr, fma(-xi, wi, e.x));
+        xi = fma(xr, wi, fma(xi, wr, e.y));
+        xr = nr;
+      }
+    }
+    mu += kCoh;
+  }
+  if ((live >> lane_id()) & 1ull) {
+    dr = xr;
+    di = xi;
+    m = mu;
+    it = mu - 1;
+  }
+}
+
 // The series start kernel: per sample the reference's series start
-// (mandelbrot.cpp:144-206) and the first perturbation step; samples that need
-// more are flagged for the iterate kernel.  Held to 80 VGPRs (6 waves per SIMD):
-// 5% less time than at its natural 89 (5 waves) where the stop search dominates.
-// FXS: the series test and skip in floatexp.
-template <bool FXS>
+// (mandelbrot.cpp:144-206) and the first perturbation step, then (COH: FP64
+// deltas) the coherent phase; samples that need more are flagged for the iterate
+// kernel.  FXS: the series test and skip in floatexp.
+template <bool FXS, bool COH>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_series_start(SeriesArgs a) {
   const Common& c = a.c;
-  unsigned long long ncard = 0, nres = 0, skipped = 0, credited = 0;
+  unsigned long long ncard = 0, nres = 0, skipped = 0, credited = 0, executed = 0;
   const uint32_t ntiles = start_tiles(c.total);
   for (uint32_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
     uint32_t mine = 0;
@@ -1424,6 +1585,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(6, 8))
       }
       // phase 3 (valid lanes): the reference's series start for this sample
       bool want = false;
+      double ndr = 0.0, ndi = 0.0;  // the handed-on delta, iteration and orbit index
+      int hit = 0, hm = 0;
       if (valid) {
         EscapeValue res{c.N, 0.0f};
         if (in) {
@@ -1489,11 +1652,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(6, 8))
               wi = pi;
               m = 0;
             }
-            double ndr = fma(dr, wr, fma(-di, wi, e.x));
-            double ndi = fma(dr, wi, fma(di, wr, e.y));
-            // the delta only: the iterate kernel reads epsilon from the tables
-            ((double2*)c.state)[gid] = make_double2(ndr, ndi);
-            c.state_i[gid] = make_int2(found + 1, m + 1);
+            ndr = fma(dr, wr, fma(-di, wi, e.x));
+            ndi = fma(dr, wi, fma(di, wr, e.y));
+            hit = found + 1;
+            hm = m + 1;
             want = true;
             skipped += (unsigned long long)(found + 1);
           } else {
@@ -1503,13 +1665,23 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(6, 8))
         if (!want) c.out[gid] = res;
         if (!want && !in) credited += (unsigned long long)res.iterations;
       }
+      if constexpr (COH) {
+        const int it0 = hit;
+        coherent_phase(a, want, ndr, ndi, e, hit, hm);
+        executed += (unsigned long long)(hit - it0);
+      }
+      if (want) {
+        // the delta only: the iterate kernel reads epsilon from the tables
+        ((double2*)c.state)[gid] = make_double2(ndr, ndi);
+        c.state_i[gid] = make_int2(hit, hm);
+      }
       mine += store_hand(c.hand, gid, want);
     }
     tile_count_add(c.tile_count, tile, mine);
   }
-  const unsigned long long v[4] = {ncard, nres, skipped, credited};
-  const int idx[4] = {C_CARDIOID, C_SA_RES, C_SKIPPED, C_CREDITED};
-  block_partial(c.part, kSlotStart + blockIdx.x, v, idx, 4);
+  const unsigned long long v[5] = {ncard, nres, skipped, credited, executed};
+  const int idx[5] = {C_CARDIOID, C_SA_RES, C_SKIPPED, C_CREDITED, C_EXEC_START};
+  block_partial(c.part, kSlotStart + blockIdx.x, v, idx, COH ? 5 : 4);
 }
 
 // epsilon of sample gid (its pixel's offset from the reference point), from the
@@ -1696,13 +1868,23 @@ __device__ __forceinline__ void pert_block_fx(float& wr, float& wi, int& ex, flo
 // FP64 (FX = false) or FP32X (FX = true) perturbation with rebasing (replaces the
 // HP continuation of mandelbrot.cpp:209-224).  Persistent waves, lanes refilled
 // from 64-sample chunks; blocks of K steps, each lane reading the orbit through
-// its own cursor into the workgroup's LDS windows or HBM.  The FP64 kernel is
-// held to 64 VGPRs (8 waves per SIMD, four 512-thread workgroups per CU): only
-// the next chunk's sample ids are prefetched, its states are loaded when it
-// becomes current (a wave waits one load per 64 refills, while the other waves
-// of its SIMD run).  The chunk map and claims are inlined (as calls they kept
+// its own cursor into the workgroup's LDS windows or HBM.  Only the next chunk's
+// sample ids are prefetched, its states are loaded when it becomes current (a wave
+// waits one load per 64 refills, while the other waves of its SIMD run).  The chunk map and claims are inlined (as calls they kept
 // their objects in scratch and spilled the LDS head pointer, reloaded in the
 // step loop's rebase branch): no scratch at all.
+// A workgroup's LDS: the waves' retire queues and the orbit windows (tail[t] =
+// Zd[tail_lo + t], head[h] = Zd[h]).  Half a CU's 160 KB, for the two workgroups a
+// CU holds by default (4 waves per SIMD); of static size, so that a rebase's base
+// address is a literal (from a register it was one of 64 spilled ones, +18% time on
+// the 1e-30 view).  The head sits above 16 K positions so that a rebased lane's
+// base address (head - 16 j) stays non-negative.
+struct SeriesLds {
+  RetireEntry retire[kSeriesIterThreads / 64][kRetireCap];
+  double2 tail[kLdsTail];
+  double2 head[kLdsHead];
+};
+static_assert(2 * (sizeof(SeriesLds) + 256) <= 160 * 1024, "two workgroups per CU");
 template <int K, bool FX>
 __global__ __launch_bounds__(kSeriesIterThreads) __attribute__((amdgpu_waves_per_eu(4, 8)))
 void k_series_iterate(SeriesArgs a) {
@@ -1715,23 +1897,20 @@ void k_series_iterate(SeriesArgs a) {
   ChunkClaim q;
   q.init(c.part, cm.nch);
   if (blockIdx.x >= q.base) return;  // no chunk for any wave of the workgroup
-  __shared__ RetireEntry retire[kSeriesIterThreads / 64][kRetireCap];
-  RetireEntry* const rq = retire[threadIdx.x >> 6];
+  // entries past Zd's allocation read 0
+  __shared__ SeriesLds lds;
+  RetireEntry* const rq = lds.retire[threadIdx.x >> 6];
+  double2* const zlds = lds.tail;
   int rn = 0;
   unsigned long long credited = 0;
-  // the orbit's tail and head windows (zlds[t] = Zd[tail_lo + t],
-  // zlds[kLdsTail + h] = Zd[h] for h < kLdsHead); entries past Zd's allocation
-  // read 0.  The head sits above 16 K positions so that a rebased lane's base
-  // address (head - 16 j) stays non-negative.
-  __shared__ double2 zlds[kLdsTail + kLdsHead];
   const int tail_lo = max(kLdsHead, min(a.zd_count, a.len + 2 + K) - kLdsTail);
   const int tail_hi = tail_lo + kLdsTail;
-  for (int i = threadIdx.x; i < kLdsHead + kLdsTail; i += blockDim.x) {
+  for (int i = threadIdx.x; i < kLdsTail + kLdsHead; i += blockDim.x) {
     const int src = i < kLdsTail ? tail_lo + i : i - kLdsTail;
     zlds[i] = src < a.zd_count ? a.Zd[src] : make_double2(0.0, 0.0);
   }
   __syncthreads();
-  const double2* zhead = zlds + kLdsTail;  // rebased lanes read the orbit from its start
+  const double2* zhead = lds.head;  // rebased lanes read the orbit from its start
   const uint32_t c0 = q.first(), c1 = q.next();
   uint32_t ncur = cm.items(c0), nnext = cm.items(c1);
   uint32_t cur_pix = cm.pix(c.active, c0, ncur), nxt_pix = cm.pix(c.active, c1, nnext);
@@ -1948,9 +2127,18 @@ __global__ __launch_bounds__(kReduceThreads) void k_reduce_partials(const unsign
 }
 
 // clears the counter slots p[0, n) and the tile counts q[0, m)
-__global__ void k_zero(unsigned long long* p, int n, uint32_t* q, uint32_t m) {
+__device__ __forceinline__ void zero_counters(unsigned long long* p, int n, uint32_t* q, uint32_t m) {
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = 0ull;
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < m; i += gridDim.x * blockDim.x) q[i] = 0u;
+}
+__global__ void k_zero(unsigned long long* p, int n, uint32_t* q, uint32_t m) { zero_counters(p, n, q, m); }
+// the same, and the safe radii of orbit indices 0 .. mend (they depend on the
+// frames' largest |e| and the bailout, so they are made on each pass)
+__global__ void k_zero_safe(unsigned long long* p, int n, uint32_t* q, uint32_t m, const double2* Zd, int mend,
+                            double radius, double emax, double* safe) {
+  zero_counters(p, n, q, m);
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i <= mend; i += gridDim.x * blockDim.x)
+    safe_radius(Zd, mend, radius, emax, safe, i);
 }
 
 // ================================================================== engine
@@ -1966,9 +2154,25 @@ constexpr int iter_threads() { return kThreads; }
 template <>
 constexpr int iter_threads<SeriesArgs>() { return kSeriesIterThreads; }
 
+// workgroups of an iterate launch of `ti` threads: `waves` per SIMD
+static int iterate_grid(int num_cu, int waves, int ti) {
+  return std::max(1, std::min(num_cu * waves * 256 / ti, kPartSlots - kSlotIter));
+}
+
 // workgroups of the tile kernels (start, scatter, emit)
 static int tile_grid(uint64_t total, int num_cu) {
   return start_grid(total, num_cu, (uint64_t)(kSlotIter - kSlotStart));
+}
+
+static void launch_zero(hipStream_t stream, unsigned long long* part, const PlainArgs& a, uint32_t ntiles) {
+  hipLaunchKernelGGL(k_zero, dim3(256), dim3(256), 0, stream, part, kPartWords, a.c.tile_count, ntiles);
+}
+static void launch_zero(hipStream_t stream, unsigned long long* part, const SeriesArgs& a, uint32_t ntiles) {
+  if (a.safe)
+    hipLaunchKernelGGL(k_zero_safe, dim3(512), dim3(256), 0, stream, part, kPartWords, a.c.tile_count, ntiles, a.Zd,
+                       a.mend, a.radius, a.emax, a.safe);
+  else
+    hipLaunchKernelGGL(k_zero, dim3(256), dim3(256), 0, stream, part, kPartWords, a.c.tile_count, ntiles);
 }
 
 // The kernels of one pass on `stream`: zero the counters (part: kPartWords
@@ -1983,14 +2187,14 @@ static hipError_t launch_pass_on(hipStream_t stream, int num_cu, unsigned long l
   const int gtile = tile_grid(c.total, num_cu);
   // waves = persistent waves per SIMD: 4 per CU for each 256 threads
   const int ti = iter_threads<Args>();
-  const int giter = std::max(1, std::min(num_cu * waves * 256 / ti, kPartSlots - kSlotIter));
+  const int giter = iterate_grid(num_cu, waves, ti);
   hipError_t e;
 #define NM_LAUNCH_OK(expr)                   \
   do {                                       \
     expr;                                    \
     if ((e = hipGetLastError()) != hipSuccess) return e; \
   } while (0)
-  NM_LAUNCH_OK(hipLaunchKernelGGL(k_zero, dim3(256), dim3(256), 0, stream, part, kPartWords, c.tile_count, ntiles));
+  NM_LAUNCH_OK(launch_zero(stream, part, args, ntiles));
   if (evs && (e = hipEventRecord(evs[0], stream)) != hipSuccess) return e;
   NM_LAUNCH_OK(hipLaunchKernelGGL(start, dim3(gtile), dim3(kThreads), 0, stream, args));
   if (evs && (e = hipEventRecord(evs[1], stream)) != hipSuccess) return e;
@@ -2053,6 +2257,7 @@ class EngineImpl : public Engine {
   void* d_ttabs = nullptr; size_t n_ttabs_bytes = 0;  // tile search: epsilon tables
   void* d_tio = nullptr; size_t n_tio_bytes = 0;      // tile search: probes, predictions, results
   void* d_tile_ua = nullptr; size_t n_tile_ua_bytes = 0;  // per-tile skips of a render
+  void* d_safe = nullptr; size_t n_safe_bytes = 0;        // safe radius per orbit index
   unsigned long long* d_part = nullptr;               // kPartSlots x C_COUNT
   uint32_t* d_nactive = nullptr;
   uint64_t ref_serial = 0;
@@ -2192,6 +2397,7 @@ class EngineImpl : public Engine {
   // with the same pair and unmoved buffers reuses them
   uint64_t tab_serial = 0;
   int tab_tile = -1;
+  double tab_emax = 0.0;  // at least |epsilon| of every sample of the tables on the device (series path)
   bool tables_stale(const RenderOpts& opt, bool same_buffers) const {
     return opt.set_serial == 0 || opt.set_serial != tab_serial || opt.tile != tab_tile || !same_buffers;
   }
@@ -2505,7 +2711,10 @@ class EngineImpl : public Engine {
       std::vector<double> er, ei;
       std::vector<uint32_t> mask;
       er.reserve(ncol); ei.reserve(nrow); mask.reserve(nmask);
+      double mr = 0.0, mi = 0.0;
       for (auto* f : frames) {
+        for (double v : f->epsre) mr = std::max(mr, std::fabs(v));
+        for (double v : f->epsim) mi = std::max(mi, std::fabs(v));
         if (f->card_mode == CARD_MASK) mask.insert(mask.end(), f->mask.begin(), f->mask.end());
         er.insert(er.end(), f->epsre.begin(), f->epsre.end());
         ei.insert(ei.end(), f->epsim.begin(), f->epsim.end());
@@ -2516,6 +2725,7 @@ class EngineImpl : public Engine {
       if (!mask.empty())
         NM_HIP(hipMemcpyAsync(d_mask, mask.data(), mask.size() * 4, hipMemcpyHostToDevice, stream));
       NM_HIP(hipStreamSynchronize(stream));  // the host vectors end with this scope
+      tab_emax = (mr + mi) * (1.0 + 0x1p-40);
       tables_uploaded(opt);
     }
     a.epsre = t;
@@ -2543,23 +2753,38 @@ class EngineImpl : public Engine {
       a.skip_tpf = ntc * ntr;
     }
     const bool fx = opt.delta_mode == DELTA_FP32X;
-    // FP64 blocks hold one orbit entry per lane whatever K is (64 VGPRs), so the
-    // longest block amortises its set-up best; FP32X blocks renormalise their
+    // FP64 blocks hold one orbit entry per lane whatever K is.  After the coherent
+    // phase most samples of the double-series views have some 50 steps left, where
+    // a lane that is done waits half a block: 32 (iterate kernel 2.03 -> 1.96 ms on
+    // the 1e-30 view, 0.91 -> 0.87 ms on 16 frames of the 1e-40 video); with
+    // the thousands of steps of the floatexp-series views the longer block's set-up
+    // counts: 64 (5.27 -> 4.97 ms at 1e-100).  FP32X blocks renormalise their
     // mantissa at block ends, so they stay short
-    const int K = opt.block_k > 0 ? opt.block_k : fx ? 8 : 64;
-    // FP64: 4 persistent waves per SIMD (2 of the 512-thread workgroups per CU;
-    // against 8: the 1e-30 deep-zoom frame within 1%, the 1e-100 and 1e-200
-    // views 8% and 11% faster, their waves stalling less on the HBM path);
-    // an even count keeps the workgroups on the CUs evenly
-    const int waves = opt.waves_per_simd > 0 ? opt.waves_per_simd : fx ? 8 : 4;
+    const int K = opt.block_k > 0 ? opt.block_k : fx ? 8 : a.fxs ? 64 : 32;
+    // 4 persistent waves per SIMD: the two workgroups whose queues and windows fill
+    // a CU's LDS (more would wait for these to end; fewer hide too little latency:
+    // 2 waves 2.8-3.0 against 2.0 ms on the 1e-30 view, 1.29 against 0.91 ms on 16
+    // frames of the 1e-40 video).  FP32X ran 8 with smaller windows: 1.18 -> 1.07 ms
+    // on the 1279x719 frame of the 1e-200 view
+    const int waves = opt.waves_per_simd > 0 ? opt.waves_per_simd : 4;
     if (stats) {
       stats->block_k = K;
       stats->waves_per_simd = waves;
       stats->chunk_run = 1 << a.run_shift;
     }
+    a.safe = nullptr;
+    a.emax = tab_emax;
+    a.radius = opt.bailout;
+    if (!fx) {
+      if ((st = grow(&d_safe, &n_safe_bytes, ((size_t)a.mend + 1) * sizeof(double)))) return st;
+      a.safe = (double*)d_safe;
+    }
     auto go = [&](auto iter) {
-      return a.fxs ? run(a, k_series_start<true>, iter, waves, opt, stats, nout, host_out, emit_to)
-                   : run(a, k_series_start<false>, iter, waves, opt, stats, nout, host_out, emit_to);
+      if (fx)
+        return a.fxs ? run(a, k_series_start<true, false>, iter, waves, opt, stats, nout, host_out, emit_to)
+                     : run(a, k_series_start<false, false>, iter, waves, opt, stats, nout, host_out, emit_to);
+      return a.fxs ? run(a, k_series_start<true, true>, iter, waves, opt, stats, nout, host_out, emit_to)
+                   : run(a, k_series_start<false, true>, iter, waves, opt, stats, nout, host_out, emit_to);
     };
     switch (K) {
       case 8: return fx ? go(k_series_iterate<8, true>) : go(k_series_iterate<8, false>);
