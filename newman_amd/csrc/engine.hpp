@@ -71,11 +71,9 @@ struct SaReferenceHost {
   std::vector<double> CX, CN;  // max / min log2 |C_j|^2
   std::vector<int32_t> SP;     // count of special j (zero or non-finite B_j or C_j)
   // For views whose series terms under/overflow in the exact test (widths below
-  // about 1e-90): the thresholds T_j themselves, their sparse table of range
-  // minima (level k at [k * len], minima over [i, i + 2^k)), and suffix minima of
-  // log2 |B_j|^2 and log2 |C_j|^2 (over j >= i).
-  std::vector<double> T, ST, BNs, CNs;
-  int st_levels = 0;
+  // about 1e-90): the minimum tree of the thresholds T_j (tree_first_le), and
+  // suffix minima of log2 |B_j|^2 and log2 |C_j|^2 (over j >= i).
+  std::vector<double> T, tree, BNs, CNs;
   // Lookup of the stop search: PMT[k] = first i >= 1 with PM[i] <= pmt_base + k h
   // (len if none), k = 0 .. pmt_n, h = 1 / pmt_inv_h, over the finite range of
   // PM; pmt_n = 0 when PM has fewer than two distinct finite values.
@@ -83,6 +81,13 @@ struct SaReferenceHost {
   double pmt_base = 0.0, pmt_inv_h = 0.0;
   int pmt_n = 0;
 };
+
+// leaves of the thresholds' minimum tree (tree_first_le)
+inline uint32_t tree_leaves(uint32_t len) {
+  uint32_t p = 1;
+  while (p < len) p <<= 1;
+  return p;
+}
 
 // The series iterate kernel's active-list chunk setting (RenderOpts::chunk_run;
 // 0 or 64: 64 consecutive entries per chunk; 1, 2, 4, 8, 16, 32: interleaved

@@ -23,6 +23,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <limits>
 #include <vector>
 
 #include "sample_index.hpp"
@@ -393,4 +394,34 @@ long long nm_index_check(int nr, int nc, int nframes, int tile, int num_cu, int 
   return (long long)R.violations;
 }
 
+
+// tree_first_le against a linear scan: `len` thresholds from a seed (some +-inf,
+// many equal), every start, values below, at, between and above them.  Returns the
+// number of differing answers.
+long long nm_tree_check(int len, unsigned seed) {
+  if (len <= 0) return -1;
+  uint32_t leaves = 1;
+  while (leaves < (uint32_t)len) leaves <<= 1;
+  const double inf = std::numeric_limits<double>::infinity();
+  std::vector<double> tree(2 * (size_t)leaves, inf);
+  std::vector<double> vals = {-inf, -1.0, 41.0};
+  unsigned s = seed;
+  for (int i = 0; i < len; i++) {
+    s = s * 1664525u + 1013904223u;
+    const unsigned r = s >> 24;
+    const double t = r < 8 ? inf : r < 12 ? -inf : (double)(r % 41);
+    tree[leaves + (size_t)i] = t;
+  }
+  for (int v = 0; v < 41; v += 5) vals.push_back(v), vals.push_back(v + 0.5);
+  for (size_t k = leaves - 1; k >= 1; k--) tree[k] = std::min(tree[2 * k], tree[2 * k + 1]);
+  long long bad = 0;
+  for (double v : vals) {
+    int want = len;  // first i >= lo with T_i <= v, from the end
+    for (int lo = len; lo >= 0; lo--) {
+      if (lo < len && tree[leaves + (size_t)lo] <= v) want = lo;
+      bad += nm::tree_first_le(tree.data(), leaves, len, lo, v) != want;
+    }
+  }
+  return bad;
+}
 }  // extern "C"

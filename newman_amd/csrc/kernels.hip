@@ -137,13 +137,13 @@ struct SeriesArgs {
   const double* CX;
   const double* CN;
   const int* SP;
-  const double* ST;   // range-minimum sparse table of the thresholds (st_levels x len)
+  const double* tree;  // minimum tree of the thresholds (tree_first_le), tree_leaves(len) leaves
   const double* BNs;  // suffix minima of log2 |B_j|^2, |C_j|^2
   const double* CNs;
   const int* PMT;  // stop-search lookup over the finite PM range (pmt_n + 1 entries)
   double pmt_base, pmt_inv_h;
   int pmt_n;
-  int st_levels;
+  uint32_t tree_n;  // its leaves
   int len;
   int mend;  // len + 1
   int zd_count;  // entries allocated in Zd (past len + 1: zero padding)
@@ -1160,15 +1160,6 @@ __device__ __forceinline__ bool rounding_certified(const SeriesArgs& a, double L
          cmax + 3.0 * L < kLogHi;
 }
 
-// first i >= lo with T_i <= v (last + 1 if none), by the sparse table
-__device__ __forceinline__ int first_le_from(const SeriesArgs& a, int lo, double v) {
-  const int len = a.len;
-  int pos = lo;
-  for (int k = a.st_levels - 1; k >= 0; k--)
-    if (pos + (1 << k) <= len && a.ST[(size_t)k * len + pos] > v) pos += 1 << k;
-  return pos;
-}
-
 // Where the reference's exact scan must start when the prefix certificate of
 // sa_stop_index fails (its terms under- or overflow somewhere before the stop).
 // Indices whose |C_j e^3|^2 lies below 2^-1080 are stable whatever their
@@ -1183,7 +1174,7 @@ __device__ int deep_start(const SeriesArgs& a, double L) {
   if (ic > 0 && a.SP[ic] != 0) ic = 0;
   const int lo = ic + 1;
   if (lo > last || !(L > kLMin && L < kLMax)) return lo;
-  const int ia = first_le_from(a, lo, L + kMarg);
+  const int ia = tree_first_le(a.tree, a.tree_n, a.len, lo, L + kMarg);
   const int sidx = min(ia, last + 1) - 1;  // the last index the table certifies
   if (sidx < lo) return lo;
   const bool ok = a.SP[sidx] - a.SP[lo - 1] == 0 &&
@@ -1295,7 +1286,7 @@ __device__ int sa_stop_index_fx(const SeriesArgs& a, double L, int2 br, const Ep
   if (i > br.y && br.y < last) i = first_le(a.PM, br.y + 1, last, v);
   while (i <= last) {
     if (unstable_fx(a, i, p)) return i;
-    i = first_le_from(a, i + 1, v);
+    i = tree_first_le(a.tree, a.tree_n, a.len, i + 1, v);
   }
   return 0;
 }
@@ -1548,7 +1539,7 @@ __device__ __forceinline__ void coherent_phase(const SeriesArgs& a, const bool w
 template <bool FXS, bool COH>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_series_start(SeriesArgs a) {
   const Common& c = a.c;
-  unsigned long long ncard = 0, nres = 0, skipped = 0, credited = 0, executed = 0;
+  unsigned long long ncard = 0, nres = 0, skipped = 0, credited = 0, executed = 0, rebased = 0;
   const uint32_t ntiles = start_tiles(c.total);
   for (uint32_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
     uint32_t mine = 0;
@@ -1669,6 +1660,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(6, 8))
         const int it0 = hit;
         coherent_phase(a, want, ndr, ndi, e, hit, hm);
         executed += (unsigned long long)(hit - it0);
+        rebased += hm == 1 && hit > it0 ? 1ull : 0ull;
       }
       if (want) {
         // the delta only: the iterate kernel reads epsilon from the tables
@@ -1679,9 +1671,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(6, 8))
     }
     tile_count_add(c.tile_count, tile, mine);
   }
-  const unsigned long long v[5] = {ncard, nres, skipped, credited, executed};
-  const int idx[5] = {C_CARDIOID, C_SA_RES, C_SKIPPED, C_CREDITED, C_EXEC_START};
-  block_partial(c.part, kSlotStart + blockIdx.x, v, idx, COH ? 5 : 4);
+  const unsigned long long v[6] = {ncard, nres, skipped, credited, executed, rebased};
+  const int idx[6] = {C_CARDIOID, C_SA_RES, C_SKIPPED, C_CREDITED, C_EXEC_START, C_REBASED};
+  block_partial(c.part, kSlotStart + blockIdx.x, v, idx, COH ? 6 : 4);
 }
 
 // epsilon of sample gid (its pixel's offset from the reference point), from the
@@ -2141,6 +2133,10 @@ __global__ void k_zero_safe(unsigned long long* p, int n, uint32_t* q, uint32_t 
     safe_radius(Zd, mend, radius, emax, safe, i);
 }
 
+__global__ void k_clear(double* p, int n) {
+  for (int i = threadIdx.x; i < n; i += blockDim.x) p[i] = 0.0;
+}
+
 // ================================================================== engine
 #define NM_HIP(expr)                              \
   do {                                            \
@@ -2269,8 +2265,7 @@ class EngineImpl : public Engine {
   int rfxs = 0;
   const double *rPM = nullptr, *rBX = nullptr, *rBN = nullptr, *rCX = nullptr, *rCN = nullptr;
   const int* rSP = nullptr;
-  const double *rST = nullptr, *rBNs = nullptr, *rCNs = nullptr;
-  int rst_levels = 0;
+  const double *rtree = nullptr, *rBNs = nullptr, *rCNs = nullptr;
   const int* rPMT = nullptr;
   int rpmt_n = 0;
   double rpmt_base = 0.0, rpmt_inv_h = 0.0;
@@ -2319,49 +2314,42 @@ class EngineImpl : public Engine {
     // LDS orbit head (kHead + 1 entries) always exists
     const size_t nz = (size_t)len + 2 + kHead + 64;
     ref_zd_count = (int)nz;
-    size_t off = 0;
-    auto place = [&](size_t bytes) {
-      size_t o = off;
-      off += (bytes + 255) & ~(size_t)255;
-      return o;
-    };
-    size_t oZ = place(nz * 16), oXlo = place((size_t)len * 16), oA = place((size_t)len * 16),
-           oB = place((size_t)len * 16), oC = place((size_t)len * 16), oPM = place((size_t)len * 8),
-           oBX = place((size_t)len * 8), oBN = place((size_t)len * 8), oCX = place((size_t)len * 8),
-           oCN = place((size_t)len * 8), oSP = place((size_t)len * 4), oST = place(ref.ST.size() * 8),
-           oBNs = place(ref.BNs.size() * 8), oCNs = place(ref.CNs.size() * 8), oPMT = place(ref.PMT.size() * 4);
+    // The tables that the mode's kernels read, each copied from where the host
+    // keeps it.  (One zeroed staging image of all of them cost 8.3 ms of a 15 ms
+    // pass on a view with a new reference of length 100000, most of it page faults
+    // and copies on the host.)
     const bool fxs = ref.fxs && ref.Am.size() == 2 * (size_t)len;
-    const size_t nfm = fxs ? (size_t)len * 16 : 0, nfe = fxs ? (size_t)len * 8 : 0;
-    size_t oAm = place(nfm), oBm = place(nfm), oCm = place(nfm), oAe = place(nfe), oBe = place(nfe), oCe = place(nfe);
-    std::vector<char> h(off, 0);
-    std::memcpy(h.data() + oZ, ref.Zd.data(), ref.Zd.size() * 8);
-    std::memcpy(h.data() + oXlo, ref.Xlo.data(), ref.Xlo.size() * 8);
-    std::memcpy(h.data() + oA, ref.A.data(), ref.A.size() * 8);
-    std::memcpy(h.data() + oB, ref.B.data(), ref.B.size() * 8);
-    std::memcpy(h.data() + oC, ref.C.data(), ref.C.size() * 8);
-    std::memcpy(h.data() + oPM, ref.PM.data(), ref.PM.size() * 8);
-    std::memcpy(h.data() + oBX, ref.BX.data(), ref.BX.size() * 8);
-    std::memcpy(h.data() + oBN, ref.BN.data(), ref.BN.size() * 8);
-    std::memcpy(h.data() + oCX, ref.CX.data(), ref.CX.size() * 8);
-    std::memcpy(h.data() + oCN, ref.CN.data(), ref.CN.size() * 8);
-    std::memcpy(h.data() + oSP, ref.SP.data(), ref.SP.size() * 4);
-    std::memcpy(h.data() + oST, ref.ST.data(), ref.ST.size() * 8);
-    std::memcpy(h.data() + oBNs, ref.BNs.data(), ref.BNs.size() * 8);
-    std::memcpy(h.data() + oCNs, ref.CNs.data(), ref.CNs.size() * 8);
-    if (!ref.PMT.empty()) std::memcpy(h.data() + oPMT, ref.PMT.data(), ref.PMT.size() * 4);
-    if (fxs) {
-      std::memcpy(h.data() + oAm, ref.Am.data(), nfm);
-      std::memcpy(h.data() + oBm, ref.Bm.data(), nfm);
-      std::memcpy(h.data() + oCm, ref.Cm.data(), nfm);
-      std::memcpy(h.data() + oAe, ref.Ae.data(), nfe);
-      std::memcpy(h.data() + oBe, ref.Be.data(), nfe);
-      std::memcpy(h.data() + oCe, ref.Ce.data(), nfe);
-    }
+    struct Piece {
+      const void* src;
+      size_t bytes, off, room;
+    };
+    std::vector<Piece> pieces;
+    size_t off = 0;
+    auto place = [&](const void* src, size_t bytes, size_t room = 0) {
+      pieces.push_back({src, bytes, off, std::max(bytes, room)});
+      off += (std::max(bytes, room) + 255) & ~(size_t)255;
+      return pieces.back().off;
+    };
+    auto dbl = [&](const std::vector<double>& v, bool used = true) { return place(v.data(), used ? v.size() * 8 : 0); };
+    auto i32 = [&](const std::vector<int32_t>& v, bool used = true) { return place(v.data(), used ? v.size() * 4 : 0); };
+    const size_t oZ = place(ref.Zd.data(), ref.Zd.size() * 8, nz * 16), oXlo = dbl(ref.Xlo), oPM = dbl(ref.PM),
+                 otree = dbl(ref.tree), oPMT = i32(ref.PMT);
+    // the double test and its certificate
+    const size_t oA = dbl(ref.A, !fxs), oB = dbl(ref.B, !fxs), oC = dbl(ref.C, !fxs), oBX = dbl(ref.BX, !fxs),
+                 oBN = dbl(ref.BN, !fxs), oCX = dbl(ref.CX, !fxs), oCN = dbl(ref.CN, !fxs), oSP = i32(ref.SP, !fxs),
+                 oBNs = dbl(ref.BNs, !fxs), oCNs = dbl(ref.CNs, !fxs);
+    const size_t oAm = dbl(ref.Am, fxs), oBm = dbl(ref.Bm, fxs), oCm = dbl(ref.Cm, fxs), oAe = i32(ref.Ae, fxs),
+                 oBe = i32(ref.Be, fxs), oCe = i32(ref.Ce, fxs);
+    ref_serial = 0;  // no reference until all of the new one is there
     int st = grow(&d_ref, &n_ref_bytes, off);
     if (st) return st;
-    NM_HIP(hipMemcpyAsync(d_ref, h.data(), off, hipMemcpyHostToDevice, stream));
-    NM_HIP(hipStreamSynchronize(stream));
     char* b = (char*)d_ref;
+    for (const Piece& p : pieces)
+      if (p.bytes) NM_HIP(hipMemcpyAsync(b + p.off, p.src, p.bytes, hipMemcpyHostToDevice, stream));
+    const size_t zd = ref.Zd.size() * 8;  // zero past the orbit's end
+    hipLaunchKernelGGL(k_clear, dim3(1), dim3(256), 0, stream, (double*)(b + oZ + zd), (int)((nz * 16 - zd) / 8));
+    NM_HIP(hipGetLastError());
+    NM_HIP(hipStreamSynchronize(stream));
     rZd = (const double2*)(b + oZ);
     rXlo = (const double2*)(b + oXlo);
     rA = (const double2*)(b + oA);
@@ -2373,10 +2361,9 @@ class EngineImpl : public Engine {
     rCX = (const double*)(b + oCX);
     rCN = (const double*)(b + oCN);
     rSP = (const int*)(b + oSP);
-    rST = (const double*)(b + oST);
+    rtree = (const double*)(b + otree);
     rBNs = (const double*)(b + oBNs);
     rCNs = (const double*)(b + oCNs);
-    rst_levels = ref.st_levels;
     rPMT = (const int*)(b + oPMT);
     rpmt_n = ref.PMT.empty() ? 0 : ref.pmt_n;
     rpmt_base = ref.pmt_base;
@@ -2810,10 +2797,10 @@ class EngineImpl : public Engine {
     a.CX = rCX;
     a.CN = rCN;
     a.SP = rSP;
-    a.ST = rST;
+    a.tree = rtree;
+    a.tree_n = tree_leaves((uint32_t)ref_len);
     a.BNs = rBNs;
     a.CNs = rCNs;
-    a.st_levels = rst_levels;
     a.PMT = rPMT;
     a.pmt_n = rpmt_n;
     a.pmt_base = rpmt_base;

@@ -395,7 +395,7 @@ void Mandelbrot::buildThresholds() {
     }
     ref_.PM[i] = pm; ref_.BX[i] = bx; ref_.BN[i] = bn; ref_.CX[i] = cx; ref_.CN[i] = cn; ref_.SP[i] = sp;
   }
-  // thresholds, their range-minimum sparse table and the magnitude suffix minima
+  // thresholds and the magnitude suffix minima
   ref_.T.assign(len, INFINITY);
   ref_.BNs.assign(len + 1, INFINITY);
   ref_.CNs.assign(len + 1, INFINITY);
@@ -419,7 +419,7 @@ void Mandelbrot::buildThresholds() {
 // so only the thresholds matter: T_i = log2 tol + log2 |B_i|^2 - log2 |C_i|^2
 // from the floatexp coefficients, -inf where B_i = 0 and C_i != 0 (the test
 // fires for every e != 0), +inf where C_i = 0 (it never fires); PM is their
-// prefix minimum, ST their sparse table of range minima and PMT the lookup over
+// prefix minimum, tree their minimum tree and PMT the lookup over
 // the finite range of PM.  The magnitude tables (BX, BN, CX, CN, BNs, CNs) and
 // the special counts (SP) belong to the double test's certificate and are not
 // read in this mode.
@@ -448,8 +448,8 @@ void Mandelbrot::buildThresholdsFx() {
 }
 
 // the stop-search lookup (cells of the finite PM range, each holding the first
-// index whose prefix minimum reaches the cell's lower edge) and the sparse table
-// of range minima of T
+// index whose prefix minimum reaches the cell's lower edge) and the minimum tree
+// of T
 void Mandelbrot::buildStopLookup() {
   const int len = ref_.len;
   double pmax = -INFINITY, pmin = INFINITY;
@@ -474,15 +474,10 @@ void Mandelbrot::buildStopLookup() {
       ref_.PMT[k] = i;
     }
   }
-  int K = 1;
-  while ((1 << K) <= len) K++;
-  ref_.st_levels = K;
-  ref_.ST.assign((size_t)K * len, INFINITY);
-  for (int i = 0; i < len; i++) ref_.ST[i] = ref_.T[i];
-  for (int k = 1; k < K; k++)
-    for (int i = 0; i + (1 << k) <= len; i++)
-      ref_.ST[(size_t)k * len + i] =
-          std::min(ref_.ST[(size_t)(k - 1) * len + i], ref_.ST[(size_t)(k - 1) * len + i + (1 << (k - 1))]);
+  const size_t P = tree_leaves((uint32_t)len);
+  ref_.tree.assign(2 * P, INFINITY);
+  std::copy(ref_.T.begin(), ref_.T.end(), ref_.tree.begin() + P);
+  for (size_t k = P - 1; k >= 1; k--) ref_.tree[k] = std::min(ref_.tree[2 * k], ref_.tree[2 * k + 1]);
 }
 
 int Mandelbrot::setSeriesMode(int mode) {
@@ -541,7 +536,6 @@ int Mandelbrot::findProbeGPU(Engine* eng) {
   tmp.T = tmp.PM;
   tmp.BNs.assign((size_t)lenc + 1, 0.0);
   tmp.CNs = tmp.BNs;
-  tmp.st_levels = 0;
   int st = eng->set_reference(tmp, next_serial());
   if (st != NM_OK) return st;
   // frame A: rows nr/4, nr/2, 3nr/4 x even columns; frame B: even rows x column nc/2

@@ -159,6 +159,28 @@ __host__ __device__ inline uint32_t claim_lo(uint32_t nch, uint32_t h) {
   return (uint32_t)((uint64_t)nch * h / kQueues);
 }
 
+// ---- the thresholds' minimum tree: tree[P + i] = T_i for i < len, +inf up to 2 P,
+// tree[k] = min(tree[2 k], tree[2 k + 1]), P (leaves) a power of two at or above len.
+// (A sparse table of range minima answers as fast but holds log2(len) doubles per
+// index: 13.6 of the 35 MB a reference of length 100000 uploaded.)
+// the first i >= lo with T_i <= v (len if none)
+__host__ __device__ inline int tree_first_le(const double* tree, uint32_t leaves, int len, int lo, double v) {
+  if (lo >= len) return len;
+  uint32_t k = leaves + (uint32_t)lo;
+  do {
+    while (!(k & 1u)) k >>= 1;  // the largest subtree that starts here
+    if (tree[k] <= v) {
+      while (k < leaves) {
+        k <<= 1;
+        if (!(tree[k] <= v)) k++;
+      }
+      return (int)(k - leaves);
+    }
+    k++;
+  } while ((k & (k - 1u)) != 0);  // a power of two: past the last subtree of its level
+  return len;
+}
+
 // samples per frame in the sample order (tiles pad the frame); 0 = bad tile
 inline uint64_t frame_samples(int nr, int nc, int tile) {
   if (tile == 0) return (uint64_t)nr * nc;

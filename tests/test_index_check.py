@@ -68,3 +68,12 @@ def test_the_checker_finds_planted_mistakes(plant):
     scatter that selects the next set bit are each reported."""
     v, msg, _ = _check(3, 7, 5, 16, 7, 1, 8, plant=plant)
     assert v > 0 and msg
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 7, 8, 9, 63, 64, 65, 1000, 4097])
+def test_threshold_tree_search(n):
+    """The minimum tree's search equals a linear scan from every start."""
+    L = _lib()
+    L.nm_tree_check.restype = C.c_longlong
+    L.nm_tree_check.argtypes = [C.c_int, C.c_uint]
+    assert all(L.nm_tree_check(n, seed) == 0 for seed in range(1, 6))
