@@ -45,15 +45,19 @@ class SkipNet {
   uint64_t version = 0;  // bumped whenever the parameters change
 
  private:
-  int reserve(size_t nx, size_t nb);
-  int batch_grad(int n);
+  static constexpr int kMaxEpochsAtOnce = 64;
+  struct AdamStep {
+    float lr = 0.0f, c1 = 1.0f, c2 = 1.0f;
+  };
+  int reserve(size_t nx, size_t nb, size_t ni);
+  int batch(const int* idx, int n, float* G, const AdamStep& a, float* loss);
   void release();
   std::string err_;
   float *dP = nullptr, *dG = nullptr, *dM = nullptr, *dV = nullptr, *dX = nullptr, *dT = nullptr;
-  float *dXB = nullptr, *dTB = nullptr, *dH1 = nullptr, *dH2 = nullptr, *dY = nullptr, *dDY = nullptr;
+  float *dH1 = nullptr, *dH2 = nullptr, *dY = nullptr, *dDY = nullptr;
   float *dD1 = nullptr, *dD2 = nullptr, *dLoss = nullptr;
   int* dIdx = nullptr;
-  size_t capX = 0, capB = 0;
+  size_t capX = 0, capB = 0, capI = 0;
 };
 
 }  // namespace nm
