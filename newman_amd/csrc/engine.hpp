@@ -30,26 +30,50 @@ enum DeltaMode : int32_t { DELTA_FP64 = 0, DELTA_FP32X = 1 };
 enum SeriesMode : int32_t { SERIES_DOUBLE = 0, SERIES_FLOATEXP = 1 };
 constexpr int32_t kFxZeroExp = -0x40000000;  // the exponent of a floatexp zero
 
-// One frame of the plain-double path (mandelbrot.cpp:231-254): per-column and
-// per-row truncated coordinates (descend of the HP pixel map) plus the remainder
-// as a double-double low part for the cardioid test.
+// A high-precision value as the device reads it: hpfloat.hpp's hpf, field for field
+// (value = sign * 0.m * 2^exp, m[L - 1] the most significant limb).
+constexpr int kHpMaxLimbs = 40;
+struct HpVal {
+  int32_t L, sign;
+  int64_t exp;
+  uint64_t m[kHpMaxLimbs];
+};
+// What a frame's coordinate tables are made from (coords.hpp): centre, sample size
+// and on the series path the reference point, the working precision in limbs, and
+// the most limbs that any of the values holds.
+struct FrameHp {
+  HpVal cre, cim, sre, sim, x0re, x0im;
+  int32_t L, limbs;
+};
+
+// the offsets of column c and row r of an nr x nc frame from its centre, in samples
+constexpr long column_offset(int c, int nc) { return (long)(c - nc / 2); }
+constexpr long row_offset(int r, int nr) { return (long)(nr / 2 - r - 1); }
+
+// One frame of the plain-double path (mandelbrot.cpp:231-254); its per-column and
+// per-row truncated coordinates (descend of the HP pixel map), with the remainder
+// as a double-double low part for the cardioid test, are made on the device.
 struct HwFrameHost {
   int nr = 0, nc = 0;
   int card_mode = CARD_TEST_DD;
   // every coordinate is 0 or at least 2^-200 in magnitude: the device may fold
   // (2x) y + c into fma(x y, 2, c) bit for bit (see plain_update)
   bool fma_ok = false;
-  double c_bound = HUGE_VAL;        // at least every |c| of the frame (grouped_test_ok; unknown: +inf)
-  std::vector<double> cre, crelo;  // nc
-  std::vector<double> cim, cimlo;  // nr
+  double c_bound = HUGE_VAL;  // at least every |c| of the frame (grouped_test_ok; unknown: +inf)
+  FrameHp hp;
 };
 
 // One frame of the series-approximation path (mandelbrot.cpp:144-229): per-column
-// and per-row epsilon = descend(Y0 - X[0]), and the cardioid classification.
+// and per-row epsilon = descend(Y0 - X[0]), and the cardioid classification.  The
+// epsilon tables are made on the device, or given (own_tables: samples off the
+// regular grid; the tile search also reads the given ones on the host).
 struct SaFrameHost {
   int nr = 0, nc = 0;
   int card_mode = CARD_NONE;
-  std::vector<double> epsre;      // nc
+  bool own_tables = false;        // the device takes epsre, epsim
+  FrameHp hp;
+  double emax = 0.0;              // at least |epsilon| of every sample
+  std::vector<double> epsre;      // nc (or empty: device only)
   std::vector<double> epsim;      // nr
   std::vector<uint32_t> mask;     // CARD_MASK: nr*nc bits, 1 = in cardioid/bulb
 };
@@ -149,22 +173,12 @@ struct RenderStats {
   int block_k = 0, waves_per_simd = 0;
 };
 
-// A plain-path frame as tables the caller keeps (render_hw_noalloc).
-struct HwFrameView {
-  int nr = 0, nc = 0;
-  int card_mode = CARD_TEST_DD;
-  bool fma_ok = false;
-  double c_bound = HUGE_VAL;
-  const double *cre = nullptr, *crelo = nullptr;  // nc each
-  const double *cim = nullptr, *cimlo = nullptr;  // nr each
-};
-
 // The plain path of one frame (at most 2^19 samples, rows and columns at most
 // 8192) with every device buffer in a file-scope device array: no device
 // allocation, no stream or event created (the null stream), no engine buffer
 // touched.  Results in host_out (nr x nc, row-major).  Calls overlapping on one
 // device share that array and race.
-int render_hw_noalloc(const HwFrameView& f, int N, double bailout, EscapeValue* host_out, std::string& err);
+int render_hw_noalloc(const HwFrameHost& f, int N, double bailout, EscapeValue* host_out, std::string& err);
 
 // Device engine: one per process per device.  All calls are synchronous.
 class Engine {

@@ -20,12 +20,15 @@
 //    partitioning the chunks.
 // Test support, not part of the render path: built as its own library and called
 // from the CPU tests.
+#include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
 #include <limits>
 #include <vector>
 
+#include "coords.hpp"
+#include "hpfloat.hpp"
 #include "sample_index.hpp"
 
 namespace {
@@ -423,5 +426,91 @@ long long nm_tree_check(int len, unsigned seed) {
     }
   }
   return bad;
+}
+
+// The device's coordinate entries against hpfloat.cpp: `n` cases from a seed, with
+// random mantissas (some sparse), exponents, signs and offsets, every combination of
+// precisions that `ML` limbs hold; the truncated coordinate, its remainder and the
+// truncated difference from a reference point near it.  Returns the number of cases
+// that differ in a bit.
+}  // extern "C"
+namespace {
+uint64_t next_u64(uint64_t& s) {
+  uint64_t z = (s += 0x9E3779B97F4A7C15ull);
+  z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+  z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+  return z ^ (z >> 31);
+}
+nm::HpVal val_of(const nm::hpf& v) {
+  nm::HpVal d;
+  std::memcpy((void*)&d, (const void*)&v, sizeof d);
+  return d;
+}
+// as mandelbrot.cpp's get_d_nearest
+double nearest(const nm::hpf& a) {
+  const double t = a.get_d();
+  if (a.sign == 0 || !std::isfinite(t)) return t;
+  nm::hpf td(2), r(a.L), half(2);
+  nm::hp_set_d(td, t);
+  nm::hp_sub(r, a, td);
+  if (r.sign == 0) return t;
+  const double up = std::nextafter(t, a.sign > 0 ? INFINITY : -INFINITY);
+  nm::hp_set_d(half, (up - t) * 0.5);
+  r.sign = half.sign = 1;
+  const int c = nm::hp_cmp(r, half);
+  uint64_t bits;
+  std::memcpy(&bits, &t, 8);
+  return c > 0 || (c == 0 && (bits & 1)) ? up : t;
+}
+template <int ML>
+long long coords_check(unsigned seed, int n) {
+  uint64_t s = seed;
+  auto random_hpf = [&](int64_t e) {
+    nm::hpf v(1 + (int)(next_u64(s) % ML));
+    if (next_u64(s) % 16 == 0) return v;  // zero
+    const int kind = (int)(next_u64(s) % 4);
+    for (int i = 0; i < v.L; i++) v.m[i] = kind == 0 ? 0 : kind == 1 ? ~0ull : next_u64(s);
+    if (kind == 3 && v.L > 2) v.m[1] = 0;
+    v.m[v.L - 1] |= 1ull << 63;
+    v.sign = next_u64(s) & 1 ? 1 : -1;
+    v.exp = e;
+    return v;
+  };
+  auto same = [](double a, double b) { return std::memcmp(&a, &b, 8) == 0 || a == b; };
+  long long bad = 0;
+  for (int t = 0; t < n; t++) {
+    const int L = 1 + (int)(next_u64(s) % ML);
+    const nm::hpf c = random_hpf((int64_t)(next_u64(s) % 5) - 2);
+    const nm::hpf z = random_hpf(-(int64_t)(next_u64(s) % (next_u64(s) % 2 ? 40 : 64 * ML + 80)));
+    const long k = (long)(next_u64(s) % 16385) - 8192;
+    nm::hpf step(L), p(L), x0(L), y(L), td(2), rem(L);
+    nm::hp_mul_si(step, z, k);
+    nm::hp_add(p, c, step);
+    if (next_u64(s) % 2) nm::hp_set(x0, c);  // a reference point: the centre, or one step off
+    else nm::hp_add(x0, c, z);
+    nm::hp_sub(y, p, x0);
+    const double hi = p.get_d();
+    nm::hp_set_d(td, hi);
+    nm::hp_sub(rem, p, td);
+    const double lo = nearest(rem);
+    const auto q = nm::hpd_pixel<ML>(val_of(c), val_of(z), k, L);
+    const double dy = nm::hpd_get_d(nm::hpd_add(q, nm::hpd_load<ML>(val_of(x0)), -1, L));
+    // the remainder serves the plain path alone, whose sample size is at least
+    // 1.5e-16: it stays far above the subnormal doubles
+    const bool rest = rem.sign == 0 || rem.exp > -900;
+    bad += !same(nm::hpd_get_d(q), hi) || (rest && !same(nm::hpd_rest(q), lo)) || !same(dy, y.get_d());
+  }
+  return bad;
+}
+}  // namespace
+extern "C" {
+long long nm_coords_check(int limbs, unsigned seed, int n) {
+  switch (limbs) {
+    case 4: return coords_check<4>(seed, n);
+    case 8: return coords_check<8>(seed, n);
+    case 16: return coords_check<16>(seed, n);
+    case 40: return coords_check<40>(seed, n);
+    default: return -1;
+  }
 }
 }  // extern "C"

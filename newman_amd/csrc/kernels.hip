@@ -54,6 +54,7 @@
 #include <vector>
 
 #include "colour.hpp"
+#include "coords.hpp"
 #include "engine.hpp"
 #include "sample_index.hpp"
 #include "video.hpp"
@@ -2133,6 +2134,7 @@ __global__ void k_zero_safe(unsigned long long* p, int n, uint32_t* q, uint32_t 
     safe_radius(Zd, mend, radius, emax, safe, i);
 }
 
+__global__ void k_put_frame(DevFrame* p, DevFrame f) { *p = f; }
 __global__ void k_clear(double* p, int n) {
   for (int i = threadIdx.x; i < n; i += blockDim.x) p[i] = 0.0;
 }
@@ -2253,6 +2255,8 @@ class EngineImpl : public Engine {
   void* d_ttabs = nullptr; size_t n_ttabs_bytes = 0;  // tile search: epsilon tables
   void* d_tio = nullptr; size_t n_tio_bytes = 0;      // tile search: probes, predictions, results
   void* d_tile_ua = nullptr; size_t n_tile_ua_bytes = 0;  // per-tile skips of a render
+  void* d_hp = nullptr; size_t n_hp_bytes = 0;            // what the coordinate tables are made from
+  void* h_stage = nullptr; size_t n_stage_bytes = 0;      // pinned staging of a set's frame records
   void* d_safe = nullptr; size_t n_safe_bytes = 0;        // safe radius per orbit index
   unsigned long long* d_part = nullptr;               // kPartSlots x C_COUNT
   uint32_t* d_nactive = nullptr;
@@ -2391,6 +2395,38 @@ class EngineImpl : public Engine {
   void tables_uploaded(const RenderOpts& opt) {
     tab_serial = opt.set_serial;
     tab_tile = opt.tile;
+  }
+
+  // the frame records and coordinate tables of a frame set, on the device: a single
+  // frame's come with the kernel's arguments, several frames' through the pinned
+  // staging buffer (free again: every render ends with a wait for the stream)
+  int make_tables(const std::vector<DevFrame>& df, const std::vector<FrameHp>& hp, int nr, int nc, bool series,
+                  const CoordTables& t) {
+    const size_t nf = df.size(), fbytes = (nf * sizeof(DevFrame) + 255) & ~(size_t)255;
+    int st, limbs = 0;
+    for (const FrameHp& h : hp) limbs = std::max(limbs, h.limbs);
+    const bool one = nf == 1;
+    if (!one) {
+      const size_t bytes = fbytes + nf * sizeof(FrameHp);
+      if ((st = grow(&d_hp, &n_hp_bytes, nf * sizeof(FrameHp)))) return st;
+      if (bytes > n_stage_bytes) {
+        if (h_stage) NM_HIP(hipHostFree(h_stage));
+        h_stage = nullptr;
+        n_stage_bytes = 0;
+        NM_HIP(hipHostMalloc(&h_stage, bytes, hipHostMallocDefault));
+        n_stage_bytes = bytes;
+      }
+      std::memcpy(h_stage, df.data(), nf * sizeof(DevFrame));
+      std::memcpy((char*)h_stage + fbytes, hp.data(), nf * sizeof(FrameHp));
+      NM_HIP(hipMemcpyAsync(d_frames, h_stage, nf * sizeof(DevFrame), hipMemcpyHostToDevice, stream));
+      NM_HIP(hipMemcpyAsync(d_hp, (char*)h_stage + fbytes, nf * sizeof(FrameHp), hipMemcpyHostToDevice, stream));
+    } else {
+      hipLaunchKernelGGL(k_put_frame, dim3(1), dim3(1), 0, stream, (DevFrame*)d_frames, df[0]);
+      NM_HIP(hipGetLastError());
+    }
+    if (coords_launch((void*)stream, one ? &hp[0] : nullptr, (const FrameHp*)d_hp, (int)nf, nr, nc, limbs, series, t))
+      return fail("k_coords launch", hipGetLastError());
+    return NM_OK;
   }
 
   // buffers and the common kernel arguments for `total` samples
@@ -2555,8 +2591,8 @@ class EngineImpl : public Engine {
       d.tab_c = (uint32_t)tc;
       d.tab_r = (uint32_t)tr;
       d.card_mode = f->card_mode;
-      tc += f->cre.size();
-      tr += f->cim.size();
+      tc += (size_t)f->nc;
+      tr += (size_t)f->nr;
       total += fs;
       nout += (uint64_t)f->nr * f->nc;
       df.push_back(d);
@@ -2578,22 +2614,11 @@ class EngineImpl : public Engine {
     a.c.inv_frame = 1.0 / (double)a.c.frame_size;
     double* t = (double*)d_tabs;
     if (upload) {
-      // the coordinate tables of every frame, concatenated (built only when the
-      // device copy is stale: a repeated frame set reuses it)
-      std::vector<double> cre, crelo, cim, cimlo;
-      cre.reserve(ncol); crelo.reserve(ncol); cim.reserve(nrow); cimlo.reserve(nrow);
-      for (auto* f : frames) {
-        cre.insert(cre.end(), f->cre.begin(), f->cre.end());
-        crelo.insert(crelo.end(), f->crelo.begin(), f->crelo.end());
-        cim.insert(cim.end(), f->cim.begin(), f->cim.end());
-        cimlo.insert(cimlo.end(), f->cimlo.begin(), f->cimlo.end());
-      }
-      NM_HIP(hipMemcpyAsync(d_frames, df.data(), df.size() * sizeof(DevFrame), hipMemcpyHostToDevice, stream));
-      NM_HIP(hipMemcpyAsync(t, cre.data(), ncol * 8, hipMemcpyHostToDevice, stream));
-      NM_HIP(hipMemcpyAsync(t + ncol, crelo.data(), ncol * 8, hipMemcpyHostToDevice, stream));
-      NM_HIP(hipMemcpyAsync(t + 2 * ncol, cim.data(), nrow * 8, hipMemcpyHostToDevice, stream));
-      NM_HIP(hipMemcpyAsync(t + 2 * ncol + nrow, cimlo.data(), nrow * 8, hipMemcpyHostToDevice, stream));
-      NM_HIP(hipStreamSynchronize(stream));  // the host vectors end with this scope
+      // made again only when the device copy is stale: a repeated frame set reuses it
+      std::vector<FrameHp> hp;
+      for (auto* f : frames) hp.push_back(f->hp);
+      if ((st = make_tables(df, hp, frames[0]->nr, frames[0]->nc, false, {t, t + ncol, t + 2 * ncol, t + 2 * ncol + nrow})))
+        return st;
       tables_uploaded(opt);
     }
     a.pre_iter = opt.pre_iter > 0 ? opt.pre_iter : kPreIterDefault;
@@ -2669,8 +2694,8 @@ class EngineImpl : public Engine {
         if (f->mask.size() * 32 < (size_t)f->nr * f->nc) return NM_ERR_ARG;
         tm += f->mask.size();
       }
-      tc += f->epsre.size();
-      tr += f->epsim.size();
+      tc += (size_t)f->nc;
+      tr += (size_t)f->nr;
       total += fs;
       nout += (uint64_t)f->nr * f->nc;
       df.push_back(d);
@@ -2693,26 +2718,34 @@ class EngineImpl : public Engine {
     a.c.inv_frame = 1.0 / (double)a.c.frame_size;
     double* t = (double*)d_tabs;
     if (upload) {
-      // every frame's delta tables and cardioid masks, concatenated (built only
-      // when the device copy is stale: a repeated frame set reuses it)
-      std::vector<double> er, ei;
+      // made again only when the device copy is stale: a repeated frame set reuses it
       std::vector<uint32_t> mask;
-      er.reserve(ncol); ei.reserve(nrow); mask.reserve(nmask);
-      double mr = 0.0, mi = 0.0;
+      std::vector<double> er, ei;
+      std::vector<FrameHp> hp;
+      double emax = 0.0;
       for (auto* f : frames) {
-        for (double v : f->epsre) mr = std::max(mr, std::fabs(v));
-        for (double v : f->epsim) mi = std::max(mi, std::fabs(v));
         if (f->card_mode == CARD_MASK) mask.insert(mask.end(), f->mask.begin(), f->mask.end());
-        er.insert(er.end(), f->epsre.begin(), f->epsre.end());
-        ei.insert(ei.end(), f->epsim.begin(), f->epsim.end());
+        emax = std::max(emax, f->emax);
+        if (f->own_tables != frames[0]->own_tables) return NM_ERR_ARG;
+        if (f->own_tables) {
+          er.insert(er.end(), f->epsre.begin(), f->epsre.end());
+          ei.insert(ei.end(), f->epsim.begin(), f->epsim.end());
+        } else {
+          hp.push_back(f->hp);
+        }
       }
-      NM_HIP(hipMemcpyAsync(d_frames, df.data(), df.size() * sizeof(DevFrame), hipMemcpyHostToDevice, stream));
-      NM_HIP(hipMemcpyAsync(t, er.data(), ncol * 8, hipMemcpyHostToDevice, stream));
-      NM_HIP(hipMemcpyAsync(t + ncol, ei.data(), nrow * 8, hipMemcpyHostToDevice, stream));
       if (!mask.empty())
         NM_HIP(hipMemcpyAsync(d_mask, mask.data(), mask.size() * 4, hipMemcpyHostToDevice, stream));
-      NM_HIP(hipStreamSynchronize(stream));  // the host vectors end with this scope
-      tab_emax = (mr + mi) * (1.0 + 0x1p-40);
+      if (!hp.empty()) {
+        if ((st = make_tables(df, hp, frames[0]->nr, frames[0]->nc, true, {t, nullptr, t + ncol, nullptr}))) return st;
+      } else {
+        if (er.size() != ncol || ei.size() != nrow) return NM_ERR_ARG;
+        NM_HIP(hipMemcpyAsync(d_frames, df.data(), df.size() * sizeof(DevFrame), hipMemcpyHostToDevice, stream));
+        NM_HIP(hipMemcpyAsync(t, er.data(), ncol * 8, hipMemcpyHostToDevice, stream));
+        NM_HIP(hipMemcpyAsync(t + ncol, ei.data(), nrow * 8, hipMemcpyHostToDevice, stream));
+      }
+      if (!mask.empty() || hp.empty()) NM_HIP(hipStreamSynchronize(stream));  // the host vectors end with this scope
+      tab_emax = emax * (1.0 + 0x1p-40);
       tables_uploaded(opt);
     }
     a.epsre = t;
@@ -3058,9 +3091,8 @@ static int noalloc_setup(int dev, NoAllocDevice** out, std::string& err) {
   return NM_OK;
 }
 
-int render_hw_noalloc(const HwFrameView& f, int N, double bailout, EscapeValue* host_out, std::string& err) {
-  if (f.nr <= 0 || f.nc <= 0 || N <= 0 || !(bailout > 0.0) || !host_out || !f.cre || !f.crelo || !f.cim ||
-      !f.cimlo) {
+int render_hw_noalloc(const HwFrameHost& f, int N, double bailout, EscapeValue* host_out, std::string& err) {
+  if (f.nr <= 0 || f.nc <= 0 || N <= 0 || !(bailout > 0.0) || !host_out) {
     err = "bad argument";
     return NM_ERR_ARG;
   }
@@ -3115,11 +3147,11 @@ int render_hw_noalloc(const HwFrameView& f, int N, double bailout, EscapeValue* 
       return NM_ERR_HIP;                                           \
     }                                                              \
   } while (0)
-  NA_HIP(hipMemcpyAsync(frame, &df, sizeof df, hipMemcpyHostToDevice, s));
-  NA_HIP(hipMemcpyAsync(tabs, f.cre, (size_t)f.nc * 8, hipMemcpyHostToDevice, s));
-  NA_HIP(hipMemcpyAsync(tabs + f.nc, f.crelo, (size_t)f.nc * 8, hipMemcpyHostToDevice, s));
-  NA_HIP(hipMemcpyAsync(tabs + 2 * f.nc, f.cim, (size_t)f.nr * 8, hipMemcpyHostToDevice, s));
-  NA_HIP(hipMemcpyAsync(tabs + 2 * f.nc + f.nr, f.cimlo, (size_t)f.nr * 8, hipMemcpyHostToDevice, s));
+  hipLaunchKernelGGL(k_put_frame, dim3(1), dim3(1), 0, s, frame, df);
+  NA_HIP(hipGetLastError());
+  if (coords_launch((void*)s, &f.hp, nullptr, 1, f.nr, f.nc, f.hp.limbs, false,
+                    {tabs, tabs + f.nc, tabs + 2 * (size_t)f.nc, tabs + 2 * (size_t)f.nc + f.nr}))
+    NA_HIP(hipGetLastError());
   PlainArgs a{};
   Common& c = a.c;
   c.frames = frame;

@@ -558,6 +558,13 @@ int Mandelbrot::findProbeGPU(Engine* eng) {
   for (int r : {rows() / 4, rows() / 2, 3 * rows() / 4}) fa.epsim.push_back(eps_im(r));
   fb.epsre.push_back(eps_re(cols() / 2));
   for (int k = 0; k < nrb; k++) fb.epsim.push_back(eps_im(2 * k));
+  for (SaFrameHost* f : {&fa, &fb}) {
+    f->own_tables = true;
+    double mr = 0.0, mi = 0.0;
+    for (double v : f->epsre) mr = std::max(mr, std::fabs(v));
+    for (double v : f->epsim) mi = std::max(mi, std::fabs(v));
+    f->emax = mr + mi;
+  }
   RenderOpts o;
   applyLaunch(o);
   o.tile = 0;
@@ -705,54 +712,72 @@ static int classify_frame(const HPComplex& center, const HPComplex& sz, int nr, 
   return -1;
 }
 
-// Per-column / per-row truncated coordinates of the plain-double path
-// (descend(Y0) in getIterationsHW, mandelbrot.cpp:234) plus the double-double
-// remainder used by the device cardioid test.
-int Mandelbrot::buildHwFrame(HwFrameHost& f, const HPComplex& cen, const HPComplex& s) {
+// The values that a frame's coordinate tables are made from; X0: the reference
+// point of the series path, or null.
+static_assert(sizeof(HpVal) == sizeof(hpf) && kHpMaxLimbs == HP_MAXL, "HpVal is hpf's layout");
+static FrameHp frame_hp(const HPComplex& cen, const HPComplex& s, const HPComplex* X0) {
+  FrameHp h;
+  auto put = [](HpVal& d, const hpf& v) { std::memcpy((void*)&d, (const void*)&v, sizeof(HpVal)); };
+  put(h.cre, cen.re);
+  put(h.cim, cen.im);
+  put(h.sre, s.re);
+  put(h.sim, s.im);
+  put(h.x0re, X0 ? X0->re : cen.re);
+  put(h.x0im, X0 ? X0->im : cen.im);
+  h.L = hp_limbs_for_bits(hp_default_bits());
+  h.limbs = h.L;
+  for (const HpVal* v : {&h.cre, &h.cim, &h.sre, &h.sim, &h.x0re, &h.x0im}) h.limbs = std::max(h.limbs, v->L);
+  return h;
+}
+
+// descend(center + k * size), less the reference point x0 when it is given
+static double coordinate(const hpf& center, const hpf& size, long k, const hpf* x0) {
+  const int L = hp_limbs_for_bits(hp_default_bits());
+  hpf p(L), y(L);
+  pixel_re(p, center, size, k);
+  if (!x0) return p.get_d();
+  hp_sub(y, p, *x0);
+  return y.get_d();
+}
+
+// A plain frame's card mode, update form and |c| bound, and what its tables are
+// made from.  The coordinates grow with the column and fall with the row (the size
+// is positive on the plain path, and truncation keeps the order), so their largest
+// magnitudes are at the ends and the smallest ones beside 0 next to a sign change,
+// found by bisection.
+int Mandelbrot::buildHwFrame(HwFrameHost& f, const HPComplex& cen, const HPComplex& s) const {
   f.nr = rows();
   f.nc = cols();
-  f.cre.resize(f.nc); f.crelo.resize(f.nc);
-  f.cim.resize(f.nr); f.cimlo.resize(f.nr);
-  fillHwTables(cen, s, f.cre.data(), f.crelo.data(), f.cim.data(), f.cimlo.data(), &f.card_mode, &f.fma_ok,
-               &f.c_bound);
+  f.hp = frame_hp(cen, s, nullptr);
+  const int m = classify_frame(cen, s, f.nr, f.nc);
+  f.card_mode = m < 0 ? CARD_TEST_DD : m;
+  auto clear = [](double v) { return v == 0.0 || std::fabs(v) >= 0x1p-200; };
+  // offsets [lo, hi] of one axis: the largest magnitude, and whether all are clear
+  auto axis = [&](const hpf& c, const hpf& size, long lo, long hi, bool& ok) {
+    auto at = [&](long k) { return coordinate(c, size, k, nullptr); };
+    const double a = at(lo), b = at(hi);
+    ok = clear(a) && clear(b);
+    if (a < 0.0 && b >= 0.0) {  // the last negative one
+      long l = lo, h = hi;
+      while (h - l > 1) (at((l + h) / 2) < 0.0 ? l : h) = (l + h) / 2;
+      ok = ok && clear(at(l));
+    }
+    if (a <= 0.0 && b > 0.0) {  // the first positive one
+      long l = lo, h = hi;
+      while (h - l > 1) (at((l + h) / 2) > 0.0 ? h : l) = (l + h) / 2;
+      ok = ok && clear(at(h));
+    }
+    return std::max(std::fabs(a), std::fabs(b));
+  };
+  bool okc = true, okr = true;
+  const double mx = axis(cen.re, s.re, column_offset(0, f.nc), column_offset(f.nc - 1, f.nc), okc);
+  const double my = axis(cen.im, s.im, row_offset(f.nr - 1, f.nr), row_offset(0, f.nr), okr);
+  f.fma_ok = okc && okr;
+  f.c_bound = std::sqrt(mx * mx + my * my) * (1.0 + 0x1p-40);  // rounded up
   return NM_OK;
 }
 
-// The tables of buildHwFrame into caller-owned arrays (cols() and rows()
-// entries); allocates nothing.
-void Mandelbrot::fillHwTables(const HPComplex& cen, const HPComplex& s, double* cre, double* crelo, double* cim,
-                              double* cimlo, int* card_mode, bool* fma_ok, double* c_bound) const {
-  const int L = hp_limbs_for_bits(hp_default_bits());
-  const int nr = rows(), nc = cols();
-  hpf p(L), rem(L), td(2);
-  for (int c = 0; c < nc; c++) {
-    pixel_re(p, cen.re, s.re, (long)(c - nc / 2));
-    double t = p.get_d();
-    hp_set_d(td, t);
-    hp_sub(rem, p, td);
-    cre[c] = t;
-    crelo[c] = get_d_nearest(rem);
-  }
-  for (int r = 0; r < nr; r++) {
-    pixel_re(p, cen.im, s.im, (long)(nr / 2 - r - 1));
-    double t = p.get_d();
-    hp_set_d(td, t);
-    hp_sub(rem, p, td);
-    cim[r] = t;
-    cimlo[r] = get_d_nearest(rem);
-  }
-  int m = classify_frame(cen, s, nr, nc);
-  *card_mode = m < 0 ? CARD_TEST_DD : m;
-  auto clear = [](double v) { return v == 0.0 || std::fabs(v) >= 0x1p-200; };
-  *fma_ok = std::all_of(cre, cre + nc, clear) && std::all_of(cim, cim + nr, clear);
-  double mx = 0.0, my = 0.0;
-  for (int c = 0; c < nc; c++) mx = std::max(mx, std::fabs(cre[c]));
-  for (int r = 0; r < nr; r++) my = std::max(my, std::fabs(cim[r]));
-  *c_bound = std::sqrt(mx * mx + my * my) * (1.0 + 0x1p-40);  // rounded up
-}
-
-// computeAll without device allocation (render_hw_noalloc): the plain path
-// only; the coordinate tables go through a static host buffer.
+// computeAll without device allocation (render_hw_noalloc): the plain path only.
 int Mandelbrot::computeAllNoAlloc(EscapeValue* out, size_t n) {
   if (!out || N <= 0) return NM_ERR_ARG;
   if (!useHardware()) return NM_ERR_STATE;  // deep views need the device reference orbit
@@ -761,39 +786,28 @@ int Mandelbrot::computeAllNoAlloc(EscapeValue* out, size_t n) {
   constexpr int kSide = 8192;
   if (nr > kSide || nc > kSide || (uint64_t)nr * nc > (1ull << 19)) return NM_ERR_RANGE;
   static std::mutex mu;
-  static double tab[4 * kSide];
   std::lock_guard<std::mutex> lk(mu);
-  HwFrameView v;
-  v.nr = nr;
-  v.nc = nc;
-  double *cre = tab, *crelo = tab + kSide, *cim = tab + 2 * kSide, *cimlo = tab + 3 * kSide;
-  fillHwTables(center, sz, cre, crelo, cim, cimlo, &v.card_mode, &v.fma_ok, &v.c_bound);
-  v.cre = cre;
-  v.crelo = crelo;
-  v.cim = cim;
-  v.cimlo = cimlo;
-  return render_hw_noalloc(v, N, bailout, out, noalloc_err_);
+  HwFrameHost f;
+  buildHwFrame(f, center, sz);
+  return render_hw_noalloc(f, N, bailout, out, noalloc_err_);
 }
 
-// Per-column / per-row epsilon = descend(Y0 - X[0]) (mandelbrot.cpp:155-159).
-int Mandelbrot::buildSaFrame(SaFrameHost& f, const HPComplex& cen, const HPComplex& s) {
+// Per-column / per-row epsilon = descend(Y0 - X[0]) (mandelbrot.cpp:155-159): made
+// on the device; tables: on the host as well.
+int Mandelbrot::buildSaFrame(SaFrameHost& f, const HPComplex& cen, const HPComplex& s, bool tables) {
   if (!have_ref_) return NM_ERR_STATE;
-  const int L = hp_limbs_for_bits(hp_default_bits());
   f.nr = rows();
   f.nc = cols();
-  f.epsre.resize(f.nc);
-  f.epsim.resize(f.nr);
-  hpf p(L), y(L);
-  for (int c = 0; c < f.nc; c++) {
-    pixel_re(p, cen.re, s.re, (long)(c - cols() / 2));
-    hp_sub(y, p, X[0].re);
-    f.epsre[c] = y.get_d();
-  }
-  for (int r = 0; r < f.nr; r++) {
-    pixel_re(p, cen.im, s.im, (long)(rows() / 2 - r - 1));
-    hp_sub(y, p, X[0].im);
-    f.epsim[r] = y.get_d();
-  }
+  f.hp = frame_hp(cen, s, &X[0]);
+  auto eps_re = [&](int c) { return coordinate(cen.re, s.re, column_offset(c, f.nc), &X[0].re); };
+  auto eps_im = [&](int r) { return coordinate(cen.im, s.im, row_offset(r, f.nr), &X[0].im); };
+  // the largest epsilons are at the ends: truncation keeps the coordinates' order
+  f.emax = std::max(std::fabs(eps_re(0)), std::fabs(eps_re(f.nc - 1))) +
+           std::max(std::fabs(eps_im(0)), std::fabs(eps_im(f.nr - 1)));
+  f.epsre.clear();
+  f.epsim.clear();
+  for (int c = 0; tables && c < f.nc; c++) f.epsre.push_back(eps_re(c));
+  for (int r = 0; tables && r < f.nr; r++) f.epsim.push_back(eps_im(r));
   int m = classify_frame(cen, s, f.nr, f.nc);
   if (m >= 0) {
     f.card_mode = m;
@@ -804,6 +818,7 @@ int Mandelbrot::buildSaFrame(SaFrameHost& f, const HPComplex& cen, const HPCompl
     f.card_mode = CARD_MASK;
     size_t n = (size_t)f.nr * f.nc;
     f.mask.assign((n + 31) / 32, 0u);
+    const int L = f.hp.L;
     std::vector<uint8_t> in(n, 0);
     parallel_for((long)f.nr, [&](long r) {
       hpf pr(L), pi(L);
@@ -875,7 +890,7 @@ int Mandelbrot::render(RenderOpts* opts, bool copy_back) {
       st = buildHwFrame(cache_.h[0]);
     } else {
       cache_.s.resize(1);
-      st = buildSaFrame(cache_.s[0]);
+      st = buildSaFrame(cache_.s[0], center, sz, skipsByTile());
     }
     if (st != NM_OK) return st;
     cache_key_ = key;
@@ -932,7 +947,7 @@ int Mandelbrot::buildFrames(const std::vector<std::string>& widths, FrameSet& se
   if (!have_ref_) return NM_ERR_STATE;
   set.s.assign(widths.size(), SaFrameHost());
   std::vector<int> sts(set.s.size(), NM_OK);
-  parallel_for((long)set.s.size(), [&](long k) { sts[k] = buildSaFrame(set.s[k], center, sizes[k]); }, 1);
+  parallel_for((long)set.s.size(), [&](long k) { sts[k] = buildSaFrame(set.s[k], center, sizes[k], skipsByTile()); }, 1);
   for (int v : sts)
     if (v != NM_OK) return v;
   return NM_OK;
@@ -1054,7 +1069,7 @@ int Mandelbrot::tileFeatures(int T, std::vector<float>& feats, const SaFrameHost
   }
   SaFrameHost own;
   if (!frame) {
-    int st = buildSaFrame(own);
+    int st = buildSaFrame(own, center, sz, true);
     if (st != NM_OK) return st;
     frame = &own;
   }
@@ -1122,7 +1137,7 @@ int Mandelbrot::tileSkips(int T, int mode, SkipNet* net, std::vector<int>& ua, s
   if (st != NM_OK) return st;
   if ((st = eng->set_reference(ref_, ref_serial_)) != NM_OK) return st;
   SaFrameHost f;
-  if ((st = buildSaFrame(f)) != NM_OK) return st;
+  if ((st = buildSaFrame(f, center, sz, true)) != NM_OK) return st;
   RenderOpts o;
   applyLaunch(o);
   const int keep_mode = skip_mode, keep_T = skip_tile;

@@ -175,16 +175,15 @@ class Mandelbrot {
   std::string cache_key_;
   uint64_t cache_serial_ = 0;
   void applyLaunch(RenderOpts& o) const;
-  int buildHwFrame(HwFrameHost& f) { return buildHwFrame(f, center, sz); }
-  int buildSaFrame(SaFrameHost& f) { return buildSaFrame(f, center, sz); }
-  int buildHwFrame(HwFrameHost& f, const HPComplex& c, const HPComplex& s);
-  void fillHwTables(const HPComplex& c, const HPComplex& s, double* cre, double* crelo, double* cim, double* cimlo,
-                    int* card_mode, bool* fma_ok, double* c_bound) const;
+  int buildHwFrame(HwFrameHost& f) const { return buildHwFrame(f, center, sz); }
+  int buildHwFrame(HwFrameHost& f, const HPComplex& c, const HPComplex& s) const;
   // computeAll into out (rows x cols) on the plain path without allocating
   // device memory (render_hw_noalloc); noalloc_err_ holds the last error
   int computeAllNoAlloc(EscapeValue* out, size_t n);
   std::string noalloc_err_;
-  int buildSaFrame(SaFrameHost& f, const HPComplex& c, const HPComplex& s);
+  int buildSaFrame(SaFrameHost& f, const HPComplex& c, const HPComplex& s, bool tables);
+  // the skip mode searches tiles, which reads the epsilon tables on the host
+  bool skipsByTile() const { return skip_mode != SKIP_PIXEL && skip_mode != SKIP_NONE; }
   void invalidate() { rendered_ = false; }
 
  protected:

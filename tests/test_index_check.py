@@ -77,3 +77,12 @@ def test_threshold_tree_search(n):
     L.nm_tree_check.restype = C.c_longlong
     L.nm_tree_check.argtypes = [C.c_int, C.c_uint]
     assert all(L.nm_tree_check(n, seed) == 0 for seed in range(1, 6))
+
+
+@pytest.mark.parametrize("limbs", [4, 8, 16, 40])
+def test_device_coordinates_equal_the_hosts(limbs):
+    """The coordinate tables' fixed-limb arithmetic gives hpfloat.cpp's bits."""
+    L = _lib()
+    L.nm_coords_check.restype = C.c_longlong
+    L.nm_coords_check.argtypes = [C.c_int, C.c_uint, C.c_int]
+    assert all(L.nm_coords_check(limbs, seed, 4000) == 0 for seed in range(1, 9))
