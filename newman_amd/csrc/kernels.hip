@@ -2399,7 +2399,7 @@ class EngineImpl : public Engine {
 
   // the frame records and coordinate tables of a frame set, on the device: a single
   // frame's come with the kernel's arguments, several frames' through the pinned
-  // staging buffer (free again: every render ends with a wait for the stream)
+  // staging buffer
   int make_tables(const std::vector<DevFrame>& df, const std::vector<FrameHp>& hp, int nr, int nc, bool series,
                   const CoordTables& t) {
     const size_t nf = df.size(), fbytes = (nf * sizeof(DevFrame) + 255) & ~(size_t)255;
@@ -2407,6 +2407,9 @@ class EngineImpl : public Engine {
     for (const FrameHp& h : hp) limbs = std::max(limbs, h.limbs);
     const bool one = nf == 1;
     if (!one) {
+      // a call refused after its tables (a block size the kernels do not have) has
+      // not waited for the copies out of the buffer
+      NM_HIP(hipStreamSynchronize(stream));
       const size_t bytes = fbytes + nf * sizeof(FrameHp);
       if ((st = grow(&d_hp, &n_hp_bytes, nf * sizeof(FrameHp)))) return st;
       if (bytes > n_stage_bytes) {
