@@ -144,6 +144,7 @@ struct RenderOpts {
   int chunk_run = 0;      // series path: active-list chunks of 64 consecutive samples (64)
                           // or interleaved runs of 1, 2, 4, 8, 16, 32 (chunk_run_shift);
                           // 0: runs of 4 for deltas on a floatexp series, else 64
+  bool timed = true;      // events around the stages (RenderStats::ms_*; without: 0)
   const int* tile_ua = nullptr;  // series path: per-tile first unstable index (null: per sample)
   int skip_T = 0;                // its tile side
   uint64_t set_serial = 0; // identifies the frame set: the engine keeps its tables

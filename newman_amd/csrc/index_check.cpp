@@ -108,7 +108,8 @@ long long nm_index_check(int nr, int nc, int nframes, int tile, int num_cu, int 
   const int grid = start_grid(total, num_cu, kStartSlots);
   for (int b = 0; b < grid; b++)
     for (uint32_t t = (uint32_t)b; t < ntiles; t += (uint32_t)grid) {
-      R.in(t, ntiles, "tile_count", t);
+      for (uint32_t w = 0; w < (uint32_t)kCountsPerTile; w++)
+        R.in(count_index(t, w), start_counts(total), "start counts", t);
       uint32_t f0, f1;
       tile_frame_span(t, total, inv_frame, &f0, &f1);
       R.in(f0, (uint64_t)nframes, "frames (tile span)", (uint64_t)t * kTile);
@@ -301,7 +302,7 @@ long long nm_index_check(int nr, int nc, int nframes, int tile, int num_cu, int 
     // the split at edge sizes: at most kScanGroups groups of consecutive,
     // non-empty count ranges covering [0, ntiles)
     const uint32_t edge[] = {0u, 1u, kScanRound - 1, kScanRound, kScanRound + 1, kScanGroups * kScanRound,
-                             kScanGroups * kScanRound + 1, 100 * kScanRound + 7, start_tiles(0xFFFFEFFFu), ntiles};
+                             kScanGroups * kScanRound + 1, 100 * kScanRound + 7, start_counts(0xFFFFEFFFu), start_counts(total), ntiles};
     for (uint32_t n : edge) {
       const ScanSplit e = scan_split(n);
       if (e.groups < 1 || e.groups > kScanGroups) R.fail("tile scan of %u counts: %u groups", n, e.groups);

@@ -19,16 +19,16 @@
 // Pipeline per render pass, with no contended device-scope atomic on the hot
 // path (one contended counter serialises at ~10 ns per atomic on this part; the
 // start kernels add one count per wave and tile, four adds per counter):
-//   k_zero      clears the per-workgroup counter slots and the tile counts (a
-//               kernel, so a captured HIP graph holds no memset node)
 //   *_start     tiles of 1024 samples: cardioid/bulb test and up to pre_iter
 //               updates (plain path), or the reference's per-sample series start
 //               (series path: stop index, series skip, escape inside the skip,
 //               first step, and with FP64 deltas the steps a wave's samples can do
 //               together); resolves what it can, marks the rest (one ballot
-//               word per wave), counts per tile
-//   scan        exclusive scan of the tile counts (range totals, then each
-//               range's scan from the earlier ranges' sum; up to 64 workgroups)
+//               word per wave), counts per tile and wave, and clears the claim
+//               counters
+//   scan        exclusive scan of the counts (range totals, then each range's scan
+//               from the earlier ranges' sum; up to 64 workgroups; up to 1 M samples
+//               the scatter sums the counts before its tile itself)
 //   scatter     compacts the marked sample ids into active[] in sample order
 //   *_iterate   persistent waves, one sample per lane; blocks of K steps; the
 //               first escape of a lane in a block records its step and |z|^2
@@ -88,6 +88,7 @@ constexpr int kSeriesIterThreads = 512;
 static_assert(kLdsTail >= 64 && kLdsHead >= 64, "a block of up to 64 steps reads inside one window");
 constexpr int kPartSlots = 6144;        // per-workgroup partial counter slots
 
+constexpr int kQueueStride = 64;  // u32 between claim counters (ChunkClaim): 256 bytes
 // partial-slot ranges of the kernels of one render
 constexpr int kSlotStart = 0;
 constexpr int kSlotIter = 4096;
@@ -102,7 +103,7 @@ struct Common {
   double4* state;  // per sample: plain (x, y, cx, cy); series: (dr, di) as double2[]
   int2* state_i;   // per sample, series path: (it, m)
   uint64_t* hand;  // hand-on bits (hand_word)
-  uint32_t* tile_count;
+  uint32_t* counts;  // marked samples per tile and wave (count_index)
   uint32_t* active;
   const uint32_t* nactive;  // written by the scan
   unsigned long long* part;
@@ -251,8 +252,9 @@ __device__ __forceinline__ unsigned long long wave_sum(unsigned long long v) {
   return v;
 }
 
-// Adds v (per thread) into the workgroup's partial slot: wave reduction, LDS
-// accumulation, one plain store per workgroup.  Called by all threads.
+// Stores the workgroup's sums of v (per thread) in its partial slot: wave reduction,
+// LDS accumulation, one plain store per workgroup and counter (the others 0), so
+// nothing has to clear the slots.  Called by all threads, once per launch.
 __device__ __forceinline__ void block_partial(unsigned long long* part, int slot, const unsigned long long* v,
                                               const int* idx, int n) {
   __shared__ unsigned long long acc[C_COUNT];
@@ -263,7 +265,7 @@ __device__ __forceinline__ void block_partial(unsigned long long* part, int slot
     if (lane_id() == 0 && s) atomicAdd(&acc[idx[k]], s);
   }
   __syncthreads();
-  if (threadIdx.x < C_COUNT) part[(size_t)slot * C_COUNT + threadIdx.x] += acc[threadIdx.x];
+  if (threadIdx.x < C_COUNT) part[(size_t)slot * C_COUNT + threadIdx.x] = acc[threadIdx.x];
 }
 
 // ---- double-double arithmetic for the plain path's cardioid test -----------
@@ -590,10 +592,15 @@ __device__ __forceinline__ uint32_t store_hand(uint64_t* hand, uint32_t gid, boo
   return (uint32_t)__popcll(w);
 }
 
-// A wave's count of marked samples of a tile into tile_count[tile] (cleared by
-// k_zero): one atomic add per wave and tile, no barrier between the waves.
-__device__ __forceinline__ void tile_count_add(uint32_t* tile_count, uint32_t tile, uint32_t wave_count) {
-  if (lane_id() == 0 && wave_count) atomicAdd(&tile_count[tile], wave_count);
+// A wave's count of marked samples of a tile.
+__device__ __forceinline__ void store_count(uint32_t* counts, uint32_t tile, uint32_t wave_count) {
+  if (lane_id() == 0) counts[count_index(tile, threadIdx.x >> 6)] = wave_count;
+}
+// The claim counters of the iterate launch that follows, cleared by the start
+// launch's first workgroup.
+__device__ __forceinline__ void clear_claims(unsigned long long* part) {
+  if (blockIdx.x == 0 && threadIdx.x < (unsigned)kQueues)
+    ((uint32_t*)(part + (size_t)kPartSlots * C_COUNT))[threadIdx.x * kQueueStride] = 0u;
 }
 
 template <bool FMA2, bool GROUPED>
@@ -601,6 +608,7 @@ __global__ __launch_bounds__(kThreads) void k_plain_start(PlainArgs a) {
   const Common& c = a.c;
   __shared__ double2 ltab[kLog2Tab];
   load_log2tab(ltab);
+  clear_claims(c.part);
   StartCounts n;
   const uint32_t ntiles = start_tiles(c.total);
   const int pre = min(a.pre_iter, c.N);
@@ -624,7 +632,7 @@ __global__ __launch_bounds__(kThreads) void k_plain_start(PlainArgs a) {
         mine += store_hand(c.hand, gid, want);
       }
     }
-    tile_count_add(c.tile_count, tile, mine);
+    store_count(c.counts, tile, mine);
   }
   const unsigned long long v[4] = {n.ncard, n.nres, n.executed, n.credited};
   const int idx[4] = {C_CARDIOID, C_SA_RES, C_EXEC_START, C_CREDITED};
@@ -632,14 +640,14 @@ __global__ __launch_bounds__(kThreads) void k_plain_start(PlainArgs a) {
 }
 
 // ============================================================ compaction
-// exclusive scan of tile_count (in place), total -> *nactive, in two launches
-// over the groups of scan_split: k_tile_sums writes each group's total of
-// counts, then k_scan_tiles starts each group at the sum of the earlier groups'
-// totals. A workgroup takes a round of 16384 consecutive counts at a time: 16
-// per thread (four 16-byte loads), wave scans, a carry between rounds; the next
-// round's loads are issued before this round's scan, so one memory latency is
-// paid per round at most. (One workgroup over all of a 512-frame 640x480 set's
-// 153,600 counts took 34 us, ten rounds back to back.)
+// exclusive scan of the start counts (in place), total -> *nactive, over the groups
+// of scan_split: k_tile_sums writes each group's total of counts, then k_scan_tiles
+// starts each group at the sum of the earlier groups' totals (one group: no sums
+// needed). A workgroup takes a round of 16384 consecutive counts at a time: 16 per
+// thread (four 16-byte loads), wave scans, a carry between rounds; the next round's
+// loads are issued before this round's scan, so one memory latency is paid per
+// round at most. (One workgroup over all of a 512-frame 640x480 set's 153,600 tile
+// counts took 34 us, ten rounds back to back.)
 constexpr int kScanPer = 16;
 static_assert(kScanRound == 1024 * kScanPer, "a scan round is 16 counts for each of 1024 threads");
 __device__ __forceinline__ void scan_load(const uint32_t* tc, uint32_t i0, uint32_t hi, uint32_t v[kScanPer]) {
@@ -749,30 +757,47 @@ __global__ __launch_bounds__(1024) void k_scan_tiles(uint32_t* tile_count, uint3
 // of set bits; then for each word (scalar) every lane writes its own sample's id
 // at hand_position (consecutive lanes, consecutive positions).  A wave's next
 // tile (words and offset) is loaded before it writes the current one, so the
-// loads' latency overlaps the stores.
+// loads' latency overlaps the stores.  SELF (at most kSelfScanTiles tiles): the
+// offset is the sum of the earlier tiles' counts, at most 16 KB read by the wave
+// itself, and the last tile's wave stores the total; a frame of that size spends
+// less here than on the launches of a scan (3.5 us each at 640 x 480).
 static_assert(kHandWordsPerTile == 16, "k_scatter: 16 words per tile, one per lane of lanes 0..15");
-__device__ __forceinline__ void scatter_load(const uint64_t* hand, const uint32_t* tile_off, uint32_t tile,
+static_assert(kCountsPerTile == 4, "k_scatter: a tile's counts are one 16-byte load");
+__device__ __forceinline__ void scatter_load(const uint64_t* hand, const uint32_t* off_at, uint32_t tile,
                                              uint32_t ntiles, uint32_t lane, uint64_t& w, uint32_t& off) {
   w = 0ull;
   off = 0u;
   if (tile < ntiles) {  // wave-uniform
     if (lane < (uint32_t)kHandWordsPerTile) w = hand[tile * kHandWordsPerTile + lane];
-    off = tile_off[tile];
+    if (off_at) off = off_at[count_index(tile, 0)];
   }
 }
-__global__ __launch_bounds__(kThreads) void k_scatter(const uint64_t* hand, const uint32_t* tile_off, uint32_t total,
-                                                      uint32_t* active) {
+template <bool SELF>
+__global__ __launch_bounds__(kThreads) void k_scatter(const uint64_t* hand, const uint32_t* counts, uint32_t total,
+                                                      uint32_t* active, uint32_t* nactive) {
   const uint32_t ntiles = start_tiles(total);
   const uint32_t lane = (uint32_t)lane_id();
   const uint32_t waves = gridDim.x * (kThreads / 64);
   uint32_t tile = blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);
+  const uint32_t* off_at = SELF ? nullptr : counts;  // scanned: each tile's offset is at its first count
   uint64_t wnext;
   uint32_t offnext;
-  scatter_load(hand, tile_off, tile, ntiles, lane, wnext, offnext);
+  scatter_load(hand, off_at, tile, ntiles, lane, wnext, offnext);
   for (; tile < ntiles; tile += waves) {
     const uint64_t w = wnext;
-    const uint32_t off = __builtin_amdgcn_readfirstlane(offnext);
-    scatter_load(hand, tile_off, tile + waves, ntiles, lane, wnext, offnext);
+    uint32_t off;
+    if constexpr (SELF) {
+      uint32_t s = 0;
+      for (uint32_t t = lane; t < tile; t += 64) {
+        const uint4 q = ((const uint4*)counts)[t];
+        s += q.x + q.y + q.z + q.w;
+      }
+      for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+      off = __builtin_amdgcn_readfirstlane(s);
+    } else {
+      off = __builtin_amdgcn_readfirstlane(offnext);
+    }
+    scatter_load(hand, off_at, tile + waves, ntiles, lane, wnext, offnext);
     const uint32_t n = (uint32_t)__popcll(w);
     uint32_t x = n;  // inclusive scan over lanes 0..15
     for (int o = 1; o < kHandWordsPerTile; o <<= 1) {
@@ -781,6 +806,7 @@ __global__ __launch_bounds__(kThreads) void k_scatter(const uint64_t* hand, cons
     }
     const uint32_t before = x - n;
     const uint32_t m = __builtin_amdgcn_readlane(x, kHandWordsPerTile - 1);  // the tile's marked samples
+    if (SELF && tile == ntiles - 1 && lane == 0) *nactive = off + m;
     if (m <= kScatterSparse) {  // wave-uniform: one store per 64 marked samples
       const uint32_t wlo = (uint32_t)w, whi = (uint32_t)(w >> 32);
       for (uint32_t p0 = 0; p0 < m; p0 += 64) {
@@ -859,7 +885,6 @@ __device__ __forceinline__ void retire_push(const Common& c, RetireEntry* q, int
 // time and the last ones ran nearly alone on their SIMDs; claiming lets fast
 // waves take more.  One atomic per 64 samples; counters sharing one cache line
 // had serialised the claims (~100 ns each).
-constexpr int kQueueStride = 64;  // u32 between counters: 256 bytes
 // d_part (u64 words): the partial counter slots, the claim counters, then the
 // tile scan's group totals (kScanGroups u32)
 constexpr int kPartWords = kPartSlots * C_COUNT + kQueues * kQueueStride / 2 + kScanGroups / 2;
@@ -1541,6 +1566,7 @@ template <bool FXS, bool COH>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_series_start(SeriesArgs a) {
   const Common& c = a.c;
   unsigned long long ncard = 0, nres = 0, skipped = 0, credited = 0, executed = 0, rebased = 0;
+  clear_claims(c.part);
   const uint32_t ntiles = start_tiles(c.total);
   for (uint32_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
     uint32_t mine = 0;
@@ -1670,7 +1696,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(6, 8))
       }
       mine += store_hand(c.hand, gid, want);
     }
-    tile_count_add(c.tile_count, tile, mine);
+    store_count(c.counts, tile, mine);
   }
   const unsigned long long v[6] = {ncard, nres, skipped, credited, executed, rebased};
   const int idx[6] = {C_CARDIOID, C_SA_RES, C_SKIPPED, C_CREDITED, C_EXEC_START, C_REBASED};
@@ -1889,7 +1915,10 @@ void k_series_iterate(SeriesArgs a) {
   cm.init(total, a.run_shift);
   ChunkClaim q;
   q.init(c.part, cm.nch);
-  if (blockIdx.x >= q.base) return;  // no chunk for any wave of the workgroup
+  if (blockIdx.x >= q.base) {  // no chunk for any wave of the workgroup
+    block_partial(c.part, kSlotIter + blockIdx.x, nullptr, nullptr, 0);
+    return;
+  }
   // entries past Zd's allocation read 0
   __shared__ SeriesLds lds;
   RetireEntry* const rq = lds.retire[threadIdx.x >> 6];
@@ -2094,18 +2123,26 @@ __global__ void k_downsample(const EscapeValue* fine, int nr, int nc, int sc, Es
   }
 }
 
-// sum of reported iterations over the output (credited work)
-// partial slots -> one total per counter (one workgroup)
-// one workgroup of 1024: each thread sums every counter of its slots (one
-// contiguous C_COUNT-entry record per slot), then one wave reduction per counter
+// What a render's counters come back in (pinned host memory: the reduction stores
+// it there, and the wait for the results covers it).
+struct HostTotals {
+  unsigned long long count[C_COUNT];
+  uint32_t nactive;
+};
+// the partial slots that the pass's workgroups wrote (start: slots 0 .. ns - 1,
+// iterate: kSlotIter .. kSlotIter + ni - 1) -> one total per counter.  One workgroup
+// of 1024: each thread sums every counter of its slots (one contiguous
+// C_COUNT-entry record per slot), then one wave reduction per counter
 constexpr int kReduceThreads = 1024;
-__global__ __launch_bounds__(kReduceThreads) void k_reduce_partials(const unsigned long long* part, int nslots,
-                                                                    unsigned long long* totals) {
+__global__ __launch_bounds__(kReduceThreads) void k_reduce_partials(const unsigned long long* part, int ns, int ni,
+                                                                    const uint32_t* nactive, HostTotals* totals) {
   __shared__ unsigned long long acc[kReduceThreads / 64][C_COUNT];
   unsigned long long v[C_COUNT] = {};
-  for (int sl = threadIdx.x; sl < nslots; sl += blockDim.x)
+  for (int i = threadIdx.x; i < ns + ni; i += blockDim.x) {
+    const size_t sl = i < ns ? i : kSlotIter + (i - ns);
 #pragma unroll
-    for (int k = 0; k < C_COUNT; k++) v[k] += part[(size_t)sl * C_COUNT + k];
+    for (int k = 0; k < C_COUNT; k++) v[k] += part[sl * C_COUNT + k];
+  }
 #pragma unroll
   for (int k = 0; k < C_COUNT; k++) {
     const unsigned long long sk = wave_sum(v[k]);
@@ -2115,21 +2152,14 @@ __global__ __launch_bounds__(kReduceThreads) void k_reduce_partials(const unsign
   if (threadIdx.x < C_COUNT) {
     unsigned long long t = 0;
     for (int w = 0; w < kReduceThreads / 64; w++) t += acc[w][threadIdx.x];
-    totals[threadIdx.x] = t;
+    totals->count[threadIdx.x] = t;
   }
+  if (threadIdx.x == C_COUNT) totals->nactive = *nactive;
 }
 
-// clears the counter slots p[0, n) and the tile counts q[0, m)
-__device__ __forceinline__ void zero_counters(unsigned long long* p, int n, uint32_t* q, uint32_t m) {
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = 0ull;
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < m; i += gridDim.x * blockDim.x) q[i] = 0u;
-}
-__global__ void k_zero(unsigned long long* p, int n, uint32_t* q, uint32_t m) { zero_counters(p, n, q, m); }
-// the same, and the safe radii of orbit indices 0 .. mend (they depend on the
-// frames' largest |e| and the bailout, so they are made on each pass)
-__global__ void k_zero_safe(unsigned long long* p, int n, uint32_t* q, uint32_t m, const double2* Zd, int mend,
-                            double radius, double emax, double* safe) {
-  zero_counters(p, n, q, m);
+// the safe radii of orbit indices 0 .. mend (they depend on the frames' largest |e|
+// and the bailout, so they are made on each pass)
+__global__ void k_safe(const double2* Zd, int mend, double radius, double emax, double* safe) {
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i <= mend; i += gridDim.x * blockDim.x)
     safe_radius(Zd, mend, radius, emax, safe, i);
 }
@@ -2162,26 +2192,22 @@ static int tile_grid(uint64_t total, int num_cu) {
   return start_grid(total, num_cu, (uint64_t)(kSlotIter - kSlotStart));
 }
 
-static void launch_zero(hipStream_t stream, unsigned long long* part, const PlainArgs& a, uint32_t ntiles) {
-  hipLaunchKernelGGL(k_zero, dim3(256), dim3(256), 0, stream, part, kPartWords, a.c.tile_count, ntiles);
-}
-static void launch_zero(hipStream_t stream, unsigned long long* part, const SeriesArgs& a, uint32_t ntiles) {
-  if (a.safe)
-    hipLaunchKernelGGL(k_zero_safe, dim3(512), dim3(256), 0, stream, part, kPartWords, a.c.tile_count, ntiles, a.Zd,
-                       a.mend, a.radius, a.emax, a.safe);
-  else
-    hipLaunchKernelGGL(k_zero, dim3(256), dim3(256), 0, stream, part, kPartWords, a.c.tile_count, ntiles);
+static void launch_safe(hipStream_t, const PlainArgs&) {}
+static void launch_safe(hipStream_t stream, const SeriesArgs& a) {
+  if (!a.safe) return;
+  hipLaunchKernelGGL(k_safe, dim3(std::min(512, a.mend / 256 + 1)), dim3(256), 0, stream, a.Zd, a.mend, a.radius,
+                     a.emax, a.safe);
 }
 
-// The kernels of one pass on `stream`: zero the counters (part: kPartWords
-// words), start, scan, scatter, iterate (and emit for tiled sample orders).  evs != nullptr records an event before each stage (eager timing);
-// under stream capture it is null.  Returns the first launch error.
+// The kernels of one pass on `stream` (part: kPartWords words): the safe radii
+// (series path), start, scan, scatter, iterate (and emit for tiled sample orders).
+// evs != nullptr records an event before each stage (eager timing); under stream
+// capture it is null.  Returns the first launch error.
 template <class Args, class StartFn, class IterFn>
 static hipError_t launch_pass_on(hipStream_t stream, int num_cu, unsigned long long* part, uint32_t* nactive,
                                  Args& args, StartFn start, IterFn iter, int waves, EscapeValue* emit_to,
                                  hipEvent_t* evs) {
   const Common& c = args.c;
-  const uint32_t ntiles = (uint32_t)((c.total + kTile - 1) / kTile);
   const int gtile = tile_grid(c.total, num_cu);
   // waves = persistent waves per SIMD: 4 per CU for each 256 threads
   const int ti = iter_threads<Args>();
@@ -2192,18 +2218,25 @@ static hipError_t launch_pass_on(hipStream_t stream, int num_cu, unsigned long l
     expr;                                    \
     if ((e = hipGetLastError()) != hipSuccess) return e; \
   } while (0)
-  NM_LAUNCH_OK(launch_zero(stream, part, args, ntiles));
   if (evs && (e = hipEventRecord(evs[0], stream)) != hipSuccess) return e;
+  NM_LAUNCH_OK(launch_safe(stream, args));
   NM_LAUNCH_OK(hipLaunchKernelGGL(start, dim3(gtile), dim3(kThreads), 0, stream, args));
   if (evs && (e = hipEventRecord(evs[1], stream)) != hipSuccess) return e;
-  const ScanSplit sp = scan_split(ntiles);
-  uint32_t* gsum = scan_group_sums(part);
-  NM_LAUNCH_OK(hipLaunchKernelGGL(k_tile_sums, dim3(sp.groups), dim3(1024), 0, stream, (const uint32_t*)c.tile_count,
-                                  ntiles, sp.per, gsum));
-  NM_LAUNCH_OK(hipLaunchKernelGGL(k_scan_tiles, dim3(sp.groups), dim3(1024), 0, stream, c.tile_count, ntiles, sp.per,
-                                  (const uint32_t*)gsum, nactive));
-  NM_LAUNCH_OK(hipLaunchKernelGGL(k_scatter, dim3(gtile), dim3(kThreads), 0, stream, (const uint64_t*)c.hand,
-                                  (const uint32_t*)c.tile_count, c.total, c.active));
+  if (start_tiles(c.total) <= kSelfScanTiles) {
+    NM_LAUNCH_OK(hipLaunchKernelGGL(k_scatter<true>, dim3(gtile), dim3(kThreads), 0, stream, (const uint64_t*)c.hand,
+                                    (const uint32_t*)c.counts, c.total, c.active, nactive));
+  } else {
+    const uint32_t nc = start_counts(c.total);
+    const ScanSplit sp = scan_split(nc);
+    uint32_t* gsum = scan_group_sums(part);
+    if (sp.groups > 1)
+      NM_LAUNCH_OK(hipLaunchKernelGGL(k_tile_sums, dim3(sp.groups), dim3(1024), 0, stream, (const uint32_t*)c.counts,
+                                      nc, sp.per, gsum));
+    NM_LAUNCH_OK(hipLaunchKernelGGL(k_scan_tiles, dim3(sp.groups), dim3(1024), 0, stream, c.counts, nc, sp.per,
+                                    (const uint32_t*)gsum, nactive));
+    NM_LAUNCH_OK(hipLaunchKernelGGL(k_scatter<false>, dim3(gtile), dim3(kThreads), 0, stream, (const uint64_t*)c.hand,
+                                    (const uint32_t*)c.counts, c.total, c.active, nactive));
+  }
   if (evs && (e = hipEventRecord(evs[2], stream)) != hipSuccess) return e;
   NM_LAUNCH_OK(hipLaunchKernelGGL(iter, dim3(giter), dim3(ti), 0, stream, args));
   if (evs && (e = hipEventRecord(evs[3], stream)) != hipSuccess) return e;
@@ -2228,7 +2261,7 @@ class EngineImpl : public Engine {
  public:
   hipStream_t stream = nullptr;
   std::vector<hipEvent_t> evpool;  // stage boundaries of timed passes (grow-only)
-  unsigned long long* d_totals = nullptr;  // C_COUNT counter totals
+  HostTotals* h_totals = nullptr;          // the last render's counters (pinned)
   int device = 0;
   int num_cu = 256;
   std::string err;
@@ -2293,7 +2326,7 @@ class EngineImpl : public Engine {
     num_cu = prop.multiProcessorCount;
     NM_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
     NM_HIP(fill_log2_table());
-    NM_HIP(hipMalloc((void**)&d_totals, sizeof(unsigned long long) * C_COUNT));
+    NM_HIP(hipHostMalloc((void**)&h_totals, sizeof(HostTotals), hipHostMallocDefault));
     NM_HIP(hipMalloc((void**)&d_part, sizeof(unsigned long long) * kPartWords));  // slots + claim counters
     NM_HIP(hipMalloc((void**)&d_nactive, 256));
     return NM_OK;
@@ -2436,13 +2469,12 @@ class EngineImpl : public Engine {
   int prepare_common(Common& c, uint64_t total, const RenderOpts& opt) {
     // sample ids and the plain iterate kernel's chunk positions (ChunkMap) stay below 2^32
     if (total == 0 || total >= 0xFFFFF000ull) return NM_ERR_RANGE;
-    uint64_t ntiles = (total + kTile - 1) / kTile;
     int st;
     if ((st = grow(&d_out, &n_out_bytes, total * sizeof(EscapeValue)))) return st;
     if ((st = grow(&d_hand, &n_hand_bytes, (uint64_t)hand_words((uint32_t)total) * 8))) return st;
     if ((st = grow(&d_state, &n_state_bytes, total * sizeof(double4)))) return st;
     if ((st = grow(&d_state_i, &n_state_i_bytes, total * sizeof(int2)))) return st;
-    if ((st = grow(&d_tiles, &n_tiles_bytes, ntiles * 4))) return st;
+    if ((st = grow(&d_tiles, &n_tiles_bytes, (uint64_t)start_counts((uint32_t)total) * 4))) return st;
     if ((st = grow(&d_active, &n_active_bytes, total * 4))) return st;
     c.frames = (const DevFrame*)d_frames;
     c.total = (uint32_t)total;
@@ -2450,7 +2482,7 @@ class EngineImpl : public Engine {
     c.state = (double4*)d_state;
     c.state_i = (int2*)d_state_i;
     c.hand = (uint64_t*)d_hand;
-    c.tile_count = (uint32_t*)d_tiles;
+    c.counts = (uint32_t*)d_tiles;
     c.active = (uint32_t*)d_active;
     c.nactive = d_nactive;
     c.part = d_part;
@@ -2477,17 +2509,17 @@ class EngineImpl : public Engine {
     return NM_OK;
   }
 
-  // The pass `repeats` times back to back (one host synchronisation at the end);
-  // then counters and output.  Without opt.graph every pass runs eagerly with
+  // The pass `repeats` times back to back, then counters and output, and one host
+  // synchronisation.  Without opt.graph every pass runs eagerly with
   // per-stage events; with it the first pass runs eagerly, the pass is captured
   // once into a HIP graph and the other repeats replay it (timed as a whole).
   template <class Args, class StartFn, class IterFn>
   int run(Args& args, StartFn start, IterFn iter, int waves, const RenderOpts& opt, RenderStats* stats,
           uint64_t nout, EscapeValue* host_out, EscapeValue* emit_to) {
     const int repeats = std::max(1, opt.repeats);
-    const bool use_graph = opt.graph && repeats > 1;
-    int st;
-    if ((st = ensure_events(use_graph ? 5 + 2 * (size_t)repeats : 5 * (size_t)repeats))) return st;
+    const bool use_graph = opt.graph && repeats > 1, timed = opt.timed || use_graph;
+    int st = NM_OK;
+    if (timed && (st = ensure_events(use_graph ? 5 + 2 * (size_t)repeats : 5 * (size_t)repeats))) return st;
     hipEvent_t* ev = evpool.data();
     const int eager = use_graph ? 1 : repeats;
     hipGraph_t graph = nullptr;
@@ -2510,7 +2542,7 @@ class EngineImpl : public Engine {
       }
     }
     for (int rep = 0; rep < eager && st == NM_OK; rep++)
-      st = launch_pass(args, start, iter, waves, emit_to, ev + 5 * rep);
+      st = launch_pass(args, start, iter, waves, emit_to, timed ? ev + 5 * rep : nullptr);
     if (use_graph) {
       for (int rep = 1; rep < repeats && st == NM_OK; rep++) {
         hipEvent_t* e = ev + 5 + 2 * (rep - 1);
@@ -2520,13 +2552,28 @@ class EngineImpl : public Engine {
         if (e3 != hipSuccess) st = fail("graph replay", e3);
       }
     }
+    // the counters and the results follow the pass without a wait in between
+    const EscapeValue* result = emit_to ? emit_to : (const EscapeValue*)d_out;
+    hipError_t ce = hipSuccess;
+    if (st == NM_OK) {
+      hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(kReduceThreads), 0, stream, (const unsigned long long*)d_part,
+                         tile_grid(args.c.total, num_cu), iterate_grid(num_cu, waves, iter_threads<Args>()),
+                         (const uint32_t*)d_nactive, h_totals);
+      ce = hipGetLastError();
+      if (ce == hipSuccess && host_out)
+        ce = hipMemcpyAsync(host_out, result, nout * sizeof(EscapeValue), hipMemcpyDeviceToHost, stream);
+    }
     hipError_t se = hipStreamSynchronize(stream);
     if (exec) (void)hipGraphExecDestroy(exec);
     if (graph) (void)hipGraphDestroy(graph);
     if (st) return st;
+    if (ce != hipSuccess) return fail("counters and results", ce);
     if (se != hipSuccess) return fail("hipStreamSynchronize", se);
+    tag_++;
+    last_result = result;
+    last_nout = nout;
     double ms[4] = {};
-    for (int rep = 0; rep < eager; rep++)
+    for (int rep = 0; timed && rep < eager; rep++)
       for (int k = 0; k < 4; k++) {
         float t = 0;
         NM_HIP(hipEventElapsedTime(&t, ev[5 * rep + k], ev[5 * rep + k + 1]));
@@ -2538,20 +2585,8 @@ class EngineImpl : public Engine {
       NM_HIP(hipEventElapsedTime(&t, ev[5 + 2 * (rep - 1)], ev[5 + 2 * (rep - 1) + 1]));
       ms_graph += t / (repeats - 1);
     }
-    const EscapeValue* result = emit_to ? emit_to : (const EscapeValue*)d_out;
-    tag_++;
-    last_result = result;
-    last_nout = nout;
-    hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(kReduceThreads), 0, stream, (const unsigned long long*)d_part,
-                       kPartSlots, d_totals);
-    NM_HIP(hipGetLastError());
-    uint32_t nact = 0;
-    unsigned long long h[C_COUNT] = {};
-    NM_HIP(hipMemcpyAsync(h, d_totals, sizeof h, hipMemcpyDeviceToHost, stream));
-    NM_HIP(hipMemcpyAsync(&nact, d_nactive, 4, hipMemcpyDeviceToHost, stream));
-    if (host_out)
-      NM_HIP(hipMemcpyAsync(host_out, result, nout * sizeof(EscapeValue), hipMemcpyDeviceToHost, stream));
-    NM_HIP(hipStreamSynchronize(stream));
+    const unsigned long long* h = h_totals->count;
+    const uint32_t nact = h_totals->nactive;
     if (stats) {
       stats->samples = nout;
       stats->n_cardioid = h[C_CARDIOID];
@@ -3049,7 +3084,8 @@ constexpr size_t na_align(size_t b) { return (b + 255) & ~(size_t)255; }
 constexpr size_t na_bytes(uint64_t n, uint64_t nr, uint64_t nc) {
   return na_align((2 * nc + 2 * nr) * sizeof(double)) + na_align(sizeof(DevFrame)) +
          na_align(n * sizeof(EscapeValue)) + na_align(n * sizeof(double4)) +
-         na_align((n + kTile - 1) / kTile * kHandWordsPerTile * 8) + na_align((n + kTile - 1) / kTile * 4) +
+         na_align((n + kTile - 1) / kTile * kHandWordsPerTile * 8) +
+         na_align((n + kTile - 1) / kTile * kCountsPerTile * 4) +
          na_align(n * 4) +
          na_align((size_t)kPartWords * sizeof(unsigned long long)) + na_align(4);
 }
@@ -3131,7 +3167,7 @@ int render_hw_noalloc(const HwFrameHost& f, int N, double bailout, EscapeValue* 
   EscapeValue* out = (EscapeValue*)take(n * sizeof(EscapeValue));
   double4* state = (double4*)take(n * sizeof(double4));
   uint64_t* hand = (uint64_t*)take((size_t)hand_words((uint32_t)n) * 8);
-  uint32_t* tiles = (uint32_t*)take((n + kTile - 1) / kTile * 4);
+  uint32_t* tiles = (uint32_t*)take((size_t)start_counts((uint32_t)n) * 4);
   uint32_t* active = (uint32_t*)take(n * 4);
   unsigned long long* part = (unsigned long long*)take((size_t)kPartWords * sizeof(unsigned long long));
   uint32_t* nactive = (uint32_t*)take(4);
@@ -3166,7 +3202,7 @@ int render_hw_noalloc(const HwFrameHost& f, int N, double bailout, EscapeValue* 
   c.state = state;
   c.state_i = nullptr;  // the plain path keeps no per-sample count
   c.hand = hand;
-  c.tile_count = tiles;
+  c.counts = tiles;
   c.active = active;
   c.nactive = nactive;
   c.part = part;

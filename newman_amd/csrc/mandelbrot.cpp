@@ -569,6 +569,7 @@ int Mandelbrot::findProbeGPU(Engine* eng) {
   applyLaunch(o);
   o.tile = 0;
   o.graph = false;
+  o.timed = false;
   o.repeats = 1;
   o.delta_mode = DELTA_FP64;
   std::vector<EscapeValue> outa((size_t)3 * nca), outb((size_t)nrb);
@@ -872,6 +873,7 @@ void Mandelbrot::applyLaunch(RenderOpts& o) const {
 int Mandelbrot::render(RenderOpts* opts, bool copy_back) {
   if (N <= 0 || rows() <= 0 || cols() <= 0) return NM_ERR_ARG;
   RenderOpts o = opts ? *opts : RenderOpts();
+  o.timed = opts != nullptr;  // a call without options returns no times
   applyLaunch(o);
   EscapeValue* out = copy_back ? grid.values.data() : nullptr;
   const bool hw = useHardware();

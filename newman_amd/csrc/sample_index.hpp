@@ -84,6 +84,14 @@ __host__ __device__ inline void tile_frame_span(uint32_t tile, uint32_t total, d
 constexpr int kHandWordsPerTile = kTile / 64;
 __host__ __device__ inline uint32_t hand_words(uint32_t total) { return start_tiles(total) * kHandWordsPerTile; }
 __host__ __device__ inline uint32_t hand_word(uint32_t gid) { return gid >> 6; }
+// The start kernels' counts of marked samples: one per wave of a tile, stored
+// plainly (nothing to clear, no atomics).
+constexpr int kCountsPerTile = kThreads / 64;
+__host__ __device__ inline uint32_t start_counts(uint32_t total) { return start_tiles(total) * kCountsPerTile; }
+__host__ __device__ inline uint32_t count_index(uint32_t tile, uint32_t wave) { return tile * kCountsPerTile + wave; }
+// up to this many tiles (1 M samples) the scatter's waves sum the earlier tiles'
+// counts themselves, and no scan is launched
+constexpr uint32_t kSelfScanTiles = 1024;
 // k_scatter: the active-list position of bit l of word k of a tile, given the
 // tile's offset (the exclusive scan of the tile counts) and the set bits of the
 // tile's earlier words (before); sample ids keep their order
@@ -111,7 +119,7 @@ __host__ __device__ inline uint32_t select_bit(uint64_t w, uint32_t r) {
   return pos;
 }
 
-// ---- the exclusive scan of the per-tile counts: rounds of kScanRound counts
+// ---- the exclusive scan of the per-wave counts: rounds of kScanRound counts
 // (one 1024-thread workgroup pass), `per` consecutive rounds to each of `groups`
 // workgroups (at most kScanGroups); group g covers counts [g per kScanRound,
 // min((g + 1) per kScanRound, ntiles)), and every group has at least one count

@@ -36,3 +36,18 @@ def test_queue_lengths(gpu, n, deep):
     _check(m.grid()[0], want)
     # cardioid and bulb samples are counted apart from credited work
     assert st["credited"] == int(want["iterations"].astype(np.int64).sum()) - st["n_cardioid"] * view[0]
+
+
+@pytest.mark.parametrize("nr,nc", [(1023, 1024), (1024, 1024), (1024, 1025), (4100, 4100)])
+def test_scatter_around_the_scan(gpu, nr, nc):
+    """Up to 1024 start tiles the scatter sums the counts before its tile itself;
+    beyond, the scan does, in one group of 16384 counts or (16.8 M samples) two."""
+    m, o = gpu.Mandelbrot(nr, nc), O.OView(nr, nc)
+    view = (60, "-0.75", "0.1", "3.0")
+    m.set_view(*view)
+    o.set_view(*view)
+    st = m.render()
+    rows = np.arange(nr, dtype=np.int32)[::1 if nr < 2000 else 16]
+    want = o.render_rows(rows)
+    _check(m.grid()[rows], want)
+    assert st["n_iterated"] + st["n_cardioid"] + st["n_sa_resolved"] == nr * nc
