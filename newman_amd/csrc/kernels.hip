@@ -56,6 +56,7 @@
 #include "colour.hpp"
 #include "coords.hpp"
 #include "engine.hpp"
+#include "hostcopy.hpp"
 #include "sample_index.hpp"
 #include "video.hpp"
 
@@ -2261,6 +2262,7 @@ class EngineImpl : public Engine {
  public:
   hipStream_t stream = nullptr;
   std::vector<hipEvent_t> evpool;  // stage boundaries of timed passes (grow-only)
+  HostCopy copier;
   HostTotals* h_totals = nullptr;          // the last render's counters (pinned)
   int device = 0;
   int num_cu = 256;
@@ -2561,7 +2563,7 @@ class EngineImpl : public Engine {
                          (const uint32_t*)d_nactive, h_totals);
       ce = hipGetLastError();
       if (ce == hipSuccess && host_out)
-        ce = hipMemcpyAsync(host_out, result, nout * sizeof(EscapeValue), hipMemcpyDeviceToHost, stream);
+        ce = copier.copy(stream, host_out, result, nout * sizeof(EscapeValue));
     }
     hipError_t se = hipStreamSynchronize(stream);
     if (exec) (void)hipGraphExecDestroy(exec);
@@ -2985,7 +2987,7 @@ class EngineImpl : public Engine {
     if (colour_launch(stream, num_cu, grid, nr, nc, sc, N, d_pal, smooth, (uint8_t*)d_img))
       return fail("k_colour launch", hipGetLastError());
     NM_HIP(hipEventRecord(evpool[1], stream));
-    if (nout) NM_HIP(hipMemcpyAsync(host_out, d_img, nout * 3, hipMemcpyDeviceToHost, stream));
+    if (nout) NM_HIP(copier.copy(stream, host_out, d_img, nout * 3));
     NM_HIP(hipStreamSynchronize(stream));
     float t = 0.0f;
     NM_HIP(hipEventElapsedTime(&t, evpool[0], evpool[1]));
@@ -3017,8 +3019,7 @@ class EngineImpl : public Engine {
     if (video_launch((void*)stream, kp, kn, kr, kc, nr, nc, ks, rate, wide, (uint8_t*)d_vframes))
       return fail("k_video_frames launch", hipGetLastError());
     NM_HIP(hipEventRecord(evpool[1], stream));
-    NM_HIP(hipMemcpyAsync(out, d_vframes, obytes, hipMemcpyDeviceToHost, stream));
-    NM_HIP(hipStreamSynchronize(stream));
+    NM_HIP(copier.copy(stream, out, d_vframes, obytes));
     float t = 0.0f;
     NM_HIP(hipEventElapsedTime(&t, evpool[0], evpool[1]));
     if (ms) *ms = t;
@@ -3036,8 +3037,7 @@ class EngineImpl : public Engine {
     hipLaunchKernelGGL(k_downsample, dim3(num_cu * 4), dim3(256), 0, stream, (const EscapeValue*)din, nr, nc, sc,
                        dout);
     NM_HIP(hipGetLastError());
-    NM_HIP(hipMemcpyAsync(out, dout, nout * sizeof(EscapeValue), hipMemcpyDeviceToHost, stream));
-    NM_HIP(hipStreamSynchronize(stream));
+    NM_HIP(copier.copy(stream, out, dout, nout * sizeof(EscapeValue)));
     return NM_OK;
   }
 };
