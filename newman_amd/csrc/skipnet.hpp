@@ -35,7 +35,6 @@ class SkipNet {
   int predict(const float* raw, size_t n, float* y);
   // mean-squared-error loss and its gradient for normalised inputs, on the GPU
   int gradient(const float* xn, const float* t, size_t n, float* grad, float* loss);
-  void normalise(const float* raw, size_t n, std::vector<float>& out) const;
   void fit_normaliser(const float* raw, size_t n);
   const char* last_error() const { return err_.c_str(); }
 
@@ -49,13 +48,15 @@ class SkipNet {
   struct AdamStep {
     float lr = 0.0f, c1 = 1.0f, c2 = 1.0f;
   };
+  int inputs(const float* raw, size_t n, bool norm);
+  int weights();
   int reserve(size_t nx, size_t nb, size_t ni);
   int batch(const int* idx, int n, float* G, const AdamStep& a, float* loss);
   void release();
   std::string err_;
-  float *dP = nullptr, *dG = nullptr, *dM = nullptr, *dV = nullptr, *dX = nullptr, *dT = nullptr;
+  float *dP = nullptr, *dG = nullptr, *dM = nullptr, *dV = nullptr, *dX = nullptr, *dT = nullptr, *dXB = nullptr;
   float *dH1 = nullptr, *dH2 = nullptr, *dY = nullptr, *dDY = nullptr;
-  float *dD1 = nullptr, *dD2 = nullptr, *dLoss = nullptr;
+  float *dD1 = nullptr, *dD2 = nullptr, *dLoss = nullptr, *dNorm = nullptr;
   int* dIdx = nullptr;
   size_t capX = 0, capB = 0, capI = 0;
 };

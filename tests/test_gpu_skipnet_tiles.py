@@ -1,6 +1,6 @@
-"""The skip network's matrix-unit kernels at the edges of their 16-sample tiles and
-of the 128 samples a gradient round holds: forward pass, loss and every gradient
-against numpy in doubles.
+"""The skip network's kernels at the edges of their workgroups (4 samples) and of the
+samples that a gradient round holds (256): forward pass, loss and every gradient
+against numpy in doubles, and bit for bit against numpy in FP32 with the same order.
 
 Tolerance: each value is a chain of at most three FP32 contractions of at most 132
 terms (hidden layers, deltas) and one over the batch, so it is off by at most
@@ -55,6 +55,40 @@ def test_gradient_tiles(gpu, n):
     assert (np.abs(y - yd) <= u * ya).all()
     assert (np.abs(g - want) <= u * top + 1e-37).all()
     assert abs(loss - np.mean((yd - td) ** 2)) <= u * np.mean((ya + np.abs(td)) ** 2)
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 31, 33, 255, 256, 257, 513])
+def test_sums_keep_their_order(gpu, n):
+    """Every sum one rounded term after the other, over the inputs and over the batch: no tolerance."""
+    rng = np.random.default_rng(100 + n)
+    p = (rng.normal(size=gpu.SKIPNET_PARAMS) * 0.15).astype(np.float32)
+    x = rng.normal(size=(n, gpu.SKIPNET_INPUTS)).astype(np.float32)
+    t = rng.normal(size=n).astype(np.float32)
+    w1, b1, w2, b2, w3, b3 = _split(p)
+
+    def chain(s, terms):
+        for v in terms:
+            s = s + v
+        return s
+
+    h1 = np.maximum(chain(np.tile(b1, (n, 1)), (w1[:, k] * x[:, k:k + 1] for k in range(132))), np.float32(0))
+    h2 = np.maximum(chain(np.tile(b2, (n, 1)), (w2[:, k] * h1[:, k:k + 1] for k in range(64))), np.float32(0))
+    y = chain(np.full(n, b3), (w3[k] * h2[:, k] for k in range(64)))
+    dy = np.float32(2) * (y - t) / np.float32(n)
+    d2 = np.where(h2 > 0, dy[:, None] * w3, np.float32(0))
+    d1 = np.where(h1 > 0, chain(np.zeros_like(d2), (w2[i] * d2[:, i:i + 1] for i in range(64))), np.float32(0))
+
+    def grad(d, h):
+        return chain(np.zeros((d.shape[1], h.shape[1]), np.float32), (d[b][:, None] * h[b] for b in range(n))).ravel()
+
+    one = np.ones((n, 1), np.float32)
+    want = np.concatenate([grad(d1, x), grad(d1, one), grad(d2, h1), grad(d2, one), grad(dy[:, None], h2),
+                           grad(dy[:, None], one)])
+    net = gpu.SkipNet()
+    net.set(p, np.zeros(gpu.SKIPNET_INPUTS, np.float32), np.ones(gpu.SKIPNET_INPUTS, np.float32))
+    assert y.dtype == want.dtype == np.float32
+    assert np.array_equal(net.predict(x), y)
+    assert np.array_equal(net.gradient(x, t)[1], want)
 
 
 @pytest.mark.parametrize("n,batch", [(5, 8), (33, 16), (300, 100)])
