@@ -183,6 +183,70 @@ __host__ __device__ inline double hpd_rest(const hpd<ML>& a) {
   return a.sign < 0 ? -d : d;
 }
 
+// a * b at L limbs
+template <int ML>
+__host__ __device__ inline hpd<ML> hpd_mul(const hpd<ML>& a, const hpd<ML>& b, int L) {
+  hpd<ML> r;
+  r.sign = a.sign * b.sign;
+  uint64_t t[2 * ML];
+#pragma unroll
+  for (int i = 0; i < 2 * ML; i++) t[i] = 0;
+#pragma unroll
+  for (int i = 0; i < ML; i++) {
+    unsigned __int128 c = 0;
+#pragma unroll
+    for (int j = 0; j < ML; j++) {
+      c += (unsigned __int128)a.m[i] * b.m[j] + t[i + j];
+      t[i + j] = (uint64_t)c;
+      c >>= 64;
+    }
+    t[i + ML] = (uint64_t)c;
+  }
+  const int lead = t[2 * ML - 1] >> 63 ? 0 : 1;  // both mantissas are at least 1/2
+#pragma unroll
+  for (int i = 0; i < ML; i++)
+    r.m[i] = r.sign == 0 ? 0 : lead ? (t[ML + i] << 1) | (t[ML + i - 1] >> 63) : t[ML + i];
+  r.exp = r.sign == 0 ? 0 : a.exp + b.exp - lead;
+  hpd_trunc(r, L);
+  return r;
+}
+
+// a double as it is
+template <int ML>
+__host__ __device__ inline hpd<ML> hpd_from_d(double d) {
+  hpd<ML> r;
+  int e = 0;
+  const bool zero = d == 0.0 || !(fabs(d) <= 1.7976931348623157e308);
+  const double f = zero ? 0.0 : frexp(fabs(d), &e);
+  for (int i = 0; i < ML; i++) r.m[i] = 0;
+  r.m[ML - 1] = (uint64_t)ldexp(f, 64);
+  r.exp = zero ? 0 : e;
+  r.sign = zero ? 0 : d < 0.0 ? -1 : 1;
+  return r;
+}
+
+// the nearest double (ties to even), by way of the truncated one
+template <int ML>
+__host__ __device__ inline double hpd_nearest(const hpd<ML>& a, int L) {
+  const double t = hpd_get_d(a);
+  if (a.sign == 0 || !(fabs(t) <= 1.7976931348623157e308)) return t;
+  const hpd<ML> r = hpd_add(a, hpd_from_d<ML>(t), -1, L);
+  if (r.sign == 0) return t;
+  union {
+    double d;
+    uint64_t u;
+  } up, low;
+  low.d = t;
+  if (t == 0.0) up.u = 1ull | (a.sign < 0 ? 1ull << 63 : 0);
+  else up.u = low.u + 1;  // one step away from zero
+  const hpd<ML> half = hpd_from_d<ML>((up.d - t) * 0.5);
+  int c = r.exp > half.exp ? 1 : r.exp < half.exp ? -1 : 0;
+  if (c == 0)
+    for (int i = 0; i < ML; i++)  // the last differing limb decides
+      if (r.m[i] != half.m[i]) c = r.m[i] > half.m[i] ? 1 : -1;
+  return c > 0 ? up.d : c < 0 ? t : (low.u & 1) ? up.d : t;
+}
+
 // the coordinate of offset k: center + k * size at L limbs
 template <int ML>
 __host__ __device__ inline hpd<ML> hpd_pixel(const HpVal& center, const HpVal& size, long k, int L) {

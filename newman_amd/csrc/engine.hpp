@@ -189,6 +189,9 @@ class Engine {
   // Make `ref` the device reference; `serial` identifies it so an unchanged
   // reference is not uploaded again.
   virtual int set_reference(const SaReferenceHost& ref, uint64_t serial) = 0;
+  // A reference's tables from its orbit, on the device (OrbitTables::make); false: the
+  // host's work.
+  virtual bool orbit_tables(const HpVal* x, int len, int L, bool series, SaReferenceHost& r) = 0;
   virtual int render_hw(const std::vector<const HwFrameHost*>& frames, const RenderOpts& opt,
                         EscapeValue* host_out, RenderStats* stats) = 0;
   virtual int render_sa(const std::vector<const SaFrameHost*>& frames, const RenderOpts& opt,

@@ -463,6 +463,50 @@ double nearest(const nm::hpf& a) {
   std::memcpy(&bits, &t, 8);
   return c > 0 || (c == 0 && (bits & 1)) ? up : t;
 }
+// The orbit tables' arithmetic: sums, differences and products of random values at
+// random precisions, and the nearest double, from exponents near 0 to the ends of the
+// doubles' range and far past it.
+template <int ML>
+long long hp_ops_check(unsigned seed, int n) {
+  uint64_t s = seed;
+  long long bad = 0;
+  for (int t = 0; t < n; t++) {
+    const int L = 1 + (int)(next_u64(s) % ML);
+    const int64_t range = t % 4 == 0 ? 3 : t % 4 == 1 ? 64 * ML + 130 : t % 4 == 2 ? 1100 : 40000;
+    auto random_hpf = [&] {
+      nm::hpf v(L);
+      if (next_u64(s) % 16 == 0) return v;  // zero
+      const int kind = (int)(next_u64(s) % 5);
+      for (int i = 0; i < v.L; i++) v.m[i] = kind == 0 ? 0 : kind == 1 ? ~0ull : next_u64(s);
+      if (kind == 3) v.m[v.L - 1] &= ~0ull << 10;  // a double and half of its last bit, or nearly
+      if (kind == 4) v.m[v.L - 1] |= (1ull << 10) - 1;
+      v.m[v.L - 1] |= 1ull << 63;
+      v.sign = next_u64(s) & 1 ? 1 : -1;
+      v.exp = (int64_t)(next_u64(s) % (uint64_t)(2 * range)) - range;
+      return v;
+    };
+    const nm::hpf a = random_hpf();
+    nm::hpf b = random_hpf();
+    if (a.sign && t % 7 == 0) {  // cancellation down to the last limb
+      b = a;
+      b.sign = -a.sign;
+      b.m[0] ^= next_u64(s) % 3;
+    }
+    const auto da = nm::hpd_load<ML>(val_of(a)), db = nm::hpd_load<ML>(val_of(b));
+    auto differ = [&](const nm::hpd<ML>& x, const nm::hpf& y) {
+      const auto z = nm::hpd_load<ML>(val_of(y));
+      return x.sign != z.sign || (z.sign && (x.exp != z.exp || std::memcmp(x.m, z.m, sizeof x.m) != 0));
+    };
+    nm::hpf sum(L), less(L), product(L);
+    nm::hp_add(sum, a, b);
+    nm::hp_sub(less, a, b);
+    nm::hp_mul(product, a, b);
+    const double want = nearest(a), got = nm::hpd_nearest(da, L);
+    bad += differ(nm::hpd_add(da, db, 1, L), sum) || differ(nm::hpd_add(da, db, -1, L), less) ||
+           differ(nm::hpd_mul(da, db, L), product) || std::memcmp(&want, &got, 8) != 0;
+  }
+  return bad;
+}
 template <int ML>
 long long coords_check(unsigned seed, int n) {
   uint64_t s = seed;
@@ -505,6 +549,15 @@ long long coords_check(unsigned seed, int n) {
 }
 }  // namespace
 extern "C" {
+long long nm_hp_ops_check(int limbs, unsigned seed, int n) {
+  switch (limbs) {
+    case 4: return hp_ops_check<4>(seed, n);
+    case 6: return hp_ops_check<6>(seed, n);
+    case 8: return hp_ops_check<8>(seed, n);
+    case 16: return hp_ops_check<16>(seed, n);
+    default: return -1;
+  }
+}
 long long nm_coords_check(int limbs, unsigned seed, int n) {
   switch (limbs) {
     case 4: return coords_check<4>(seed, n);

@@ -57,6 +57,7 @@
 #include "coords.hpp"
 #include "engine.hpp"
 #include "hostcopy.hpp"
+#include "orbit.hpp"
 #include "sample_index.hpp"
 #include "video.hpp"
 
@@ -2308,6 +2309,7 @@ class EngineImpl : public Engine {
  public:
   hipStream_t stream = nullptr;
   std::vector<hipEvent_t> evpool;  // stage boundaries of timed passes (grow-only)
+  OrbitTables orbit;
   HostCopy copier;
   HostTotals* h_totals = nullptr;          // the last render's counters (pinned)
   int device = 0;
@@ -2391,6 +2393,9 @@ class EngineImpl : public Engine {
     return NM_OK;
   }
 
+  bool orbit_tables(const HpVal* x, int len, int L, bool series, SaReferenceHost& r) override {
+    return orbit.make(stream, x, len, L, series, r);
+  }
   int set_reference(const SaReferenceHost& ref, uint64_t serial) override {
     if (serial == ref_serial && serial != 0) return NM_OK;
     const int len = ref.len;

@@ -289,6 +289,7 @@ void Mandelbrot::findProbe() {
 // reads are kept.
 void Mandelbrot::computeSeries() {
   const int len = ref_.len;
+  if (orbitTables(len, true, ref_)) return;
   const int L = hp_limbs_for_bits(hp_default_bits());
   ref_.A.assign(2 * (size_t)len, 0.0);
   ref_.B.assign(2 * (size_t)len, 0.0);
@@ -338,6 +339,19 @@ void Mandelbrot::computeSeries() {
       (*fe[k / 2])[2 * i + k % 2] = m == 0.0 ? kFxZeroExp : (int32_t)e;
     }
   }
+}
+
+// the device's work on X: r's orbit in doubles, and with `series` its coefficients
+bool Mandelbrot::orbitTables(int len, bool series, SaReferenceHost& r) {
+  static_assert(sizeof(HPComplex) == 2 * sizeof(HpVal), "X is pairs of HpVal");
+  Engine* eng = nullptr;
+  r.len = len;
+  if (Engine::instance(&eng) == NM_OK && X.size() == (size_t)len + 1 &&
+      eng->orbit_tables((const HpVal*)X.data(), len, hp_limbs_for_bits(hp_default_bits()), series, r))
+    return true;
+  r = SaReferenceHost();
+  r.len = len;
+  return false;
 }
 
 // log2 |z|^2 without overflow (long double has a 15-bit exponent)
@@ -525,8 +539,7 @@ int Mandelbrot::findProbeGPU(Engine* eng) {
   const int lenc = computeOrbit(c0, true);
   X.resize((size_t)lenc + 1);
   SaReferenceHost tmp;
-  tmp.len = lenc;
-  fillOrbit(tmp);
+  if (!orbitTables(lenc, false, tmp)) fillOrbit(tmp);
   tmp.A.assign(2 * (size_t)lenc, 0.0);
   tmp.B = tmp.A;
   tmp.C = tmp.A;
@@ -669,7 +682,7 @@ void Mandelbrot::fillOrbit(SaReferenceHost& r) const {
 }
 
 int Mandelbrot::uploadReference() {
-  fillOrbit(ref_);
+  if (ref_.Zd.empty()) fillOrbit(ref_);
   buildThresholds();
   have_ref_ = true;
   rendered_ = false;

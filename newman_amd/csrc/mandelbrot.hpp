@@ -200,6 +200,7 @@ class Mandelbrot {
 
   void findProbe();
   int findProbeGPU(Engine* eng);
+  bool orbitTables(int len, bool series, SaReferenceHost& r);
   void fillOrbit(SaReferenceHost& r) const;
   int computeOrbit(const HPComplex& X0, bool store);
   void computeSeries();

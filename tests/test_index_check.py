@@ -86,3 +86,12 @@ def test_device_coordinates_equal_the_hosts(limbs):
     L.nm_coords_check.restype = C.c_longlong
     L.nm_coords_check.argtypes = [C.c_int, C.c_uint, C.c_int]
     assert all(L.nm_coords_check(limbs, seed, 4000) == 0 for seed in range(1, 9))
+
+
+@pytest.mark.parametrize("limbs", [4, 6, 8, 16])
+def test_device_arithmetic_equals_the_hosts(limbs):
+    """The orbit tables' sums, products and roundings give hpfloat.cpp's bits."""
+    L = _lib()
+    L.nm_hp_ops_check.restype = C.c_longlong
+    L.nm_hp_ops_check.argtypes = [C.c_int, C.c_uint, C.c_int]
+    assert all(L.nm_hp_ops_check(limbs, seed, 20000) == 0 for seed in range(1, 5))
