@@ -423,6 +423,9 @@ __device__ __forceinline__ void park(double& x, double& y, double& r2, double& i
 // reference's sqMag of each bit for bit (their r2 and i2 stay in registers):
 // three adds and three compare-and-branches less per four updates.  A lane that
 // escaped inside the group runs the group's remaining updates unrecorded.
+// A longer group may overflow past the escape: r2 or i2 is infinite then, x' = r2 -
+// i2 + cx infinite or NaN, and from there on every |z|^2 is infinite or NaN; so
+// !(|z|^2 <= R^2) on its last update still tells the lanes that escaped in it.
 inline bool grouped_test_ok(double radius, double c_bound) {
   return radius >= 2.0 && radius <= 0x1p30 && c_bound <= 0.999 * (radius * radius - radius);
 }
@@ -487,7 +490,7 @@ constexpr int kPlainWaves = 4;
 // Group sizes of the grouped escape test: the start kernel's pre-iteration,
 // where most lanes escape within a few updates, and the iteration kernel.
 constexpr int kStartGroup = 4;
-constexpr int kIterGroup = 4;
+constexpr int kIterGroup = 16;
 
 // The frame record at a wave-uniform index, through the constant address space
 // (the records are written before the launch and only read by it), so the
@@ -971,58 +974,56 @@ struct ChunkMap {
   }
 };
 
-// An escape of the plain iterate kernel as its wave's queue holds it: |z|^2 after
-// each update of the group it fell in (r2 + i2 as the reference's sqMag,
-// mandelbrot.cpp:245), the last one past the bailout; k: the updates done before the
-// group.
-template <int G>
+// An escape of the plain iterate kernel as its wave's queue holds it: the value before
+// the group of updates it fell in, and the updates done before (k).
 struct PlainEscape {
-  double m[G];
+  double x, y, cx, cy;
   uint32_t pix;
   int32_t k;
 };
-template <int G>
-using EscapeQueue = __attribute__((address_space(3))) PlainEscape<G>*;
+typedef __attribute__((address_space(3))) PlainEscape* EscapeQueue;
 constexpr int kEscapeCap = 128;  // per wave: up to 63 waiting, one per lane more in a block
 
 // A wave's state inside a block of the plain iterate kernel; `live`: the scalar mask
 // of lanes still iterating.  A lane that is not keeps updating unrecorded (its
 // values overflow to inf or NaN), so an escape costs no parking.
-template <int G>
 struct PlainWave {
   double &x, &y, &r2, &i2;
   const double cx, cy;
   const uint32_t pix;
   const int k;
   unsigned long long& live;
-  EscapeQueue<G> q;
+  EscapeQueue q;
   int& qn;  // wave-uniform: entries waiting
 };
 
 // Updates J .. K - 1 of a block in groups of G (unrolled by recursion).  A group
-// tests its last update's |z|^2 (one update if G = 1); a lane that escaped in it
-// puts the group's |z|^2 into the queue, where 64 at a time are looked through for
-// the first escaping update and smoothed (escapes_out).  Doing that here, for the
-// one or two lanes that escape, and parking them, cost 30 instructions at every
-// second group of the 7680x4320 plain view: 11.1 a update against 6.5 without.
+// tests its last update's |z|^2 (G = 1: every update's, as the reference does); a
+// lane that escaped in it puts the value before the group into the queue, and 64 at
+// a time run the group again for their first escaping update (escapes_out).  On the
+// 7680x4320 plain view some lane escapes in every second group of four: looking for
+// the update there and parking the lane took 3.28 ms (the iterate kernel), queueing
+// the group's four |z|^2 3.12, the value before the group 2.98 with groups of 8 or
+// 16, 3.04 of 32, 3.21 of 64; on 7680x4320 of the whole set groups of 16 are ahead of
+// 8 (346 us against 359).  6.5 instructions an update are the updates and a test in
+// four, 6.1 with a test in 16.
 template <int J, int K, int G, bool FMA2>
-__device__ __forceinline__ void plain_block(PlainWave<G>& L, const double b2) {
+__device__ __forceinline__ void plain_block(PlainWave& L, const double b2) {
   static_assert(K % G == 0, "a block holds whole groups");
   if constexpr (J < K) {
-    double m2[G], n2[G];
+    const double x0 = L.x, y0 = L.y;
 #pragma unroll
-    for (int t = 0; t < G; t++) {
-      plain_update<FMA2>(L.x, L.y, L.r2, L.i2, L.cx, L.cy);
-      m2[t] = L.r2;
-      n2[t] = L.i2;
-    }
-    const unsigned long long e = __ballot(m2[G - 1] + n2[G - 1] > b2) & L.live;
+    for (int t = 0; t < G; t++) plain_update<FMA2>(L.x, L.y, L.r2, L.i2, L.cx, L.cy);
+    const double m = L.r2 + L.i2;
+    const unsigned long long e = __ballot(G == 1 ? m > b2 : !(m <= b2)) & L.live;
     if (__builtin_expect(e != 0, 0)) {
       L.live &= ~e;
       if (__builtin_amdgcn_inverse_ballot_w64(e)) {
-        const EscapeQueue<G> p = L.q + __builtin_amdgcn_mbcnt_hi((uint32_t)(e >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)e, L.qn));
-#pragma unroll
-        for (int t = 0; t < G; t++) p->m[t] = m2[t] + n2[t];
+        const EscapeQueue p = L.q + __builtin_amdgcn_mbcnt_hi((uint32_t)(e >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)e, L.qn));
+        p->x = x0;
+        p->y = y0;
+        p->cx = L.cx;
+        p->cy = L.cy;
         p->pix = L.pix;
         p->k = L.k + J;
       }
@@ -1032,23 +1033,24 @@ __device__ __forceinline__ void plain_block(PlainWave<G>& L, const double b2) {
   }
 }
 
-// The last n (at most 64) of the wave's waiting escapes: counts and smooth values.
-template <int G>
-__device__ __forceinline__ void escapes_out(const PlainArgs& a, EscapeQueue<G> q, int& qn, int n,
+// The last n (at most 64) of the wave's waiting escapes: their groups' updates up to
+// the first that escapes, counts and smooth values.
+template <int G, bool FMA2>
+__device__ __forceinline__ void escapes_out(const PlainArgs& a, EscapeQueue q, int& qn, int n,
                                             unsigned long long& executed, unsigned long long& credited) {
   const Common& c = a.c;
   __builtin_amdgcn_wave_barrier();
   qn -= n;
   if (lane_id() < n) {
-    const EscapeQueue<G> e = q + (qn + lane_id());
-    int j = G - 1;
-    double mg = e->m[G - 1];
-#pragma unroll
-    for (int t = G - 2; t >= 0; t--)
-      if (e->m[t] > c.b2) {
-        j = t;
-        mg = e->m[t];
-      }
+    const EscapeQueue e = q + (qn + lane_id());
+    double x = e->x, y = e->y, r2 = x * x, i2 = y * y, mg;
+    const double cx = e->cx, cy = e->cy;
+    int j = 0;
+    for (;; j++) {
+      plain_update<FMA2>(x, y, r2, i2, cx, cy);
+      mg = r2 + i2;
+      if (mg > c.b2 || j == G - 1) break;
+    }
     // the reference tests k >= N before each update: an escape counts only below N
     const int it = min(e->k + j, c.N);
     c.out[e->pix] = EscapeValue{it, it < c.N ? smooth_of(mg, c) : 0.0f};
@@ -1067,9 +1069,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 8))
   cm.init(total);
   ChunkClaim q;
   q.init(c.part, cm.nch);
-  constexpr int G = GROUPED ? kIterGroup : 1;
-  __shared__ PlainEscape<G> escapes[kThreads / 64][kEscapeCap];
-  const EscapeQueue<G> eq = (EscapeQueue<G>)escapes[threadIdx.x >> 6];
+  constexpr int G = GROUPED ? (K < kIterGroup ? K : kIterGroup) : 1;
+  __shared__ PlainEscape escapes[kThreads / 64][kEscapeCap];
+  const EscapeQueue eq = (EscapeQueue)escapes[threadIdx.x >> 6];
   int en = 0;
   unsigned long long credited = 0;
   const uint32_t c0 = q.first(), c1 = q.next(), c2 = q.next();
@@ -1123,7 +1125,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 8))
     }
     unsigned long long live = __ballot(act);  // wave-uniform: the lanes iterating a sample
     if (live == 0) break;
-    PlainWave<G> L{x, y, r2, i2, cx, cy, pix, k, live, eq, en};
+    PlainWave L{x, y, r2, i2, cx, cy, pix, k, live, eq, en};
     plain_block<0, K, G, FMA2>(L, c.b2);
     k += K;
     const bool on = (live >> lane_id()) & 1ull;
@@ -1133,9 +1135,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 8))
       executed += (unsigned long long)(N - a.k_start);
     }
     act = on && k < N;
-    if (en >= 64) escapes_out<G>(a, eq, en, 64, executed, credited);
+    if (en >= 64) escapes_out<G, FMA2>(a, eq, en, 64, executed, credited);
   }
-  escapes_out<G>(a, eq, en, en, executed, credited);
+  escapes_out<G, FMA2>(a, eq, en, en, executed, credited);
   const unsigned long long v[2] = {executed, credited};
   const int idx[2] = {C_EXECUTED, C_CREDITED};
   block_partial(c.part, kSlotIter + blockIdx.x, v, idx, 2);

@@ -51,3 +51,19 @@ def test_scatter_around_the_scan(gpu, nr, nc):
     want = o.render_rows(rows)
     _check(m.grid()[rows], want)
     assert st["n_iterated"] + st["n_cardioid"] + st["n_sa_resolved"] == nr * nc
+
+
+@pytest.mark.parametrize("k", [8, 16, 32, 64])
+@pytest.mark.parametrize("bailout", [1.5, 3.0, 1024.0, 2.0 ** 30, 2.0 ** 31])
+def test_groups_that_overflow(gpu, k, bailout):
+    """A group of up to 16 updates tests its last one: past an escape the values
+    square themselves to infinity and NaN within it, and a limit may fall inside it.
+    Counts are those of a test after every update (which radii below 2 and above 2^30
+    have here, too)."""
+    for N in (77, 130, 901):
+        m, o = gpu.Mandelbrot(30, 47), O.OView(30, 47)
+        for v in (m, o):
+            v.set_view(N, "-0.7453", "0.1127", "0.3")
+            v.set_bailout(bailout)
+        m.render(block_k=k)
+        assert np.array_equal(m.grid()["iterations"], o.render_rows(np.arange(30, dtype=np.int32))["iterations"])
