@@ -1584,8 +1584,8 @@ __device__ __forceinline__ void coherent_phase(const SeriesArgs& a, const bool w
         const unsigned long long out = __ballot(r2 > c.b2) & live, reb = __ballot(r2 < dmag) & live & ~out;
         if (__builtin_expect((out | reb) != 0, 0)) {
           live &= ~(out | reb);
-          if (((out | reb) >> lane_id()) & 1ull) {
-            const bool r = (reb >> lane_id()) & 1ull;
+          if (__builtin_amdgcn_inverse_ballot_w64(out | reb)) {
+            const bool r = __builtin_amdgcn_inverse_ballot_w64(reb);
             dr = r ? fma(yr, yr, fma(-yi, yi, e.x)) : xr;
             di = r ? fma(yr, yi, fma(yi, yr, e.y)) : xi;
             m = r ? 1 : mu + j;
@@ -1617,6 +1617,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(6, 8))
   const Common& c = a.c;
   unsigned long long ncard = 0, nres = 0, skipped = 0, credited = 0, executed = 0, rebased = 0;
   clear_claims(c.part);
+  const double near_b2 = c.b2 >= 1.0 ? c.b2 * (1.0 - 0x1p-10) : 0.0;
   const uint32_t ntiles = start_tiles(c.total);
   for (uint32_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
     uint32_t mine = 0;
@@ -1681,8 +1682,19 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(6, 8))
           int found = dsize - 1;
           double2 d = term(found);
           double2 zf = a.Zd[found + 1], xl = a.Xlo[found];
-          double yr = trunc_sum3(zf.x, xl.x, d.x), yi = trunc_sum3(zf.y, xl.y, d.y);
-          if (yr * yr + yi * yi > c.b2) {
+          // escaped inside the skip?  Y = X + d, with |d| < 2^20 and a rounded |Y| a
+          // little below the bailout R >= 1, is off by less than 2^-28 R (X is within
+          // 2^-53 of Z): the reference's truncated sums (45 instructions) decide only
+          // nearer than that
+          const double qr = zf.x + d.x, qi = zf.y + d.y;
+          bool inside = false;
+          double yr, yi;
+          if (FXS || !(qr * qr + qi * qi < near_b2 && fmax(fabs(d.x), fabs(d.y)) < 0x1p20)) {
+            yr = trunc_sum3(zf.x, xl.x, d.x);
+            yi = trunc_sum3(zf.y, xl.y, d.y);
+            inside = yr * yr + yi * yi > c.b2;
+          }
+          if (inside) {
             // escape inside the skip: the reference's binary search (mandelbrot.cpp:186-206)
             int low = 0, high = dsize - 1, mid = dsize / 2;
             while (low <= high) {
@@ -1840,7 +1852,7 @@ __device__ __forceinline__ int pert_block(double& dr, double& di, const double e
     const unsigned long long first = __ballot(r2 > b2) & ~seen;
     if (__builtin_expect(first != 0, 0)) {
       seen |= first;
-      if ((first >> lane_id()) & 1ull) {
+      if (__builtin_amdgcn_inverse_ballot_w64(first)) {
         escj = j;
         esc_r2 = r2;
       }
