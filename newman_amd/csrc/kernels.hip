@@ -82,11 +82,14 @@ constexpr int kHead = 64;               // orbit padding past its end (>= max K)
 // lanes live) and the tail (where samples that have not rebased yet run out the
 // reference); lanes whose block fits a window read it from LDS, the others
 // gather from global memory, whose cache tag lookups bound the gathers
-constexpr int kLdsTail = 1024, kLdsHead = 3040;
-// The series iterate kernel runs 8 waves per workgroup: the 32 KB of LDS orbit
-// windows is shared by 8 waves, so LDS does not cap the waves a CU holds below
-// what the registers allow (8 per SIMD at 64 VGPRs: four workgroups, 128 KB).
-constexpr int kSeriesIterThreads = 512;
+constexpr int kLdsTail = 512, kLdsHead = 7648;
+// The series iterate kernel runs up to 16 waves per workgroup, all that a CU holds by
+// default (4 per SIMD), over one copy of the windows that fills its LDS: on the 1e-100
+// view 4.78 ms against 5.00 of two workgroups with 1024 + 3040 entries each (4.84 with
+// a tail of 1024, 4.83 of 2048), the 1e-30, 1e-40 and 1e-200 views the same.  More
+// waves over smaller windows: 6 per SIMD 1.88 against 2.00 ms at 1e-30, but 5.98 ms
+// at 1e-100.
+constexpr int kSeriesIterThreads = 1024;
 static_assert(kLdsTail >= 64 && kLdsHead >= 64, "a block of up to 64 steps reads inside one window");
 constexpr int kPartSlots = 6144;        // per-workgroup partial counter slots
 
@@ -1955,9 +1958,8 @@ __device__ __forceinline__ void pert_block_fx(float& wr, float& wi, int& ex, flo
 // their objects in scratch and spilled the LDS head pointer, reloaded in the
 // step loop's rebase branch): no scratch at all.
 // A workgroup's LDS: the waves' retire queues and the orbit windows (tail[t] =
-// Zd[tail_lo + t], head[h] = Zd[h]).  Half a CU's 160 KB, for the two workgroups a
-// CU holds by default (4 waves per SIMD); of static size, so that a rebase's base
-// address is a literal (from a register it was one of 64 spilled ones, +18% time on
+// Zd[tail_lo + t], head[h] = Zd[h]): a CU's 160 KB; of static size, so that a rebase's
+// base address is a literal (from a register it was one of 64 spilled ones, +18% time on
 // the 1e-30 view).  The head sits above 16 K positions so that a rebased lane's
 // base address (head - 16 j) stays non-negative.
 struct SeriesLds {
@@ -1965,7 +1967,7 @@ struct SeriesLds {
   double2 tail[kLdsTail];
   double2 head[kLdsHead];
 };
-static_assert(2 * (sizeof(SeriesLds) + 256) <= 160 * 1024, "two workgroups per CU");
+static_assert(sizeof(SeriesLds) + 256 <= 160 * 1024, "one workgroup per CU");
 template <int K, bool FX>
 __global__ __launch_bounds__(kSeriesIterThreads) __attribute__((amdgpu_waves_per_eu(4, 8)))
 void k_series_iterate(SeriesArgs a) {
@@ -2239,10 +2241,12 @@ __global__ void k_clear(double* p, int n) {
   } while (0)
 
 // threads per workgroup of a path's iterate kernel
+// threads of an iterate workgroup; the series kernel's, one per CU, takes all of the
+// CU's waves
 template <class A>
-constexpr int iter_threads() { return kThreads; }
+int iter_threads(int) { return kThreads; }
 template <>
-constexpr int iter_threads<SeriesArgs>() { return kSeriesIterThreads; }
+int iter_threads<SeriesArgs>(int waves) { return std::min(kSeriesIterThreads, 256 * std::max(1, waves)); }
 
 // workgroups of an iterate launch of `ti` threads: `waves` per SIMD
 static int iterate_grid(int num_cu, int waves, int ti) {
@@ -2272,7 +2276,7 @@ static hipError_t launch_pass_on(hipStream_t stream, int num_cu, unsigned long l
   const Common& c = args.c;
   const int gtile = tile_grid(c.total, num_cu);
   // waves = persistent waves per SIMD: 4 per CU for each 256 threads
-  const int ti = iter_threads<Args>();
+  const int ti = iter_threads<Args>(waves);
   const int giter = iterate_grid(num_cu, waves, ti);
   hipError_t e;
 #define NM_LAUNCH_OK(expr)                   \
@@ -2624,7 +2628,7 @@ class EngineImpl : public Engine {
     hipError_t ce = hipSuccess;
     if (st == NM_OK) {
       hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(kReduceThreads), 0, stream, (const unsigned long long*)d_part,
-                         tile_grid(args.c.total, num_cu), iterate_grid(num_cu, waves, iter_threads<Args>()),
+                         tile_grid(args.c.total, num_cu), iterate_grid(num_cu, waves, iter_threads<Args>(waves)),
                          (const uint32_t*)d_nactive, h_totals);
       ce = hipGetLastError();
       if (ce == hipSuccess && host_out)
@@ -2886,8 +2890,8 @@ class EngineImpl : public Engine {
     // counts: 64 (5.27 -> 4.97 ms at 1e-100).  FP32X blocks renormalise their
     // mantissa at block ends, so they stay short
     const int K = opt.block_k > 0 ? opt.block_k : fx ? 8 : a.fxs ? 64 : 32;
-    // 4 persistent waves per SIMD: the two workgroups whose queues and windows fill
-    // a CU's LDS (more would wait for these to end; fewer hide too little latency:
+    // 4 persistent waves per SIMD: the workgroup whose queues and windows fill a CU's
+    // LDS (more would wait for it to end; fewer hide too little latency:
     // 2 waves 2.8-3.0 against 2.0 ms on the 1e-30 view, 1.29 against 0.91 ms on 16
     // frames of the 1e-40 video).  FP32X ran 8 with smaller windows: 1.18 -> 1.07 ms
     // on the 1279x719 frame of the 1e-200 view
