@@ -166,6 +166,7 @@ struct SeriesArgs {
   const int2 *Ae, *Be, *Ce;
   int fxs;
   uint32_t run_shift;  // active-list chunks (ChunkMap): runs of 2^run_shift entries
+  int fx_runs;         // FP32X: blocks between refills (together at most 64 steps)
   double* safe;        // safe radius per orbit index (safe_radius); null: no coherent phase (FP32X deltas)
   double emax, radius;  // what the radii hold for: |e| of every sample, the bailout
 };
@@ -1893,60 +1894,81 @@ __device__ __forceinline__ void fx_normalise(double yr, double yi, double er, do
   esi = (float)ldexp(ei, -ex);
 }
 
+// `runs` blocks of K steps, the mantissas renormalised after each (kept near 1: |w|
+// grows by at most |W| per step; results depend on K, not on the runs between refills).
 template <int K, bool END, class P>
 __device__ __forceinline__ void pert_block_fx(float& wr, float& wi, int& ex, float& esr, float& esi, const double er,
-                                              const double ei, int& m, const int it, P zp, const P head,
-                                              const int endj, const int mend, const double b2, const float b2g,
+                                              const double ei, int& m, int it, P zp, const P head, const int mend,
+                                              const int N, const int runs, const double b2, const float b2g,
                                               int& esc, double& esc_r2, unsigned int& rb) {
   const float qnanf = __int_as_float(0x7fc00000);
-  bool moved = false;
   ld_double2 z = zp[0];
+#pragma unroll 1
+  for (int r = 0; r < runs; r++) {
+    bool moved = false;
+    const int endj = mend - m;
 #pragma unroll
-  for (int j = 0; j < K; j++) {
-    const double zrd = z.x;
-    const double zid = z.y;
-    const float zr = (float)zrd, zi = (float)zid;
-    const float dr = ldexpf(wr, ex), di = ldexpf(wi, ex);
-    const float yr = zr + dr, yi = zi + di;
-    const float r2 = fmaf(yr, yr, yi * yi);
-    // near the bailout: the reference's test in FP64 (only on wave-steps where
-    // some lane comes near it)
-    if (__builtin_expect(__ballot(r2 > b2g) != 0, 0)) {
-      if (r2 > b2g) {
-        const double ydr = zrd + ldexp((double)wr, ex), ydi = zid + ldexp((double)wi, ex);
-        const double r2d = ydr * ydr + ydi * ydi;
-        if (r2d > b2) {  // first escape: NaN in wr reaches every later step
-          esc = it + j;
-          esc_r2 = r2d;
-          wr = qnanf;
+    for (int j = 0; j < K; j++) {
+      const double zrd = z.x;
+      const double zid = z.y;
+      const float zr = (float)zrd, zi = (float)zid;
+      const float dr = ldexpf(wr, ex), di = ldexpf(wi, ex);
+      const float yr = zr + dr, yi = zi + di;
+      const float r2 = fmaf(yr, yr, yi * yi);
+      // near the bailout: the reference's test in FP64 (only on wave-steps where
+      // some lane comes near it)
+      if (__builtin_expect(__ballot(r2 > b2g) != 0, 0)) {
+        if (r2 > b2g) {
+          const double ydr = zrd + ldexp((double)wr, ex), ydi = zid + ldexp((double)wi, ex);
+          const double r2d = ydr * ydr + ydi * ydi;
+          if (r2d > b2) {  // first escape: NaN in wr reaches every later step
+            esc = it + j;
+            esc_r2 = r2d;
+            wr = qnanf;
+          }
         }
       }
+      // the rebase test |Y|^2 < |d|^2 in the mantissa's scale: |Z 2^-ex + w|^2 <
+      // |w|^2 (d = w 2^ex underflows FP32 long before the deltas this form is for;
+      // Z 2^-ex is formed in FP64, then rounded; an overflow to inf means |Y| >> |d|)
+      const float ysr = (float)ldexp(zrd, -ex) + wr, ysi = (float)ldexp(zid, -ex) + wi;
+      bool reb = fmaf(ysr, ysr, ysi * ysi) < fmaf(wr, wr, wi * wi);
+      if (END) reb = reb || (moved ? orbit_index(zp, head) + j == mend : j == endj);
+      float Wr = zr + yr, Wi = zi + yi;
+      if (__builtin_expect(__ballot(reb) != 0, 0)) {
+        if (reb) {  // rebase in FP64: d = Y against Zd[0] = 0, so W = Y
+          const double ydr = zrd + ldexp((double)wr, ex), ydi = zid + ldexp((double)wi, ex);
+          fx_normalise(ydr, ydi, er, ei, wr, wi, ex, esr, esi);
+          Wr = (float)ydr;
+          Wi = (float)ydi;
+          zp = orbit_back(head, j);
+          moved = true;
+        }
+      }
+      if (j + 1 < K) z = zp[j + 1];
+      else if (r + 1 < runs) z = zp[K];
+      const float nwr = fmaf(wr, Wr, fmaf(-wi, Wi, esr));
+      const float nwi = fmaf(wr, Wi, fmaf(wi, Wr, esi));
+      wr = nwr;
+      wi = nwi;
     }
-    // the rebase test |Y|^2 < |d|^2 in the mantissa's scale: |Z 2^-ex + w|^2 <
-    // |w|^2 (d = w 2^ex underflows FP32 long before the deltas this form is for;
-    // Z 2^-ex is formed in FP64, then rounded; an overflow to inf means |Y| >> |d|)
-    const float ysr = (float)ldexp(zrd, -ex) + wr, ysi = (float)ldexp(zid, -ex) + wi;
-    bool reb = fmaf(ysr, ysr, ysi * ysi) < fmaf(wr, wr, wi * wi);
-    if (END) reb = reb || (moved ? orbit_index(zp, head) + j == mend : j == endj);
-    float Wr = zr + yr, Wi = zi + yi;
-    if (__builtin_expect(__ballot(reb) != 0, 0)) {
-      if (reb) {  // rebase in FP64: d = Y against Zd[0] = 0, so W = Y
-        const double ydr = zrd + ldexp((double)wr, ex), ydi = zid + ldexp((double)wi, ex);
-        fx_normalise(ydr, ydi, er, ei, wr, wi, ex, esr, esi);
-        Wr = (float)ydr;
-        Wi = (float)ydi;
-        zp = orbit_back(head, j);
-        moved = true;
+    m = moved ? orbit_index(zp, head) + K : m + K;
+    // blocks of a lane that escaped in an earlier one or reached N do not count
+    rb += moved && (uint32_t)esc >= (uint32_t)it && it < N ? 1u : 0u;
+    zp = zp + K;
+    it += K;
+    const float mx = fmaxf(fabsf(wr), fabsf(wi));
+    if (mx > 0.0f && mx < INFINITY) {
+      const int k = ilogbf(mx);
+      if (k > 8 || k < -8) {
+        wr = ldexpf(wr, -k);
+        wi = ldexpf(wi, -k);
+        ex += k;
+        esr = (float)ldexp(er, -ex);
+        esi = (float)ldexp(ei, -ex);
       }
     }
-    if (j + 1 < K) z = zp[j + 1];
-    const float nwr = fmaf(wr, Wr, fmaf(-wi, Wi, esr));
-    const float nwi = fmaf(wr, Wi, fmaf(wi, Wr, esi));
-    wr = nwr;
-    wi = nwi;
   }
-  m = moved ? orbit_index(zp, head) + K : m + K;
-  rb += moved ? 1u : 0u;
 }
 
 // FP64 (FX = false) or FP32X (FX = true) perturbation with rebasing (replaces the
@@ -1971,6 +1993,7 @@ static_assert(sizeof(SeriesLds) + 256 <= 160 * 1024, "one workgroup per CU");
 template <int K, bool FX>
 __global__ __launch_bounds__(kSeriesIterThreads) __attribute__((amdgpu_waves_per_eu(4, 8)))
 void k_series_iterate(SeriesArgs a) {
+  const int runs = FX ? a.fx_runs : 1, KB = K * runs;  // the steps between refills
   const Common& c = a.c;
   const uint32_t total = *c.nactive;
   uint32_t executed = 0, rebased = 0;  // per lane (< 2^32 steps per lane per launch)
@@ -1989,7 +2012,7 @@ void k_series_iterate(SeriesArgs a) {
   double2* const zlds = lds.tail;
   int rn = 0;
   unsigned long long credited = 0;
-  const int tail_lo = max(kLdsHead, min(a.zd_count, a.len + 2 + K) - kLdsTail);
+  const int tail_lo = max(kLdsHead, min(a.zd_count, a.len + 2 + KB) - kLdsTail);
   const int tail_hi = tail_lo + kLdsTail;
   for (int i = threadIdx.x; i < kLdsTail + kLdsHead; i += blockDim.x) {
     const int src = i < kLdsTail ? tail_lo + i : i - kLdsTail;
@@ -2067,13 +2090,13 @@ void k_series_iterate(SeriesArgs a) {
       it = 0;
     }
     // lanes whose block crosses the reference's end rebase there (END variant)
-    const bool end_zone = __ballot(act && m + K > mend) != 0 || mend <= K;
-    const bool in_head = m + K <= kLdsHead;
-    const bool in_tail = !in_head && m >= tail_lo && m + K <= tail_hi;
+    const bool end_zone = __ballot(act && m + KB > mend) != 0 || mend <= KB;
+    const bool in_head = m + KB <= kLdsHead;
+    const bool in_tail = !in_head && m >= tail_lo && m + KB <= tail_hi;
     int esc = -1;
     double esc_r2 = 0.0;
     unsigned int rb = 0;
-    int kdone = K;
+    int kdone = KB;
     const int it0 = it;
     const bool can_refill = pos < ncur || nnext > 0;  // wave-uniform
     if (FX) {
@@ -2082,34 +2105,22 @@ void k_series_iterate(SeriesArgs a) {
         const lds_orbit lhead = (lds_orbit)(const void*)zhead;
         const lds_orbit zp = in_head ? lhead + m : (lds_orbit)(const void*)zlds + (m - tail_lo);
         if (end_zone)
-          pert_block_fx<K, true>(wr, wi, ex, esr, esi, er, ei, m, it, zp, lhead, mend - m, mend, c.b2, b2g, esc,
+          pert_block_fx<K, true>(wr, wi, ex, esr, esi, er, ei, m, it, zp, lhead, mend, N, runs, c.b2, b2g, esc,
                                  esc_r2, rb);
         else
-          pert_block_fx<K, false>(wr, wi, ex, esr, esi, er, ei, m, it, zp, lhead, 0, mend, c.b2, b2g, esc, esc_r2,
-                                  rb);
+          pert_block_fx<K, false>(wr, wi, ex, esr, esi, er, ei, m, it, zp, lhead, mend, N, runs, c.b2, b2g, esc,
+                                  esc_r2, rb);
       } else {
         const gen_orbit fhead = (gen_orbit)(const void*)zhead;
         const gen_orbit fz = in_head ? fhead + m
                                      : in_tail ? (gen_orbit)(const void*)zlds + (m - tail_lo)
                                                : (gen_orbit)(const void*)a.Zd + m;
         if (end_zone)
-          pert_block_fx<K, true>(wr, wi, ex, esr, esi, er, ei, m, it, fz, fhead, mend - m, mend, c.b2, b2g, esc,
+          pert_block_fx<K, true>(wr, wi, ex, esr, esi, er, ei, m, it, fz, fhead, mend, N, runs, c.b2, b2g, esc,
                                  esc_r2, rb);
         else
-          pert_block_fx<K, false>(wr, wi, ex, esr, esi, er, ei, m, it, fz, fhead, 0, mend, c.b2, b2g, esc, esc_r2,
-                                  rb);
-      }
-      // keep the mantissa near 1: |w| grows by at most |W| per step
-      const float mx = fmaxf(fabsf(wr), fabsf(wi));
-      if (mx > 0.0f && mx < INFINITY) {
-        const int k = ilogbf(mx);
-        if (k > 8 || k < -8) {
-          wr = ldexpf(wr, -k);
-          wi = ldexpf(wi, -k);
-          ex += k;
-          esr = (float)ldexp(er, -ex);
-          esi = (float)ldexp(ei, -ex);
-        }
+          pert_block_fx<K, false>(wr, wi, ex, esr, esi, er, ei, m, it, fz, fhead, mend, N, runs, c.b2, b2g, esc,
+                                  esc_r2, rb);
       }
     } else if (__ballot(act && !in_head && !in_tail) == 0) {
       // every lane's block lies in an LDS window: the whole block reads LDS
@@ -2890,6 +2901,11 @@ class EngineImpl : public Engine {
     // counts: 64 (5.27 -> 4.97 ms at 1e-100).  FP32X blocks renormalise their
     // mantissa at block ends, so they stay short
     const int K = opt.block_k > 0 ? opt.block_k : fx ? 8 : a.fxs ? 64 : 32;
+    // FP32X takes several of its short blocks between refills, as the refill and its
+    // bookkeeping are 240 instructions: one / 32 steps / 64 steps of them 1.09 / 0.93 /
+    // 0.89 ms on the 1279x719 frame of the 1e-200 view, 0.47 / 0.43 / 0.44 ms on
+    // 1600x900 of the 1e-30 view, 0.112 / 0.111 / 0.119 ms on 700x500 at 1e-25
+    a.fx_runs = fx ? std::max(1, (a.fxs ? 64 : 32) / K) : 1;
     // 4 persistent waves per SIMD: the workgroup whose queues and windows fill a CU's
     // LDS (more would wait for it to end; fewer hide too little latency:
     // 2 waves 2.8-3.0 against 2.0 ms on the 1e-30 view, 1.29 against 0.91 ms on 16

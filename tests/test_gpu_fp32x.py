@@ -122,3 +122,31 @@ def test_no_series_deltas_at_width_1e200(gpu):
     print("FP32X vs FP64 at 1e-200 (no series): counts equal on %.3f%%, max |diff| %d" % (
         100 * same.mean(), np.abs(g32["iterations"].astype(np.int64) - g64["iterations"]).max()))
     assert same.mean() >= 0.95
+
+
+@pytest.mark.parametrize("K", [8, 12, 16, 32])
+@pytest.mark.parametrize("name,nr,nc,width,N", [("t13", 31, 70, "3e-23", 8000), ("t13", 31, 70, "1e-24", 7990),
+                                                ("t11", 33, 65, "1e-15", 3000)])
+def test_blocks_between_refills_keep_results(gpu, name, nr, nc, width, N, K):
+    """Up to 64 steps of blocks run between refills where the series is in floatexp, up
+    to 32 where it is in doubles, past an escape, the orbit's end and the limit N (also
+    where it falls inside them): grids and step counts of the oracle's single blocks."""
+    import newman_amd as nm
+    v = _VIEWS[name]
+    m, o = nm.Mandelbrot(nr, nc), O.OView(nr, nc)
+    for x in (m, o):
+        x.set_view(N, v["re"], v["im"], width)
+    m.precompute()
+    o.precompute_at(*m.reference_point())
+    m.set_delta_mode(1)
+    rc = np.array([(r, c) for r in range(nr) for c in range(nc)], dtype=np.int32)
+    want = o.pert_samples_fx(rc, K).reshape(nr, nc)
+    stats = []
+    for mode in (nm.NM_SERIES_DOUBLE, nm.NM_SERIES_FLOATEXP):
+        m.set_series_mode(mode)
+        stats.append(m.render(block_k=K))
+        g = m.grid()
+        assert np.array_equal(g["iterations"], want["iterations"])
+        assert np.array_equal(g["smoothing"].view(np.uint32), want["smoothing"].view(np.uint32))
+    for k in ("executed", "credited", "n_rebased"):
+        assert stats[0][k] == stats[1][k], k
