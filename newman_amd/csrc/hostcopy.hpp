@@ -1,10 +1,11 @@
 // hostcopy.hpp - results from the device into the caller's ordinary memory.  The
 // runtime's own copy of pageable memory moves 16 GB/s here: one thread copies out of
-// a staging buffer and takes the page faults of a fresh destination.  HostCopy sends
-// the bytes through a pinned ring in chunks at the link's 56 GB/s, and up to kHelpers
-// threads besides the caller copy each chunk on as it arrives: 40 MB into a fresh
-// array 3.85 -> 1.23 ms (two helpers 1.26, one 1.66, none 2.92; 512 KB chunks 2.0,
-// as a chunk costs the link some 17 us).
+// a staging buffer and takes the page faults of a fresh destination (0.2-1 us each).
+// HostCopy sends the bytes through a pinned ring in chunks at the link's 56 GB/s, and
+// up to kHelpers threads besides the caller take pieces of a chunk: they touch the
+// piece's pages while it is on its way and copy it on when it is there.  40 MB into a
+// fresh array 3.85 -> 1.23 ms (two helpers 1.26, one 1.66, none 2.92; 512 KB chunks
+// 2.0, as a chunk costs the link some 17 us).
 //
 // The ring (at most kRing bytes) and the helpers belong to the one engine of the
 // process, whose calls are serialised: one copy at a time, and a copy is over when
@@ -12,10 +13,13 @@
 // is over.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <sys/mman.h>
 
 #include <algorithm>
 #include <atomic>
+#include <cerrno>
 #include <condition_variable>
+#include <cstdint>
 #include <cstring>
 #include <mutex>
 #include <thread>
@@ -26,10 +30,12 @@ namespace nm {
 class HostCopy {
  public:
   static constexpr size_t kRing = (size_t)32 << 20;
-  // Up to here the runtime's copy: 2.8 MB into memory in use 0.17 ms against 0.25
-  // (a chunk's fixed cost again), 7.4 MB the same either way.
-  static constexpr size_t kDirect = (size_t)8 << 20;
+  // Up to here the runtime's copy.  Whole calls that return 1.2 MB into memory in use
+  // or a fresh array: 153 and 403 us with it, 135 and 191 with the ring; 2.8 MB 233
+  // and 711, 178 and 319; 6.2 MB 425 and 930, 295 and 500.
+  static constexpr size_t kDirect = (size_t)1 << 20;
   static constexpr int kHelpers = 3;
+  static constexpr size_t kPiece = (size_t)256 << 10;  // what a thread takes at a time (128 KB of 512 KB chunks: 217 and 549 us)
 
   // dst[0, bytes) = src (device), after the stream's earlier work; returns when the
   // bytes are there (or with the first error, when no thread touches dst any more)
@@ -40,28 +46,29 @@ class HostCopy {
     }
     const size_t chunk = bytes >= ((size_t)24 << 20) ? (size_t)2 << 20 : (size_t)1 << 20;
     const int n = (int)((bytes + chunk - 1) / chunk), slots = (int)std::min<size_t>(ring_ / chunk, kEvents);
+    const int per = (int)(chunk / kPiece);
     Job j;
     j.dst = (char*)dst;
     j.ring = (const char*)pinned_;
     j.bytes = bytes;
-    j.chunk = chunk;
-    j.n = n;
+    j.per = per;
     j.slots = slots;
     j.events = events_.data();
-    std::vector<std::atomic<uint8_t>> done((size_t)n);
+    std::vector<std::atomic<int>> done((size_t)n);  // pieces of each chunk that left the ring
     j.done = done.data();
     open(&j, kHelpers);
     hipError_t err = hipSuccess;
     for (int i = 0; i < n && err == hipSuccess; i++) {
       // the slot's previous chunk must have left it; meanwhile this thread helps
-      while (i >= slots && !j.done[i - slots].load(std::memory_order_acquire))
+      while (i >= slots && j.done[i - slots].load(std::memory_order_acquire) < per)
         if (!j.step()) std::this_thread::yield();
       if (j.error.load() != hipSuccess) break;
       const size_t o = (size_t)i * chunk;
       err = hipMemcpyAsync((char*)pinned_ + (size_t)(i % slots) * chunk, (const char*)src + o, std::min(chunk, bytes - o),
                            hipMemcpyDeviceToHost, stream);
       if (err == hipSuccess) err = hipEventRecord(events_[i % slots], stream);
-      if (err == hipSuccess) j.issued.store(i + 1, std::memory_order_release);
+      if (err == hipSuccess)
+        j.issued.store((int)std::min<size_t>((size_t)(i + 1) * per, (bytes + kPiece - 1) / kPiece), std::memory_order_release);
     }
     if (err != hipSuccess) j.error.store(err);
     j.closed.store(true, std::memory_order_release);
@@ -79,29 +86,51 @@ class HostCopy {
   struct Job {
     char* dst = nullptr;
     const char* ring = nullptr;
-    size_t bytes = 0, chunk = 0;
-    int n = 0, slots = 0;
+    size_t bytes = 0;
+    int per = 0, slots = 0;  // pieces of a chunk, chunks of the ring
     const hipEvent_t* events = nullptr;
-    std::atomic<uint8_t>* done = nullptr;
+    std::atomic<int>* done = nullptr;
     std::atomic<int> next{0}, issued{0}, error{hipSuccess};
     std::atomic<bool> closed{false};
     int inside = 0;  // helpers in the job (HostCopy::mu_)
 
-    // copies one chunk on; false: none is issued that nobody has taken
+    // copies one piece on; false: none is issued that nobody has taken
     bool step() {
       int i = next.load(std::memory_order_relaxed);
       do {
         if (i >= issued.load(std::memory_order_acquire)) return false;
       } while (!next.compare_exchange_weak(i, i + 1));
-      const hipError_t e = error.load() == hipSuccess ? hipEventSynchronize(events[i % slots]) : hipErrorUnknown;
-      const size_t o = (size_t)i * chunk;
-      if (e == hipSuccess) std::memcpy(dst + o, ring + (size_t)(i % slots) * chunk, std::min(chunk, bytes - o));
+      const int c = i / per, slot = c % slots;
+      const size_t o = (size_t)i * kPiece, size = std::min(kPiece, bytes - o);
+      hipError_t e = error.load() == hipSuccess ? hipSuccess : hipErrorUnknown;
+      if (e == hipSuccess) {
+        populate(dst + o, size);
+        e = hipEventSynchronize(events[slot]);
+      }
+      if (e == hipSuccess) std::memcpy(dst + o, ring + ((size_t)slot * per + i % per) * kPiece, size);
       else if (error.load() == hipSuccess) error.store(e);
-      done[i].store(1, std::memory_order_release);
+      done[c].fetch_add(1, std::memory_order_release);
       return true;
     }
     bool over() const { return closed.load(std::memory_order_acquire) && next.load() >= issued.load(); }
   };
+
+  // the pages of a destination that nobody has touched yet, while its bytes are on
+  // their way; without the call (Linux before 5.14) the copy takes the faults
+  static void populate(char* p, size_t n) {
+#ifdef MADV_POPULATE_WRITE
+    constexpr uintptr_t page = 4096;
+    const uintptr_t a = ((uintptr_t)p + page - 1) & ~(page - 1), b = ((uintptr_t)p + n) & ~(page - 1);
+    if (b > a) {
+      const int keep = errno;
+      (void)madvise((void*)a, b - a, MADV_POPULATE_WRITE);
+      errno = keep;
+    }
+#else
+    (void)p;
+    (void)n;
+#endif
+  }
 
   // the ring and its events, and the helpers (once); false: do without
   bool prepare(size_t bytes) {

@@ -1,14 +1,17 @@
 """Large results reach the caller through a pinned ring that several threads empty:
-sizes around its threshold (8 MB), its chunk sizes (1 and 2 MB) and its 32 MB, each
-against the same frames rendered one at a time into small copies."""
+sizes around its threshold (1 MB), its pieces (256 KB), its chunks (1 and 2 MB) and its
+32 MB, each against the same frames rendered one at a time into small copies."""
 import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("nr,nc,frames", [(512, 2048, 1),      # 8 MB: the last size of the runtime's copy
-                                          (512, 2049, 1),      # just past it
+@pytest.mark.parametrize("nr,nc,frames", [(256, 512, 1),       # 1 MB: the last size of the runtime's copy
+                                          (1, 131073, 1),      # 8 bytes past it: a chunk and a piece of 8 bytes
+                                          (300, 701, 1),       # 1.7 MB: a ragged last piece
+                                          (512, 2048, 1),      # 8 MB: whole chunks
+                                          (512, 2049, 1),      # and a little more
                                           (600, 801, 6),       # 23.1 MB: 1 MB chunks, a ragged last one
                                           (1024, 1023, 4),     # 32.7 MB in 2 MB chunks: most of the ring
                                           (1000, 1111, 9)])    # 80 MB: the ring's slots are used again
