@@ -117,8 +117,11 @@ struct Common {
   double smooth_k;  // 0.5 ln 2 / ln(bailout), or 0 for a bailout below 2
 };
 
+struct PlainArgs;
+typedef void (*PlainKernel)(PlainArgs);
 struct PlainArgs {
   Common c;
+  PlainKernel direct;  // the pass in one launch (k_plain_direct), or null
   int pre_iter;  // updates tried in the start kernel before a sample is handed on
   int k_start;   // updates every handed-on sample has done: pre_iter rounded up to the start kernel's blocks of 4
   const double* cre;
@@ -522,13 +525,15 @@ __device__ __forceinline__ DevFrame uniform_frame(const DevFrame* frames, uint32
 // stay below 2^20 * 1027 < 2^31.
 struct StartCounts {
   uint32_t ncard = 0, nres = 0, executed = 0, credited = 0;
+  uint32_t handed = 0, late = 0;  // k_plain_direct: samples past k_start updates, and their updates past them
 };
 
 // One sample of the start kernel (getIterationsHW, mandelbrot.cpp:231-254): the
 // lane's sample is frame-local index gid - f.sample_base of frame f when valid.
 // Every lane of the wave runs this (no early return), so the pre-iteration is
-// wave-uniform control flow.  Returns whether the sample is handed on.
-template <bool FMA2, bool GROUPED>
+// wave-uniform control flow.  Returns whether the sample is handed on.  DIRECT (pre =
+// N: none is): the counts as a start and an iterate kernel would share them.
+template <bool FMA2, bool GROUPED, bool DIRECT = false>
 __device__ __forceinline__ bool start_sample(const PlainArgs& a, const DevFrame& f, const uint32_t gid, bool valid,
                                              const int pre, const double2* ltab, StartCounts& n) {
   const Common& c = a.c;
@@ -560,10 +565,39 @@ __device__ __forceinline__ bool start_sample(const PlainArgs& a, const DevFrame&
   double x = zx, y = zy, r2 = x * x, i2 = y * y, mgesc = 0.0;
   unsigned long long live = __ballot(alive);
   int kend = 0;
-  PreLane L{x, y, r2, i2, zx, zy, live, alive, kesc, mgesc};
-  while (live != 0 && kend < pre) {
-    pre_block<0, GROUPED ? kStartGroup : 1, FMA2>(L, c.b2, kend);
-    kend += 4;
+  if constexpr (DIRECT && GROUPED) {
+    // groups of the iterate kernel's size: an escape keeps the value before its group,
+    // which runs again at the end
+    double gx = 0.0, gy = 0.0;
+    int gk = -1;
+    for (; live != 0 && kend < pre; kend += kIterGroup) {
+      const double x0 = x, y0 = y;
+#pragma unroll
+      for (int t = 0; t < kIterGroup; t++) plain_update<FMA2>(x, y, r2, i2, zx, zy);
+      const unsigned long long e = __ballot(!(r2 + i2 <= c.b2)) & live;
+      live &= ~e;
+      if (__builtin_amdgcn_inverse_ballot_w64(e)) {
+        gx = x0;
+        gy = y0;
+        gk = kend;
+      }
+    }
+    if (gk >= 0) {
+      r2 = gx * gx;
+      i2 = gy * gy;
+      for (int j = 0;; j++) {
+        plain_update<FMA2>(gx, gy, r2, i2, zx, zy);
+        mgesc = r2 + i2;
+        kesc = gk + j;
+        if (mgesc > c.b2 || j == kIterGroup - 1) break;
+      }
+    }
+  } else {
+    PreLane L{x, y, r2, i2, zx, zy, live, alive, kesc, mgesc};
+    while (live != 0 && kend < pre) {
+      pre_block<0, GROUPED ? kStartGroup : 1, FMA2>(L, c.b2, kend);
+      kend += 4;
+    }
   }
   bool want = false;
   if (valid && in) {
@@ -572,7 +606,16 @@ __device__ __forceinline__ bool start_sample(const PlainArgs& a, const DevFrame&
   } else if (valid) {
     // the reference tests k >= N before each update: an escape counts
     // only below N; a lane still iterating after kend updates is handed on
-    if (kesc >= 0 && kesc < N) {
+    if constexpr (DIRECT) {
+      const bool esc = kesc >= 0 && kesc < N;
+      const int done = esc ? kesc + 1 : N;
+      c.out[gid] = esc ? EscapeValue{kesc, smooth_of(mgesc, c, ltab)} : EscapeValue{N, 0.0f};
+      n.credited += (uint32_t)(esc ? kesc : N);
+      n.executed += (uint32_t)min(done, a.k_start);
+      n.late += (uint32_t)max(done - a.k_start, 0);
+      if (done > a.k_start) n.handed++;
+      else n.nres++;
+    } else if (kesc >= 0 && kesc < N) {
       n.executed += (uint32_t)(kesc + 1);
       c.out[gid] = EscapeValue{kesc, smooth_of(mgesc, c, ltab)};
       n.nres++;
@@ -646,6 +689,42 @@ __global__ __launch_bounds__(kThreads) void k_plain_start(PlainArgs a) {
   const unsigned long long v[4] = {n.ncard, n.nres, n.executed, n.credited};
   const int idx[4] = {C_CARDIOID, C_SA_RES, C_EXEC_START, C_CREDITED};
   block_partial(c.part, kSlotStart + blockIdx.x, v, idx, 4);
+}
+
+// The plain pass of a small frame set in one launch, a wave per 64 consecutive samples:
+// up to kDirectSamples a SIMD has a wave or two, the pass takes as long as its longest
+// sample in any case, and handing samples on, compacting and refilling only add launches
+// to that.  Renders of 160x120 at N 256 / 1024 of the whole set 58 -> 47 / 70 -> 60 us,
+// N 2048 of the period-3 island 84 -> 76; 420x300 (two waves a SIMD) 57 -> 51, 70 -> 72
+// and 112 -> 100 us; at 640x480 the waves that wait for their longest sample cost more.
+constexpr uint32_t kDirectSamples = 1u << 17;
+template <bool FMA2, bool GROUPED>
+__global__ __launch_bounds__(64) void k_plain_direct(PlainArgs a) {
+  const Common& c = a.c;
+  StartCounts n;
+  const uint32_t first = blockIdx.x * 64u, gid = first + threadIdx.x, last = min(first + 63u, c.total - 1u);
+  const uint32_t f0 = frame_of(first, c.inv_frame);
+  if (f0 == frame_of(last, c.inv_frame)) {
+    start_sample<FMA2, GROUPED, true>(a, uniform_frame(c.frames, f0), gid, gid < c.total, c.N, d_log2tab, n);
+  } else {
+    const bool valid = gid < c.total;
+    start_sample<FMA2, GROUPED, true>(a, c.frames[valid ? frame_of(gid, c.inv_frame) : 0u], gid, valid, c.N,
+                                      d_log2tab, n);
+  }
+  const unsigned long long v[6] = {n.ncard, n.nres, n.executed, n.credited, n.late, n.handed};
+  // the plain path rebases nothing: that counter holds the samples handed on
+  const int idx[6] = {C_CARDIOID, C_SA_RES, C_EXEC_START, C_CREDITED, C_EXECUTED, C_REBASED};
+  block_partial(c.part, kSlotStart + blockIdx.x, v, idx, 6);
+}
+static_assert(kSlotStart + kDirectSamples / 64 <= kSlotIter, "a partial slot per workgroup");
+
+// null where the pass takes its usual kernels
+static PlainKernel direct_kernel(uint64_t total, bool fma2, bool grouped) {
+  if (total > kDirectSamples) return nullptr;
+  return fma2 && grouped ? k_plain_direct<true, true>
+         : fma2          ? k_plain_direct<true, false>
+         : grouped       ? k_plain_direct<false, true>
+                         : k_plain_direct<false, false>;
 }
 
 // ============================================================ compaction
@@ -2270,6 +2349,13 @@ static int tile_grid(uint64_t total, int num_cu) {
 }
 
 static void launch_safe(hipStream_t, const PlainArgs&) {}
+// the workgroups of a pass in one launch, or 0
+static int direct_grid(const PlainArgs& a) { return a.direct ? (int)((a.c.total + 63u) / 64u) : 0; }
+static int direct_grid(const SeriesArgs&) { return 0; }
+static void launch_direct(hipStream_t stream, const PlainArgs& a) {
+  hipLaunchKernelGGL(a.direct, dim3(direct_grid(a)), dim3(64), 0, stream, a);
+}
+static void launch_direct(hipStream_t, const SeriesArgs&) {}
 static void launch_safe(hipStream_t stream, const SeriesArgs& a) {
   if (!a.safe) return;
   hipLaunchKernelGGL(k_safe, dim3(std::min(512, a.mend / 256 + 1)), dim3(256), 0, stream, a.Zd, a.mend, a.radius,
@@ -2296,6 +2382,13 @@ static hipError_t launch_pass_on(hipStream_t stream, int num_cu, unsigned long l
     if ((e = hipGetLastError()) != hipSuccess) return e; \
   } while (0)
   if (evs && (e = hipEventRecord(evs[0], stream)) != hipSuccess) return e;
+  if (direct_grid(args)) {
+    NM_LAUNCH_OK(launch_direct(stream, args));
+    for (int i = 1; evs && i < 4; i++)
+      if ((e = hipEventRecord(evs[i], stream)) != hipSuccess) return e;
+    if (emit_to) NM_LAUNCH_OK(hipLaunchKernelGGL(k_emit, dim3(gtile), dim3(kThreads), 0, stream, c, emit_to));
+    return evs ? hipEventRecord(evs[4], stream) : hipSuccess;
+  }
   NM_LAUNCH_OK(launch_safe(stream, args));
   NM_LAUNCH_OK(hipLaunchKernelGGL(start, dim3(gtile), dim3(kThreads), 0, stream, args));
   if (evs && (e = hipEventRecord(evs[1], stream)) != hipSuccess) return e;
@@ -2649,11 +2742,13 @@ class EngineImpl : public Engine {
       }
     }
     // the counters and the results follow the pass without a wait in between
+    const int dgrid = direct_grid(args);
     const EscapeValue* result = emit_to ? emit_to : (const EscapeValue*)d_out;
     hipError_t ce = hipSuccess;
     if (st == NM_OK) {
       hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(kReduceThreads), 0, stream, (const unsigned long long*)d_part,
-                         tile_grid(args.c.total, num_cu), iterate_grid(num_cu, waves, iter_threads<Args>(waves)),
+                         dgrid ? dgrid : tile_grid(args.c.total, num_cu),
+                         dgrid ? 0 : iterate_grid(num_cu, waves, iter_threads<Args>(waves)),
                          (const uint32_t*)d_nactive, h_totals);
       ce = hipGetLastError();
       if (ce == hipSuccess && host_out)
@@ -2682,7 +2777,7 @@ class EngineImpl : public Engine {
       ms_graph += t / (repeats - 1);
     }
     const unsigned long long* h = h_totals->count;
-    const uint32_t nact = h_totals->nactive;
+    const uint32_t nact = dgrid ? (uint32_t)h[C_REBASED] : h_totals->nactive;
     if (stats) {
       stats->samples = nout;
       stats->n_cardioid = h[C_CARDIOID];
@@ -2691,7 +2786,7 @@ class EngineImpl : public Engine {
       stats->executed = h[C_EXECUTED] + h[C_EXEC_START];
       stats->executed_start = h[C_EXEC_START];
       stats->skipped = h[C_SKIPPED];
-      stats->n_rebased = h[C_REBASED];
+      stats->n_rebased = dgrid ? 0 : h[C_REBASED];
       stats->credited = h[C_CREDITED];
       stats->ms_start = ms[0];
       stats->ms_compact = ms[1];
@@ -2737,6 +2832,7 @@ class EngineImpl : public Engine {
     if ((st = grow(&d_tabs, &n_tabs_bytes, (2 * ncol + 2 * nrow) * sizeof(double)))) return st;
     const bool upload = tables_stale(opt, pf == d_frames && pt == d_tabs);
     PlainArgs a;
+    a.direct = nullptr;
     if ((st = prepare_common(a.c, total, opt))) return st;
     EscapeValue* emit_to = nullptr;
     if (opt.tile) {
@@ -2783,6 +2879,9 @@ class EngineImpl : public Engine {
       stats->fma2 = fma2 ? 1 : 0;
       stats->grouped = grouped ? 1 : 0;
     }
+    // launch settings are those of the usual kernels
+    if (opt.pre_iter == 0 && opt.block_k == 0 && opt.waves_per_simd == 0)
+      a.direct = direct_kernel(a.c.total, fma2, grouped);
 #define NM_PLAIN(KK)                                                                                           \
   return fma2 && grouped ? run(a, k_plain_start<true, true>, k_plain_iterate<KK, true, true>, waves, opt, stats,  \
                             nout, host_out, emit_to)                                                           \
@@ -3317,6 +3416,7 @@ int render_hw_noalloc(const HwFrameHost& f, int N, double bailout, EscapeValue* 
   a.cim = tabs + 2 * f.nc;
   a.cimlo = tabs + 2 * f.nc + f.nr;
   const bool fma2 = f.fma_ok && bailout <= 0x1p400, grouped = grouped_test_ok(bailout, f.c_bound);
+  a.direct = direct_kernel(n, fma2, grouped);
   NA_HIP(fma2 && grouped ? launch_pass_on(s, d->num_cu, part, nactive, a, k_plain_start<true, true>,
                                        k_plain_iterate<64, true, true>, kPlainWaves, nullptr, nullptr)
          : fma2       ? launch_pass_on(s, d->num_cu, part, nactive, a, k_plain_start<true, false>,

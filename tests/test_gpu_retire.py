@@ -67,3 +67,23 @@ def test_groups_that_overflow(gpu, k, bailout):
             v.set_bailout(bailout)
         m.render(block_k=k)
         assert np.array_equal(m.grid()["iterations"], o.render_rows(np.arange(30, dtype=np.int32))["iterations"])
+
+
+@pytest.mark.parametrize("nr,nc,count", [(1, 1, 1), (1, 65, 1), (7, 19, 3), (256, 512, 1), (257, 511, 1), (64, 64, 33)])
+@pytest.mark.parametrize("bailout", [1.5, 1024.0])
+def test_small_sets_in_one_launch(gpu, nr, nc, count, bailout):
+    """Up to 131072 samples of the plain path take one launch, more the usual kernels;
+    a launch setting always takes those: the same grids and the same counts, frames
+    that share a wave among them, and the oracle's."""
+    m, o = gpu.Mandelbrot(nr, nc), O.OView(nr, nc)
+    widths = ["%.6f" % (3.0 / 1.3 ** k) for k in range(count)]
+    for N in (13, 16, 300):
+        for v in (m, o):
+            v.set_view(N, "-0.6", "0.4", "3.0")
+            v.set_bailout(bailout)
+        got, st = m.render_frames(widths)
+        want, usual = m.render_frames(widths, block_k=64)
+        assert np.array_equal(got, want)
+        for k in ("n_cardioid", "n_sa_resolved", "n_iterated", "executed", "executed_start", "credited", "n_rebased"):
+            assert st[k] == usual[k], k
+        assert np.array_equal(got[0]["iterations"], o.render_rows(np.arange(nr, dtype=np.int32))["iterations"])
