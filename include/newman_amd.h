@@ -168,6 +168,10 @@ int nm_probe_candidates(const nm_mandelbrot* h);
 /* reference series as the device sees it: X (nearest), A, B, C (truncated),
  * 2*len doubles each (re, im interleaved); any pointer may be NULL */
 int nm_get_reference(const nm_mandelbrot* h, double* X, double* A, double* B, double* C);
+/* its other tables: what X leaves of the orbit (nearest), and the floatexp form of A,
+ * B, C one after the other, 2*len mantissas and exponents each (exponent -2^30 for a
+ * zero); any pointer may be NULL */
+int nm_get_reference_tables(const nm_mandelbrot* h, double* Xlo, double* m, int32_t* e);
 /* render every row with explicit engine settings and `repeats` timed launches;
  * copy_back = 0 leaves the grid on the device (benchmarks).  block_k: 0 for the
  * default (plain 64; series FP64 64, FP32X 8), else plain 8/16/32/64, series

@@ -228,6 +228,7 @@ _SIGS = [
     ("nm_set_probe_mode", C.c_int, [_H, C.c_int]),
     ("nm_probe_candidates", C.c_int, [_H]),
     ("nm_get_reference", C.c_int, [_H, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]),
+    ("nm_get_reference_tables", C.c_int, [_H, C.c_void_p, C.c_void_p, C.c_void_p]),
     ("nm_render", C.c_int, [_H, C.c_int, C.c_int, C.c_int, C.c_int, C.POINTER(RenderStats)]),
     ("nm_render_frames", C.c_int, [_H, C.POINTER(C.c_char_p), C.c_int, C.c_int, C.c_int, C.c_int, C.c_void_p,
                                    C.POINTER(RenderStats)]),
@@ -537,6 +538,14 @@ class Mandelbrot:
         _check(lib().nm_get_reference(self._h, X.ctypes.data, A.ctypes.data, B.ctypes.data, Cc.ctypes.data),
                "nm_get_reference")
         return X, A, B, Cc
+
+    def reference_tables(self):
+        """The orbit's remainders, and (mantissas, exponents) of A, B and C."""
+        n = 2 * self.reference_length()
+        xlo, m, e = np.zeros(n), np.zeros(3 * n), np.zeros(3 * n, dtype=np.int32)
+        _check(lib().nm_get_reference_tables(self._h, xlo.ctypes.data, m.ctypes.data, e.ctypes.data),
+               "nm_get_reference_tables")
+        return xlo, [(m[k * n:(k + 1) * n], e[k * n:(k + 1) * n]) for k in range(3)]
 
     def render(self, block_k=0, waves_per_simd=0, repeats=1, copy_back=True):
         st = RenderStats()

@@ -19,7 +19,7 @@ LIB = os.path.join(HERE, "libnewman_amd.so")
 INDEX_CHECK_LIB = os.path.join(HERE, "libnm_index_check.so")
 ARCH = os.environ.get("NEWMAN_AMD_ARCH", "gfx950")
 
-HOST_SRCS = ["hpfloat.cpp", "mandelbrot.cpp", "palette.cpp", "video.cpp", "capi.cpp"]
+HOST_SRCS = ["hpfloat.cpp", "series_chain.cpp", "mandelbrot.cpp", "palette.cpp", "video.cpp", "capi.cpp"]
 HIP_SRCS = ["kernels.hip", "coords.hip", "orbit.hip", "skipnet.hip", "colour.hip", "video.hip"]
 
 CXXFLAGS = ["-O2", "-fPIC", "-std=c++17", "-ffp-contract=off", "-fno-fast-math", "-Wall", "-Wno-unused-function",
@@ -60,7 +60,8 @@ def build_index_check():
     share; the HIP headers supply its host/device qualifiers."""
     tmp = INDEX_CHECK_LIB + ".tmp"
     _run(["g++"] + CXXFLAGS + ["-Wno-unknown-pragmas", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-shared", "-o", tmp,
-                               os.path.join(CSRC, "index_check.cpp"), os.path.join(CSRC, "hpfloat.cpp")])
+                               os.path.join(CSRC, "index_check.cpp"), os.path.join(CSRC, "hpfloat.cpp"),
+                               os.path.join(CSRC, "series_chain.cpp")])
     os.replace(tmp, INDEX_CHECK_LIB)
     return INDEX_CHECK_LIB
 

@@ -333,6 +333,21 @@ int nm_get_reference(const nm_mandelbrot* h, double* X, double* A, double* B, do
   return NM_OK;
 }
 
+int nm_get_reference_tables(const nm_mandelbrot* h, double* Xlo, double* m, int32_t* e) {
+  if (!h) return NM_ERR_ARG;
+  const nm::SaReferenceHost& r = h->m.reference();
+  if (r.len <= 0) return NM_ERR_STATE;
+  const size_t n = 2 * (size_t)r.len;
+  if (Xlo) std::memcpy(Xlo, r.Xlo.data(), n * sizeof(double));
+  const std::vector<double>* ms[3] = {&r.Am, &r.Bm, &r.Cm};
+  const std::vector<int32_t>* es[3] = {&r.Ae, &r.Be, &r.Ce};
+  for (int k = 0; k < 3; k++) {
+    if (m) std::memcpy(m + k * n, ms[k]->data(), n * sizeof(double));
+    if (e) std::memcpy(e + k * n, es[k]->data(), n * sizeof(int32_t));
+  }
+  return NM_OK;
+}
+
 int nm_render(nm_mandelbrot* h, int block_k, int waves_per_simd, int repeats, int copy_back,
               nm_render_stats* stats) {
   if (!h || repeats < 1 || block_k < 0 || waves_per_simd < 0) return NM_ERR_ARG;

@@ -75,6 +75,9 @@ void hp_set_d(hpf& r, double d);
 bool hp_set_str(hpf& r, const char* s);         // false on a malformed string
 int hp_cmp(const hpf& a, const hpf& b);         // -1, 0, +1 (exact)
 void hp_neg(hpf& r, const hpf& a);
+inline void times2(hpf& x) {
+  if (x.sign) x.exp += 1;  // 2.0 * x is exact
+}
 // copy value and precision (copy construction semantics into an existing object)
 inline void hp_copy_prec(hpf& d, const hpf& s) { std::memcpy((void*)&d, (const void*)&s, sizeof(hpf)); }
 

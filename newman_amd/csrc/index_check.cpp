@@ -29,7 +29,9 @@
 
 #include "coords.hpp"
 #include "hpfloat.hpp"
+#include "orbit_steps.hpp"
 #include "sample_index.hpp"
+#include "series_chain.hpp"
 
 namespace {
 
@@ -547,8 +549,166 @@ long long coords_check(unsigned seed, int n) {
   }
   return bad;
 }
+
+// The device's passes over an orbit (orbit.hip's sweeps, terms and emission, one value
+// after the other) against the host's chain.  out[0]: the bound (orbit_tables_hold)
+// accepts; out[1]: doubles, mantissas or exponents that differ; out[2]: the most bits
+// that cancelled in one step of A; out[3]: values off from the host's by more than
+// their bound; out[4]: the largest such difference in units of the bound, times 2^10.
+template <int ML>
+long long orbit_check(const std::vector<nm::HPComplex>& X, int len, int L, long long* out) {
+  typedef nm::hpd<ML> V;
+  const int n = len - 1, c = std::max(1, (int)std::ceil(std::cbrt((double)n)));
+  const int n1 = (n + c - 1) / c, n2 = (n1 + c - 1) / c;
+  std::vector<V> x(2 * (size_t)(len + 1));
+  std::vector<double> Zd(2 * (size_t)(len + 2), 0.0);
+  bool real = true;
+  for (int k = 0; k <= len; k++)
+    for (int p = 0; p < 2; p++) {
+      const nm::hpf& v = p ? X[k].im : X[k].re;
+      x[2 * (size_t)k + p] = nm::hpd_load<ML>(val_of(v));
+      Zd[2 * (size_t)(k + 1) + p] = nm::hpd_nearest(x[2 * (size_t)k + p], L);
+      if (p && k < len && v.sign) real = false;
+    }
+  // chunk q of the elements, v = factor v + terms; as orbit.hip's k_sweep
+  auto sweep = [&](const std::vector<V>& f, const V* u1, const V* u2, bool twice, bool one, int count, int chunk,
+                   const V* start, int first, V* end, V* before, V* after, V* product) {
+    for (int side = 0; side < (product ? 2 : 1); side++)
+      for (int q = 0; q * chunk < count; q++) {
+        V v[2] = {nm::hpd_small<ML>(side ? 1 : first), nm::hpd_small<ML>(0)};
+        if (start && !side) v[0] = start[2 * q], v[1] = start[2 * q + 1];
+        for (int e = q * chunk; e < std::min(count, (q + 1) * chunk); e++) {
+          V s[2];
+          for (int p = 0; p < 2; p++) {
+            if (before && !side) before[2 * e + p] = v[p];
+            s[p] = nm::sweep_part(p, f[2 * e], f[2 * e + 1], v[p], v[1 - p], twice, one && !side,
+                                  u1 && !side ? u1 + 2 * e + p : nullptr, u2 && !side ? u2 + 2 * e + p : nullptr, L);
+          }
+          for (int p = 0; p < 2; p++) {
+            v[p] = s[p];
+            if (after && !side) after[2 * e + p] = s[p];
+          }
+        }
+        for (int p = 0; p < 2; p++) {
+          if (side) product[2 * q + p] = v[p];
+          else if (end) end[2 * q + p] = v[p];
+        }
+      }
+  };
+  std::vector<V> P1(2 * n1), E1(2 * n1), S1(2 * n1), P2(2 * n2), E2(2 * n2), S2(2 * n2), y[3], u1(2 * n), u2(2 * n);
+  std::vector<V> chain[3];  // the host's chain: one chunk
+  std::vector<double> trace(3 * (size_t)len, -1.0);
+  std::fill(trace.begin(), trace.begin() + 3 * (c + 1), 0.0);
+  std::vector<uint16_t> run[3];
+  std::vector<int32_t> gap[3], ex[3];
+  nm::SaReferenceHost r;
+  nm::series_chain(X.data(), len, L, r);
+  const std::vector<double>*hd[3] = {&r.A, &r.B, &r.C}, *hm[3] = {&r.Am, &r.Bm, &r.Cm};
+  const std::vector<int32_t>* he[3] = {&r.Ae, &r.Be, &r.Ce};
+  out[1] = out[2] = 0;
+  for (int k = 0; k < 3; k++) {
+    chain[k].assign(2 * (size_t)len, nm::hpd_small<ML>(0));
+    chain[k][0] = nm::hpd_small<ML>(k == 0);
+    y[k] = chain[k];
+    auto terms = [&](const std::vector<V>* v) {
+      for (int e = 0; k && e < n; e++)
+        for (int p = 0; p < 2; p++)
+          nm::terms_part(p, &v[0][2 * (e + 1)], k == 2 ? &v[1][2 * (e + 1)] : nullptr, L, u1[2 * e + p], u2[2 * e + p]);
+    };
+    const V *t1 = k ? u1.data() : nullptr, *t2 = k ? u2.data() : nullptr;
+    terms(chain);
+    sweep(x, t1, t2, true, k == 0, n, n, nullptr, k == 0, nullptr, nullptr, chain[k].data() + 2, nullptr);
+    terms(y);
+    sweep(x, t1, t2, true, k == 0, n, c, nullptr, 0, E1.data(), nullptr, nullptr, k ? nullptr : P1.data());
+    sweep(P1, E1.data(), nullptr, false, false, n1, c, nullptr, 0, E2.data(), nullptr, nullptr, k ? nullptr : P2.data());
+    sweep(P2, E2.data(), nullptr, false, false, n2, n2, nullptr, k == 0, nullptr, S2.data(), nullptr, nullptr);
+    sweep(P1, E1.data(), nullptr, false, false, n1, c, S2.data(), 0, nullptr, S1.data(), nullptr, nullptr);
+    sweep(x, t1, t2, true, k == 0, n, c, S1.data(), 0, E1.data(), nullptr, y[k].data() + 2, nullptr);
+    for (int t = 0; t < 2 * (n1 - 1); t++) {
+      const V g = nm::hpd_add(S1[t + 2], E1[t], -1, L);
+      gap[k].push_back(g.sign ? (int32_t)g.exp : nm::kFxZeroExp);
+    }
+    for (size_t t = 0; t < 2 * (size_t)len; t++) {
+      const V& v = y[k][t];
+      const double m = v.sign ? v.sign * std::ldexp((double)(v.m[ML - 1] >> 11), -53) : 0.0;
+      ex[k].push_back(v.sign ? (int32_t)v.exp : nm::kFxZeroExp);
+      run[k].push_back(nm::hpd_run(v, L));
+      const double d = nm::hpd_get_d(v);
+      out[1] += d != (*hd[k])[t] || m != (*hm[k])[t] || ex[k][t] != (*he[k])[t];
+    }
+  }
+  out[0] = nm::orbit_tables_hold(Zd.data(), len, L, c, real, {ex[0].data(), ex[1].data(), ex[2].data()},
+                                 {run[0].data(), run[1].data(), run[2].data()},
+                                 {gap[0].data(), gap[1].data(), gap[2].data()}, trace.data());
+  int worst = 0;
+  out[3] = out[4] = 0;
+  for (int k = 0; k < 3; k++)
+    for (size_t t = 0; t < 2 * (size_t)len; t++) {
+      const double b = trace[3 * (t / 2) + k];
+      const V g = nm::hpd_add(y[k][t], chain[k][t], -1, L);
+      if (b < 0.0 || g.sign == 0) continue;  // not reached; the same
+      const int E = std::max(ex[k][t | 1], ex[k][t & ~(size_t)1]);
+      const double off = std::ldexp(0.5 * (1.0 + (double)(g.m[ML - 1] << 1) * 0x1p-64), (int)(g.exp - E) + 64 * L - 1);
+      out[3] += off > b;
+      out[4] = std::max<long long>(out[4], b > 0.0 ? (long long)(off / b * 1024.0) : 1024);
+    }
+  for (int i = 1; i < len; i++) {
+    const int e0 = std::max(ex[0][2 * (size_t)i - 2], ex[0][2 * (size_t)i - 1]),
+              e1 = std::max(ex[0][2 * (size_t)i], ex[0][2 * (size_t)i + 1]);
+    const int ez = std::ilogb(std::hypot(Zd[2 * (size_t)i], Zd[2 * (size_t)i + 1]));
+    worst = std::max(worst, std::max(e0 + ez + 1, 0) - e1);
+  }
+  out[2] = worst;
+  return 0;
+}
 }  // namespace
 extern "C" {
+// An orbit of `len` from (re, im) at L limbs through orbit_check.  out: accepted,
+// differing entries, the most bits that cancelled in a step of A.  cancel > 0: not the
+// point's own orbit, but after every `cancel` steps an x that all but cancels A's step
+// (to a double's last bits).
+long long nm_orbit_check(const char* re, const char* im, int L, int len, int cancel, long long* out) {
+  std::vector<nm::HPComplex> X;
+  nm::HPComplex c, z;
+  for (nm::hpf* v : {&c.re, &c.im, &z.re, &z.im}) *v = nm::hpf(L), v->L = L;
+  if (!nm::hp_set_str(c.re, re) || !nm::hp_set_str(c.im, im)) return -1;
+  nm::hp_copy_prec(z.re, c.re);
+  nm::hp_copy_prec(z.im, c.im);
+  nm::hpf t1(L), t2(L), ar(L), ai(L), br(L), bi(L), one(L);
+  nm::hp_set_d(one, 1.0);
+  nm::hp_set_d(ar, 1.0);
+  for (int k = 0; k <= len; k++) {
+    nm::HPComplex w;
+    w.re = nm::hpf(L), w.im = nm::hpf(L);
+    nm::hp_copy_prec(w.re, z.re);
+    nm::hp_copy_prec(w.im, z.im);
+    if (cancel > 0 && k % cancel == cancel - 1) {  // 2 x A = -1: x = -conj(A) / (2 |A|^2)
+      long er, ei;
+      double mr = ar.get_d_2exp(&er), mi = ai.get_d_2exp(&ei);
+      const long e = std::max(ar.sign ? er : -1000000l, ai.sign ? ei : -1000000l);
+      mr = ar.sign ? std::ldexp(mr, (int)std::max(-1000l, er - e)) : 0.0;
+      mi = ai.sign ? std::ldexp(mi, (int)std::max(-1000l, ei - e)) : 0.0;
+      const double q = 2.0 * (mr * mr + mi * mi);
+      nm::hp_set_d(w.re, -mr / q);
+      nm::hp_set_d(w.im, mi / q);
+      if (w.re.sign) w.re.exp -= e;
+      if (w.im.sign) w.im.exp -= e;
+    }
+    X.push_back(w);
+    // A's next value, for where to cancel
+    nm::hp_mul(br, w.re, ar); nm::hp_mul(t1, w.im, ai); nm::hp_sub(br, br, t1); nm::times2(br); nm::hp_add(br, br, one);
+    nm::hp_mul(bi, w.re, ai); nm::hp_mul(t1, w.im, ar); nm::hp_add(bi, bi, t1); nm::times2(bi);
+    nm::hp_copy_prec(ar, br);
+    nm::hp_copy_prec(ai, bi);
+    nm::hp_mul(t1, z.re, z.re); nm::hp_mul(t2, z.im, z.im); nm::hp_sub(t1, t1, t2);
+    nm::hp_mul(t2, z.re, z.im); nm::times2(t2);
+    nm::hp_add(z.re, t1, c.re);
+    nm::hp_add(z.im, t2, c.im);
+  }
+  if (L <= 4) return orbit_check<4>(X, len, L, out);
+  if (L <= 8) return orbit_check<8>(X, len, L, out);
+  return L <= 16 ? orbit_check<16>(X, len, L, out) : -1;
+}
 long long nm_hp_ops_check(int limbs, unsigned seed, int n) {
   switch (limbs) {
     case 4: return hp_ops_check<4>(seed, n);

@@ -12,6 +12,8 @@
 #include <limits>
 #include <thread>
 
+#include "series_chain.hpp"
+
 namespace nm {
 
 static constexpr double kMinPreview = 1.5e-16;  // mandelbrot.cpp:257
@@ -42,10 +44,6 @@ static void parallel_for(long total, F&& fn, long chunk = 4) {
 }
 
 // ------------------------------------------------------------------ helpers
-static inline void times2(hpf& x) {
-  if (x.sign) x.exp += 1;  // 2.0 * x is exact
-}
-
 // nearest-rounded double of an HP value (the perturbation kernels' reference
 // orbit), built on the truncating conversion
 static double get_d_nearest(const hpf& a) {
@@ -284,61 +282,10 @@ void Mandelbrot::findProbe() {
   ref_.len = len;
 }
 
-// mandelbrot.cpp:112-131, the recurrence exactly as written (A[i], B[i] on the
-// right-hand side of B[i], C[i]).  Only the truncated doubles the per-pixel work
-// reads are kept.
+// mandelbrot.cpp:112-131: on the device, or as the host's chain
 void Mandelbrot::computeSeries() {
   const int len = ref_.len;
-  if (orbitTables(len, true, ref_)) return;
-  const int L = hp_limbs_for_bits(hp_default_bits());
-  ref_.A.assign(2 * (size_t)len, 0.0);
-  ref_.B.assign(2 * (size_t)len, 0.0);
-  ref_.C.assign(2 * (size_t)len, 0.0);
-  ref_.Am.assign(2 * (size_t)len, 0.0);
-  ref_.Bm.assign(2 * (size_t)len, 0.0);
-  ref_.Cm.assign(2 * (size_t)len, 0.0);
-  ref_.Ae.assign(2 * (size_t)len, kFxZeroExp);
-  ref_.Be.assign(2 * (size_t)len, kFxZeroExp);
-  ref_.Ce.assign(2 * (size_t)len, kFxZeroExp);
-  ref_.Am[0] = 0.5;
-  ref_.Ae[0] = 1;
-  hpf Ar(L), Ai(L), Br(L), Bi(L), Cr(L), Ci(L), nAr(L), nAi(L), nBr(L), nBi(L), nCr(L), nCi(L), t(L);
-  hpf one(2);
-  hp_set_d(one, 1.0);
-  hp_set_d(Ar, 1.0);
-  ref_.A[0] = 1.0;
-  for (int i = 1; i < len; i++) {
-    const hpf& xr = X[i - 1].re;
-    const hpf& xi = X[i - 1].im;
-    hp_mul(nAr, xr, Ar); hp_mul(t, xi, Ai); hp_sub(nAr, nAr, t); times2(nAr); hp_add(nAr, nAr, one);
-    hp_mul(nAi, xr, Ai); hp_mul(t, xi, Ar); hp_add(nAi, nAi, t); times2(nAi);
-    hp_mul(nBr, xr, Br); hp_mul(t, xi, Bi); hp_sub(nBr, nBr, t); times2(nBr);
-    hp_mul(t, nAr, nAr); hp_add(nBr, nBr, t);
-    hp_mul(t, nAi, nAi); hp_sub(nBr, nBr, t);
-    hp_mul(nBi, xr, Bi); hp_mul(t, xi, Br); hp_add(nBi, nBi, t);
-    hp_mul(t, nAr, nAi); hp_add(nBi, nBi, t); times2(nBi);
-    hp_mul(nCr, xr, Cr); hp_mul(t, xi, Ci); hp_sub(nCr, nCr, t);
-    hp_mul(t, nAr, nBr); hp_add(nCr, nCr, t);
-    hp_mul(t, nAi, nBi); hp_sub(nCr, nCr, t); times2(nCr);
-    hp_mul(nCi, xr, Ci); hp_mul(t, xi, Cr); hp_add(nCi, nCi, t);
-    hp_mul(t, nAr, nBi); hp_add(nCi, nCi, t);
-    hp_mul(t, nAi, nBr); hp_add(nCi, nCi, t); times2(nCi);
-    hp_copy_prec(Ar, nAr); hp_copy_prec(Ai, nAi);
-    hp_copy_prec(Br, nBr); hp_copy_prec(Bi, nBi);
-    hp_copy_prec(Cr, nCr); hp_copy_prec(Ci, nCi);
-    ref_.A[2 * i] = Ar.get_d(); ref_.A[2 * i + 1] = Ai.get_d();
-    ref_.B[2 * i] = Br.get_d(); ref_.B[2 * i + 1] = Bi.get_d();
-    ref_.C[2 * i] = Cr.get_d(); ref_.C[2 * i + 1] = Ci.get_d();
-    const hpf* hv[6] = {&Ar, &Ai, &Br, &Bi, &Cr, &Ci};
-    std::vector<double>* fm[3] = {&ref_.Am, &ref_.Bm, &ref_.Cm};
-    std::vector<int32_t>* fe[3] = {&ref_.Ae, &ref_.Be, &ref_.Ce};
-    for (int k = 0; k < 6; k++) {
-      long e = 0;
-      const double m = hv[k]->get_d_2exp(&e);
-      (*fm[k / 2])[2 * i + k % 2] = m;
-      (*fe[k / 2])[2 * i + k % 2] = m == 0.0 ? kFxZeroExp : (int32_t)e;
-    }
-  }
+  if (!orbitTables(len, true, ref_)) series_chain(X.data(), len, hp_limbs_for_bits(hp_default_bits()), ref_);
 }
 
 // the device's work on X: r's orbit in doubles, and with `series` its coefficients

@@ -20,10 +20,10 @@
 //
 // A chunk's first value comes by another order of operations than the host's chain, so
 // its last bits differ (the first chunk's do not).  What is kept of a value is its
-// truncation to 53 bits: another order can change it only where the value's next bits
-// are all ones or all zeros as far down as errors reach.  k_emit looks for such a value
-// (64 L - 48 bits down, less what cancellation between the parts takes), and where one
-// is found the host makes the tables.
+// truncation to 53 bits, which the difference changes only where it reaches the value's
+// neighbours.  The kernels give each value's distance to those and each chunk's step at
+// its start, orbit_tables_hold() (orbit_steps.hpp) bounds the difference along the
+// orbit from them, and where the bound does not do the host makes the tables.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -33,20 +33,11 @@
 
 #include "coords.hpp"
 #include "orbit.hpp"
+#include "orbit_steps.hpp"
 
 namespace nm {
 
 namespace {
-
-template <int ML>
-__device__ __forceinline__ hpd<ML> small(int v) {  // 0 or 1
-  hpd<ML> r;
-  r.sign = v;
-  r.exp = v;
-  for (int i = 0; i < ML; i++) r.m[i] = 0;
-  if (v) r.m[ML - 1] = 1ull << 63;
-  return r;
-}
 
 // the value of the lane's neighbour (lanes 2 k and 2 k + 1)
 __device__ __forceinline__ uint32_t beside(uint32_t v) {
@@ -85,7 +76,7 @@ __global__ __launch_bounds__(64) void k_sweep(Sweep<ML> w) {
   const bool live = (t >> 1) < chunks, product = blockIdx.y != 0;
   const int q = live ? t >> 1 : chunks - 1;
   const int e0 = q * w.chunk, e1 = min(w.n, e0 + w.chunk);  // chunks * chunk < n + chunk: in 32 bits
-  hpd<ML> v = small<ML>(part == 0 ? (product ? 1 : w.first) : 0);
+  hpd<ML> v = hpd_small<ML>(part == 0 ? (product ? 1 : w.first) : 0);
   if (w.start && !product) v = w.start[2 * q + part];
   hpd<ML> fr = w.factor[2 * e0], fi = w.factor[2 * e0 + 1];
   for (int e = e0; e < e1; e++) {
@@ -93,13 +84,9 @@ __global__ __launch_bounds__(64) void k_sweep(Sweep<ML> w) {
     const hpd<ML> nr = w.factor[2 * nx], ni = w.factor[2 * nx + 1];  // the next step's
     if (w.before && live && !product) w.before[2 * e + part] = v;
     const hpd<ML> o = beside(v);
-    hpd<ML> s = hpd_add(hpd_mul(fr, v, w.L), hpd_mul(fi, o, w.L), part == 0 ? -1 : 1, w.L);
-    if (w.twice && s.sign) s.exp++;
-    if (!product) {
-      if (w.one && part == 0) s = hpd_add(s, small<ML>(1), 1, w.L);
-      if (w.u1) s = hpd_add(s, w.u1[2 * e + part], 1, w.L);
-      if (w.u2) s = hpd_add(s, w.u2[2 * e + part], 1, w.L);
-    }
+    const size_t u = 2 * (size_t)e + part;
+    const hpd<ML> s = sweep_part(part, fr, fi, v, o, w.twice != 0, !product && w.one,
+                                 product || !w.u1 ? nullptr : w.u1 + u, product || !w.u2 ? nullptr : w.u2 + u, w.L);
     v = s;
     if (w.after && live && !product) w.after[2 * e + part] = v;
     fr = nr;
@@ -110,24 +97,14 @@ __global__ __launch_bounds__(64) void k_sweep(Sweep<ML> w) {
   else if (w.end) w.end[2 * q + part] = v;
 }
 
-// the terms of B (bs null: A_i^2) or C (2 A_i B_i) at i = 1 .. n, in the order the
-// recurrence adds them: real parts a_r b_r and -a_i b_i, imaginary a_r b_i and a_i b_r
-// (for A^2 the one product doubled)
+// the terms of B (bs null) or C at i = 1 .. n (terms_part)
 template <int ML>
 __global__ __launch_bounds__(64) void k_terms(const hpd<ML>* as, const hpd<ML>* bs, int n, int L, hpd<ML>* u1,
                                               hpd<ML>* u2) {
   const int t = blockIdx.x * 64 + threadIdx.x, part = t & 1, e = t >> 1;
   if (e >= n) return;
-  const hpd<ML>*a = as + 2 * (e + 1), *b = bs ? bs + 2 * (e + 1) : a;
-  hpd<ML> p = hpd_mul(a[0], b[part], L), s = hpd_mul(a[1], b[1 - part], L);
-  if (part == 0) s.sign = -s.sign;
-  if (bs) {
-    if (p.sign) p.exp++;
-    if (s.sign) s.exp++;
-  } else if (part == 1) {
-    if (p.sign) p.exp++;
-    s = small<ML>(0);
-  }
+  hpd<ML> p, s;
+  terms_part(part, as + 2 * (e + 1), bs ? bs + 2 * (e + 1) : (const hpd<ML>*)nullptr, L, p, s);
   u1[t] = p;
   u2[t] = s;
 }
@@ -144,46 +121,30 @@ __global__ __launch_bounds__(64) void k_orbit(const hpd<ML>* x, int len, int L, 
   if (t < 2 * len) Xlo[t] = hpd_nearest(hpd_add(v, hpd_from_d<ML>(d), -1, L), L);
 }
 
-// whether an error 48 bits above the last one, of the larger part's size, could reach
-// the 53 bits kept: the bits between are all ones or all zeros
+// Y_0 .. Y_{len - 1} truncated to doubles (mpf_get_d), as mantissa and exponent, and
+// with the bits that the truncation hangs on; for chunks 1 .. n1 - 1 the exponents of
+// the step from the previous chunk's end to their start
 template <int ML>
-__device__ bool hangs(const hpd<ML>& v, const hpd<ML>& o, int L) {
-  if (v.sign == 0) return false;
-  int64_t guard = 48;
-  if (o.sign && o.exp > v.exp) guard += o.exp - v.exp;
-  const int64_t bits = 64 * (int64_t)L - guard;  // bits 54 .. bits from the top decide
-  if (bits < 53 + 40) return true;
-  uint64_t any = 0, all = ~0ull;
-  for (int i = 0; i < ML; i++) {
-    const int64_t top = 64 * (int64_t)(ML - 1 - i);  // bits above limb i
-    uint64_t mask = top == 0 ? (1ull << 11) - 1 : ~0ull;
-    if (top >= bits) mask = 0;
-    else if (top + 64 > bits) mask &= ~0ull << (top + 64 - bits);
-    any |= v.m[i] & mask;
-    all &= v.m[i] | ~mask;
-  }
-  return any == 0 || all == ~0ull;
-}
-
-// Y_0 .. Y_{len - 1} truncated to doubles (mpf_get_d) and as mantissa and exponent
-template <int ML>
-__global__ __launch_bounds__(64) void k_emit(const hpd<ML>* y, int len, int L, int same, double* d, double* m,
-                                             int32_t* e, int* doubt) {
+__global__ __launch_bounds__(64) void k_emit(const hpd<ML>* y, int len, int L, const hpd<ML>* starts,
+                                             const hpd<ML>* ends, int n1, double* d, double* m, int32_t* e,
+                                             uint16_t* run, int32_t* gap) {
   const int t = blockIdx.x * 64 + threadIdx.x;
+  if (t < 2 * (n1 - 1)) {
+    const hpd<ML> g = hpd_add(starts[t + 2], ends[t], -1, L);
+    gap[t] = g.sign ? (int32_t)g.exp : kFxZeroExp;
+  }
   if (t >= 2 * len) return;
   const hpd<ML> v = y[t];
   d[t] = hpd_get_d(v);
   const double f = v.sign * ldexp((double)(v.m[ML - 1] >> 11), -53);
   m[t] = v.sign ? f : 0.0;
   e[t] = v.sign ? (int32_t)v.exp : kFxZeroExp;
-  if ((t >> 1) >= same && hangs(v, y[t ^ 1], L)) *doubt = 1;
+  run[t] = hpd_run(v, L);
 }
 
-// Y_0, and the doubt cleared
 template <int ML>
-__global__ __launch_bounds__(64) void k_first(hpd<ML>* y, int first, int* doubt) {
-  if (threadIdx.x < 2) y[threadIdx.x] = small<ML>(threadIdx.x == 0 ? first : 0);
-  if (threadIdx.x == 0 && doubt) *doubt = 0;
+__global__ __launch_bounds__(64) void k_first(hpd<ML>* y, int first) {
+  if (threadIdx.x < 2) y[threadIdx.x] = hpd_small<ML>(threadIdx.x == 0 ? first : 0);
 }
 
 template <int ML>
@@ -229,7 +190,8 @@ bool OrbitTables::go(void* stream, const HpVal* x, int len, int L, bool series, 
   };
   const size_t count = 2 * (size_t)len;
   const size_t ox = place((count + 2) * sizeof(V)), oz = place((count + 4) * 8), ol = place(count * 8);
-  size_t oy[3], od[3], om[3], oe[3], ou[2], os[6], of = 0;
+  size_t oy[3], od[3], om[3], oe[3], ou[2], os[6], orun = 0, ogap = 0;
+  const size_t gaps = 2 * (size_t)(n1 - 1);  // of each series
   if (series) {
     for (int k = 0; k < 3; k++) {
       oy[k] = place(count * sizeof(V));
@@ -239,7 +201,8 @@ bool OrbitTables::go(void* stream, const HpVal* x, int len, int L, bool series, 
     }
     for (size_t& o : ou) o = place(count * sizeof(V));
     for (int k = 0; k < 6; k++) os[k] = place(2 * (size_t)(k < 3 ? n1 : n2) * sizeof(V));  // products, ends, starts
-    of = place(4);
+    orun = place(3 * count * 2);
+    ogap = place(3 * gaps * 4);
   }
   if (!room(off)) return false;
   V* dx = (V*)(buf_ + ox);
@@ -252,7 +215,6 @@ bool OrbitTables::go(void* stream, const HpVal* x, int len, int L, bool series, 
     V *P1 = (V*)(buf_ + os[0]), *E1 = (V*)(buf_ + os[1]), *S1 = (V*)(buf_ + os[2]);
     V *P2 = (V*)(buf_ + os[3]), *E2 = (V*)(buf_ + os[4]), *S2 = (V*)(buf_ + os[5]);
     V *u1 = (V*)(buf_ + ou[0]), *u2 = (V*)(buf_ + ou[1]);
-    int* doubt = (int*)(buf_ + of);
     const unsigned blocks = (unsigned)((count + 63) / 64);
     for (int k = 0; k < 3; k++) {
       V* y = (V*)(buf_ + oy[k]);
@@ -266,10 +228,11 @@ bool OrbitTables::go(void* stream, const HpVal* x, int len, int L, bool series, 
       sweep<ML>(s, {P1, E1, nullptr, 0, 0, n1, c, L, nullptr, 0, E2, nullptr, nullptr, p2});
       sweep<ML>(s, {P2, E2, nullptr, 0, 0, n2, n2, L, nullptr, first, nullptr, S2, nullptr, nullptr});
       sweep<ML>(s, {P1, E1, nullptr, 0, 0, n1, c, L, S2, 0, nullptr, S1, nullptr, nullptr});
-      sweep<ML>(s, {dx, t1, t2, 1, one, n, c, L, S1, 0, nullptr, nullptr, y + 2, nullptr});
-      hipLaunchKernelGGL(k_first<ML>, dim3(1), dim3(64), 0, s, y, first, k == 0 ? doubt : (int*)nullptr);
-      hipLaunchKernelGGL(k_emit<ML>, dim3(blocks), dim3(64), 0, s, (const V*)y, len, L, c + 1, (double*)(buf_ + od[k]),
-                         (double*)(buf_ + om[k]), (int32_t*)(buf_ + oe[k]), doubt);
+      sweep<ML>(s, {dx, t1, t2, 1, one, n, c, L, S1, 0, E1, nullptr, y + 2, nullptr});
+      hipLaunchKernelGGL(k_first<ML>, dim3(1), dim3(64), 0, s, y, first);
+      hipLaunchKernelGGL(k_emit<ML>, dim3(blocks), dim3(64), 0, s, (const V*)y, len, L, (const V*)S1, (const V*)E1, n1,
+                         (double*)(buf_ + od[k]), (double*)(buf_ + om[k]), (int32_t*)(buf_ + oe[k]),
+                         (uint16_t*)(buf_ + orun) + k * count, (int32_t*)(buf_ + ogap) + k * gaps);
     }
   }
   ok = ok && hipGetLastError() == hipSuccess;
@@ -279,7 +242,8 @@ bool OrbitTables::go(void* stream, const HpVal* x, int len, int L, bool series, 
   };
   fetch(r.Zd, oz, count + 4);
   fetch(r.Xlo, ol, count);
-  int doubt = 0;
+  std::vector<uint16_t> run;
+  std::vector<int32_t> gap;
   if (series) {
     std::vector<double>*fd[3] = {&r.A, &r.B, &r.C}, *fm[3] = {&r.Am, &r.Bm, &r.Cm};
     std::vector<int32_t>* fe[3] = {&r.Ae, &r.Be, &r.Ce};
@@ -288,12 +252,18 @@ bool OrbitTables::go(void* stream, const HpVal* x, int len, int L, bool series, 
       fetch(*fm[k], om[k], count);
       fetch(*fe[k], oe[k], count);
     }
-    ok = ok && hipMemcpyAsync(&doubt, buf_ + of, 4, hipMemcpyDeviceToHost, s) == hipSuccess;
+    fetch(run, orun, 3 * count);
+    fetch(gap, ogap, 3 * gaps);
   }
   ok = hipStreamSynchronize(s) == hipSuccess && ok;
   if (!ok) (void)hipGetLastError();
   if (bytes_ > kKeep) release();
-  return ok && !doubt;
+  if (!ok || !series) return ok;
+  bool real = true;
+  for (size_t k = 1; k < count && real; k += 2) real = x[k].sign == 0;
+  return orbit_tables_hold(r.Zd.data(), len, L, c, real, {r.Ae.data(), r.Be.data(), r.Ce.data()},
+                           {run.data(), run.data() + count, run.data() + 2 * count},
+                           {gap.data(), gap.data() + gaps, gap.data() + 2 * gaps});
 }
 
 bool OrbitTables::make(void* stream, const HpVal* x, int len, int L, bool series, SaReferenceHost& r) {

@@ -15,7 +15,8 @@ class OrbitTables {
   // Zd and Xlo of r, and with `series` A .. Ce, for the orbit x (2 (len + 1) values of
   // L limbs, real and imaginary parts in turn).  False where the host has to make
   // them (r may then be partly filled): more than kMaxLimbs limbs, an orbit shorter
-  // than kMinLen, no memory, or a coefficient that hangs on its last bits.
+  // than kMinLen, no memory, or coefficients whose doubles the order of operations
+  // could change (orbit_tables_hold).
   bool make(void* stream, const HpVal* x, int len, int L, bool series, SaReferenceHost& r);
   ~OrbitTables();
 
