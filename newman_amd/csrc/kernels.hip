@@ -2457,8 +2457,10 @@ class EngineImpl : public Engine {
   void* d_img = nullptr; size_t n_img_bytes = 0;
   void* d_keys = nullptr; size_t n_keys_bytes = 0;   // video: two keyframes and the schedule
   void* d_vframes = nullptr; size_t n_vframes_bytes = 0;
-  uint64_t tag_ = 0;                                 // render count (render_tag)
-  const EscapeValue* last_result = nullptr;          // the last render's row-major grids
+  // count of passes begun (render_tag): what an earlier tag named is gone from the moment
+  // its buffer is written to or freed, whether or not the render then succeeds
+  uint64_t tag_ = 0;
+  const EscapeValue* last_result = nullptr;          // the last render's row-major grids (null: none whole)
   uint64_t last_nout = 0;
   void* d_emit = nullptr; size_t n_emit_bytes = 0;  // row-major grids of a tiled sample order
   void* d_ttabs = nullptr; size_t n_ttabs_bytes = 0;  // tile search: epsilon tables
@@ -2517,6 +2519,17 @@ class EngineImpl : public Engine {
     NM_HIP(hipMalloc(p, n));
     *have = n;
     return NM_OK;
+  }
+
+  void drop_result() {
+    tag_++;
+    last_result = nullptr;
+    last_nout = 0;
+  }
+  // grow for a buffer that holds results
+  int grow_result(void** p, size_t* have, size_t need) {
+    if (need > *have || !*p) drop_result();
+    return grow(p, have, need);
   }
 
   bool orbit_tables(const HpVal* x, int len, int L, bool series, SaReferenceHost& r) override {
@@ -2656,12 +2669,16 @@ class EngineImpl : public Engine {
     return NM_OK;
   }
 
+  // sample ids and the plain iterate kernel's chunk positions (ChunkMap) stay below 2^32
+  static bool in_range(uint64_t total) { return total > 0 && total < 0xFFFFF000ull; }
+  // the series kernels' block sizes (an FP32X mantissa is renormalised at block ends)
+  static bool series_block(int K, bool fx) { return K == 8 || K == 12 || K == 16 || K == 32 || (K == 64 && !fx); }
+
   // buffers and the common kernel arguments for `total` samples
   int prepare_common(Common& c, uint64_t total, const RenderOpts& opt) {
-    // sample ids and the plain iterate kernel's chunk positions (ChunkMap) stay below 2^32
-    if (total == 0 || total >= 0xFFFFF000ull) return NM_ERR_RANGE;
+    if (!in_range(total)) return NM_ERR_RANGE;
     int st;
-    if ((st = grow(&d_out, &n_out_bytes, total * sizeof(EscapeValue)))) return st;
+    if ((st = grow_result(&d_out, &n_out_bytes, total * sizeof(EscapeValue)))) return st;
     if ((st = grow(&d_hand, &n_hand_bytes, (uint64_t)hand_words((uint32_t)total) * 8))) return st;
     if ((st = grow(&d_state, &n_state_bytes, total * sizeof(double4)))) return st;
     if ((st = grow(&d_state_i, &n_state_i_bytes, total * sizeof(int2)))) return st;
@@ -2707,6 +2724,7 @@ class EngineImpl : public Engine {
   template <class Args, class StartFn, class IterFn>
   int run(Args& args, StartFn start, IterFn iter, int waves, const RenderOpts& opt, RenderStats* stats,
           uint64_t nout, EscapeValue* host_out, EscapeValue* emit_to) {
+    drop_result();  // the passes write over it
     const int repeats = std::max(1, opt.repeats);
     const bool use_graph = opt.graph && repeats > 1, timed = opt.timed || use_graph;
     int st = NM_OK;
@@ -2762,7 +2780,6 @@ class EngineImpl : public Engine {
     if (st) return st;
     if (ce != hipSuccess) return fail("counters and results", ce);
     if (se != hipSuccess) return fail("hipStreamSynchronize", se);
-    tag_++;
     last_result = result;
     last_nout = nout;
     double ms[4] = {};
@@ -2828,6 +2845,10 @@ class EngineImpl : public Engine {
       nout += (uint64_t)f->nr * f->nc;
       df.push_back(d);
     }
+    // a call that is refused leaves the last render's result and tables as they are
+    if (!in_range(total)) return NM_ERR_RANGE;
+    const int K = opt.block_k > 0 ? opt.block_k : 64;
+    if (K != 8 && K != 16 && K != 32 && K != 64) return NM_ERR_ARG;
     int st;
     const void *pf = d_frames, *pt = d_tabs;
     if ((st = grow(&d_frames, &n_frames_bytes, df.size() * sizeof(DevFrame)))) return st;
@@ -2838,7 +2859,7 @@ class EngineImpl : public Engine {
     if ((st = prepare_common(a.c, total, opt))) return st;
     EscapeValue* emit_to = nullptr;
     if (opt.tile) {
-      if ((st = grow(&d_emit, &n_emit_bytes, nout * sizeof(EscapeValue)))) return st;
+      if ((st = grow_result(&d_emit, &n_emit_bytes, nout * sizeof(EscapeValue)))) return st;
       emit_to = (EscapeValue*)d_emit;
     }
     a.c.nframes = (int)df.size();
@@ -2859,7 +2880,6 @@ class EngineImpl : public Engine {
     a.crelo = t + ncol;
     a.cim = t + 2 * ncol;
     a.cimlo = t + 2 * ncol + nrow;
-    const int K = opt.block_k > 0 ? opt.block_k : 64;
     // 4 persistent waves per SIMD: the iterate kernel's tail is shorter than
     // with 8 (512 frames of 640x480 at N 1024: 0.93 against 0.95 ms; 2 waves
     // hide too little latency, 1.03 ms)
@@ -2897,8 +2917,7 @@ class EngineImpl : public Engine {
       case 8: NM_PLAIN(8);
       case 16: NM_PLAIN(16);
       case 32: NM_PLAIN(32);
-      case 64: NM_PLAIN(64);
-      default: return NM_ERR_ARG;
+      default: NM_PLAIN(64);
     }
 #undef NM_PLAIN
   }
@@ -2935,6 +2954,11 @@ class EngineImpl : public Engine {
       nout += (uint64_t)f->nr * f->nc;
       df.push_back(d);
     }
+    // a call that is refused leaves the last render's result and tables as they are
+    if (!in_range(total)) return NM_ERR_RANGE;
+    const bool fx = opt.delta_mode == DELTA_FP32X;
+    if (opt.block_k > 0 && !series_block(opt.block_k, fx)) return NM_ERR_ARG;
+    if (chunk_run_shift(opt.chunk_run) < 0 || (opt.tile_ua && opt.skip_T < 8)) return NM_ERR_ARG;
     int st;
     const void *pf = d_frames, *pt = d_tabs, *pm = d_mask;
     if ((st = grow(&d_frames, &n_frames_bytes, df.size() * sizeof(DevFrame)))) return st;
@@ -2945,7 +2969,7 @@ class EngineImpl : public Engine {
     if ((st = prepare_common(a.c, total, opt))) return st;
     EscapeValue* emit_to = nullptr;
     if (opt.tile) {
-      if ((st = grow(&d_emit, &n_emit_bytes, nout * sizeof(EscapeValue)))) return st;
+      if ((st = grow_result(&d_emit, &n_emit_bytes, nout * sizeof(EscapeValue)))) return st;
       emit_to = (EscapeValue*)d_emit;
     }
     a.c.nframes = (int)df.size();
@@ -2993,11 +3017,8 @@ class EngineImpl : public Engine {
     // (the 1e-100 and 1e-200 views: FP64 iterate kernel 15% and 8% faster, FP32X
     // 8% and 11%; their long samples cluster), 64 consecutive samples otherwise
     // (the 1e-30 and 1e-40 views: 8% and 0-6% slower with runs of 4)
-    const int run_shift = chunk_run_shift(opt.chunk_run == 0 && a.fxs ? 4 : opt.chunk_run);
-    if (run_shift < 0) return NM_ERR_ARG;
-    a.run_shift = (uint32_t)run_shift;
+    a.run_shift = (uint32_t)chunk_run_shift(opt.chunk_run == 0 && a.fxs ? 4 : opt.chunk_run);
     if (opt.tile_ua) {
-      if (opt.skip_T < 8) return NM_ERR_ARG;
       const uint32_t T = (uint32_t)opt.skip_T, ntc = (frames[0]->nc + T - 1) / T, ntr = (frames[0]->nr + T - 1) / T;
       const size_t nt = (size_t)ntc * ntr * frames.size();
       if ((st = grow(&d_tile_ua, &n_tile_ua_bytes, nt * 4))) return st;
@@ -3007,7 +3028,6 @@ class EngineImpl : public Engine {
       a.skip_ntc = ntc;
       a.skip_tpf = ntc * ntr;
     }
-    const bool fx = opt.delta_mode == DELTA_FP32X;
     // FP64 blocks hold one orbit entry per lane whatever K is.  After the coherent
     // phase most samples of the double-series views have some 50 steps left, where
     // a lane that is done waits half a block: 32 (iterate kernel 2.03 -> 1.96 ms on
@@ -3051,10 +3071,7 @@ class EngineImpl : public Engine {
       case 12: return fx ? go(k_series_iterate<12, true>) : go(k_series_iterate<12, false>);
       case 16: return fx ? go(k_series_iterate<16, true>) : go(k_series_iterate<16, false>);
       case 32: return fx ? go(k_series_iterate<32, true>) : go(k_series_iterate<32, false>);
-      case 64:  // FP64 only: an FP32X mantissa is renormalised at block ends
-        if (fx) return NM_ERR_ARG;
-        return go(k_series_iterate<64, false>);
-      default: return NM_ERR_ARG;
+      default: return go(k_series_iterate<64, false>);  // 64: FP64 only (series_block)
     }
   }
 
