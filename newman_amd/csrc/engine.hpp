@@ -151,6 +151,23 @@ struct RenderOpts {
                            // on the device and skips the upload when it repeats (0 = always upload)
 };
 
+// Whose frame records and coordinate tables the device holds: a frame set's serial and
+// sample order, from the moment the last of them was sent without an error until the
+// first of another set's is.
+class TableKey {
+ public:
+  bool holds(uint64_t serial, int tile) const { return serial != 0 && serial == serial_ && tile == tile_; }
+  void writing() { serial_ = 0; }
+  void written(uint64_t serial, int tile) {
+    serial_ = serial;
+    tile_ = tile;
+  }
+
+ private:
+  uint64_t serial_ = 0;
+  int tile_ = -1;
+};
+
 struct RenderStats {
   uint64_t samples = 0;
   uint64_t n_cardioid = 0;   // samples resolved by the cardioid/bulb test

@@ -431,6 +431,22 @@ long long nm_tree_check(int len, unsigned seed) {
   return bad;
 }
 
+// The engine's record of whose tables are on the device: a set's are its own after
+// they were written whole, and nobody's from the first write of another set's on, also
+// where those then fail.  Returns the number of wrong answers.
+long long nm_table_key_check() {
+  nm::TableKey k;
+  long long bad = k.holds(0, -1) + k.holds(0, 0) + k.holds(5, 0);
+  k.writing();
+  k.written(5, 32);
+  bad += !k.holds(5, 32) + k.holds(5, 0) + k.holds(6, 32) + k.holds(0, 32);
+  k.writing();  // set 6's records are under way, and fail
+  bad += k.holds(5, 32) + k.holds(6, 32) + k.holds(0, 32);
+  k.writing();
+  k.written(0, 32);  // a set without a serial
+  return bad + k.holds(0, 32) + k.holds(5, 32);
+}
+
 // The device's coordinate entries against hpfloat.cpp: `n` cases from a seed, with
 // random mantissas (some sparse), exponents, signs and offsets, every combination of
 // precisions that `ML` limbs hold; the truncated coordinate, its remainder and the

@@ -2621,18 +2621,23 @@ class EngineImpl : public Engine {
     return NM_OK;
   }
 
-  // frame tables on the device belong to (set serial, sample order); a render
-  // with the same pair and unmoved buffers reuses them
-  uint64_t tab_serial = 0;
-  int tab_tile = -1;
+  TableKey tab_key;       // a render with the same set reuses the tables
   double tab_emax = 0.0;  // at least |epsilon| of every sample of the tables on the device (series path)
-  bool tables_stale(const RenderOpts& opt, bool same_buffers) const {
-    return opt.set_serial == 0 || opt.set_serial != tab_serial || opt.tile != tab_tile || !same_buffers;
+
+  // grow for a buffer of those tables
+  int grow_tables(void** p, size_t* have, size_t need) {
+    if (need > *have || !*p) tab_key.writing();
+    return grow(p, have, need);
   }
-  void tables_uploaded(const RenderOpts& opt) {
-    tab_serial = opt.set_serial;
-    tab_tile = opt.tile;
-  }
+  // Waits for the stream where the copies of an upload out of local vectors are not
+  // known to be over: declared after them, it runs before they end.
+  struct UploadEnd {
+    hipStream_t stream;
+    bool pending;
+    ~UploadEnd() {
+      if (pending) (void)hipStreamSynchronize(stream);
+    }
+  };
 
   // the frame records and coordinate tables of a frame set, on the device: a single
   // frame's come with the kernel's arguments, several frames' through the pinned
@@ -2850,10 +2855,9 @@ class EngineImpl : public Engine {
     const int K = opt.block_k > 0 ? opt.block_k : 64;
     if (K != 8 && K != 16 && K != 32 && K != 64) return NM_ERR_ARG;
     int st;
-    const void *pf = d_frames, *pt = d_tabs;
-    if ((st = grow(&d_frames, &n_frames_bytes, df.size() * sizeof(DevFrame)))) return st;
-    if ((st = grow(&d_tabs, &n_tabs_bytes, (2 * ncol + 2 * nrow) * sizeof(double)))) return st;
-    const bool upload = tables_stale(opt, pf == d_frames && pt == d_tabs);
+    if ((st = grow_tables(&d_frames, &n_frames_bytes, df.size() * sizeof(DevFrame)))) return st;
+    if ((st = grow_tables(&d_tabs, &n_tabs_bytes, (2 * ncol + 2 * nrow) * sizeof(double)))) return st;
+    const bool upload = !tab_key.holds(opt.set_serial, opt.tile);
     PlainArgs a;
     a.direct = nullptr;
     if ((st = prepare_common(a.c, total, opt))) return st;
@@ -2868,11 +2872,12 @@ class EngineImpl : public Engine {
     double* t = (double*)d_tabs;
     if (upload) {
       // made again only when the device copy is stale: a repeated frame set reuses it
+      tab_key.writing();
       std::vector<FrameHp> hp;
       for (auto* f : frames) hp.push_back(f->hp);
       if ((st = make_tables(df, hp, frames[0]->nr, frames[0]->nc, false, {t, t + ncol, t + 2 * ncol, t + 2 * ncol + nrow})))
         return st;
-      tables_uploaded(opt);
+      tab_key.written(opt.set_serial, opt.tile);
     }
     a.pre_iter = opt.pre_iter > 0 ? opt.pre_iter : kPreIterDefault;
     a.k_start = (std::min(a.pre_iter, opt.N) + 3) / 4 * 4;
@@ -2960,11 +2965,10 @@ class EngineImpl : public Engine {
     if (opt.block_k > 0 && !series_block(opt.block_k, fx)) return NM_ERR_ARG;
     if (chunk_run_shift(opt.chunk_run) < 0 || (opt.tile_ua && opt.skip_T < 8)) return NM_ERR_ARG;
     int st;
-    const void *pf = d_frames, *pt = d_tabs, *pm = d_mask;
-    if ((st = grow(&d_frames, &n_frames_bytes, df.size() * sizeof(DevFrame)))) return st;
-    if ((st = grow(&d_tabs, &n_tabs_bytes, (ncol + nrow) * sizeof(double)))) return st;
-    if ((st = grow(&d_mask, &n_mask_bytes, std::max<size_t>(nmask, 1) * 4))) return st;
-    const bool upload = tables_stale(opt, pf == d_frames && pt == d_tabs && pm == d_mask);
+    if ((st = grow_tables(&d_frames, &n_frames_bytes, df.size() * sizeof(DevFrame)))) return st;
+    if ((st = grow_tables(&d_tabs, &n_tabs_bytes, (ncol + nrow) * sizeof(double)))) return st;
+    if ((st = grow_tables(&d_mask, &n_mask_bytes, std::max<size_t>(nmask, 1) * 4))) return st;
+    const bool upload = !tab_key.holds(opt.set_serial, opt.tile);
     SeriesArgs a;
     if ((st = prepare_common(a.c, total, opt))) return st;
     EscapeValue* emit_to = nullptr;
@@ -2981,6 +2985,8 @@ class EngineImpl : public Engine {
       std::vector<uint32_t> mask;
       std::vector<double> er, ei;
       std::vector<FrameHp> hp;
+      UploadEnd end{stream, false};
+      tab_key.writing();
       double emax = 0.0;
       for (auto* f : frames) {
         if (f->card_mode == CARD_MASK) mask.insert(mask.end(), f->mask.begin(), f->mask.end());
@@ -2993,6 +2999,7 @@ class EngineImpl : public Engine {
           hp.push_back(f->hp);
         }
       }
+      end.pending = !mask.empty() || hp.empty();
       if (!mask.empty())
         NM_HIP(hipMemcpyAsync(d_mask, mask.data(), mask.size() * 4, hipMemcpyHostToDevice, stream));
       if (!hp.empty()) {
@@ -3003,9 +3010,10 @@ class EngineImpl : public Engine {
         NM_HIP(hipMemcpyAsync(t, er.data(), ncol * 8, hipMemcpyHostToDevice, stream));
         NM_HIP(hipMemcpyAsync(t + ncol, ei.data(), nrow * 8, hipMemcpyHostToDevice, stream));
       }
-      if (!mask.empty() || hp.empty()) NM_HIP(hipStreamSynchronize(stream));  // the host vectors end with this scope
+      if (end.pending) NM_HIP(hipStreamSynchronize(stream));
+      end.pending = false;
       tab_emax = emax * (1.0 + 0x1p-40);
-      tables_uploaded(opt);
+      tab_key.written(opt.set_serial, opt.tile);
     }
     a.epsre = t;
     a.epsim = t + ncol;
