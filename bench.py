@@ -637,7 +637,8 @@ def measure(config, args, block_k=None, waves=None):
         tuned = {"best": best, "sweep": table, "seconds": time.perf_counter() - t0}
         print("# autotune: %s (%.1f s)" % (best, tuned["seconds"]), file=sys.stderr, flush=True)
     elif args.tune and config == args.config:
-        best, rows = tune(step, [8, 16, 32, 64] if config == "c1" else [12, 16, 32, 64], [2, 4, 6, 8])
+        best, rows = tune(step, [8, 16, 32, 64] if config == "c1" else [12, 16, 32, 64],
+                          [2, 4, 6, 8] if config == "c1" else [1, 2, 3, 4])
         k, w = best[0], best[1]
         tuned = {"best": {"block_k": k, "waves_per_simd": w, "chunk_run": args.chunk_run, "ms": best[2]},
                  "sweep": [{"block_k": a, "waves_per_simd": b, "ms": c} for a, b, c in rows]}

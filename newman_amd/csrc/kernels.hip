@@ -89,7 +89,8 @@ constexpr int kLdsTail = 512, kLdsHead = 7648;
 // a tail of 1024, 4.83 of 2048), the 1e-30, 1e-40 and 1e-200 views the same.  More
 // waves over smaller windows: 6 per SIMD 1.88 against 2.00 ms at 1e-30, but 5.98 ms
 // at 1e-100.
-constexpr int kSeriesIterThreads = 1024;
+constexpr int kSeriesWaves = 4;  // per SIMD: all that such a workgroup holds
+constexpr int kSeriesIterThreads = 256 * kSeriesWaves;
 static_assert(kLdsTail >= 64 && kLdsHead >= 64, "a block of up to 64 steps reads inside one window");
 constexpr int kPartSlots = 6144;        // per-workgroup partial counter slots
 
@@ -3050,11 +3051,13 @@ class EngineImpl : public Engine {
     // 1600x900 of the 1e-30 view, 0.112 / 0.111 / 0.119 ms on 700x500 at 1e-25
     a.fx_runs = fx ? std::max(1, (a.fxs ? 64 : 32) / K) : 1;
     // 4 persistent waves per SIMD: the workgroup whose queues and windows fill a CU's
-    // LDS (more would wait for it to end; fewer hide too little latency:
+    // LDS; fewer hide too little latency:
     // 2 waves 2.8-3.0 against 2.0 ms on the 1e-30 view, 1.29 against 0.91 ms on 16
-    // frames of the 1e-40 video).  FP32X ran 8 with smaller windows: 1.18 -> 1.07 ms
-    // on the 1279x719 frame of the 1e-200 view
-    const int waves = opt.waves_per_simd > 0 ? opt.waves_per_simd : 4;
+    // frames of the 1e-40 video.  FP32X ran 8 with smaller windows: 1.18 -> 1.07 ms
+    // on the 1279x719 frame of the 1e-200 view.  More waves would be workgroups that
+    // hold their first chunks back until a CU is free (8 and 16 waves 1.34 and 2.06 ms
+    // a pass of that frame against 0.88), so a larger setting is taken as 4
+    const int waves = opt.waves_per_simd > 0 ? std::min(opt.waves_per_simd, kSeriesWaves) : kSeriesWaves;
     if (stats) {
       stats->block_k = K;
       stats->waves_per_simd = waves;

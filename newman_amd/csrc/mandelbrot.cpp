@@ -1278,8 +1278,8 @@ int Mandelbrot::zoomVideoStep(const uint8_t* pal_rgb, int npal, int smooth, int 
 }
 
 // The project's launch autotuner.  Candidates: sample order (row-major, 32x32,
-// 64x64 and 128x128 tiles), persistent waves per SIMD (2, 4, 6, 8) and the block
-// size (16, 32, 64; FP32X deltas 8, 16, 32); then, on the series path, the
+// 64x64 and 128x128 tiles), persistent waves per SIMD (2, 4, 6, 8; on the series path,
+// whose workgroups fill a CU with 4, 1 to 4) and the block size (16, 32, 64; FP32X deltas 8, 16, 32); then, on the series path, the
 // fastest of those with the active list interleaved in runs of 4 (chunk_run).
 // Each candidate renders an evenly spaced subsample of at most 16 frames (so the
 // set's depth mix is kept) once untimed and once timed; the fastest total kernel
@@ -1291,7 +1291,7 @@ int Mandelbrot::autotuneFrames(const std::vector<std::string>& widths, std::vect
   const size_t n = set.hw ? set.h.size() : set.s.size();
   const size_t step = std::max<size_t>(1, (n + 15) / 16);
   const int tiles[4] = {0, 32, 64, 128};
-  const int waves[4] = {2, 4, 6, 8};
+  const int waves_hw[4] = {2, 4, 6, 8}, waves_sa[4] = {1, 2, 3, 4};
   // series blocks: FP64 up to 64 steps, FP32X (renormalised at block ends) up to 32
   const int ks_sa[3] = {16, 32, 64}, ks_fx[3] = {8, 16, 32}, ks_hw[3] = {16, 32, 64};
   const int nks = 3;
@@ -1302,7 +1302,7 @@ int Mandelbrot::autotuneFrames(const std::vector<std::string>& widths, std::vect
   const int* ks = set.hw ? ks_hw : delta_mode == DELTA_FP32X ? ks_fx : ks_sa;
   const uint64_t subset_serial = next_serial();  // the subsample's tables stay on the device
   for (int tile : tiles)
-    for (int w : waves)
+    for (int w : set.hw ? waves_hw : waves_sa)
       for (int ki = 0; ki < nks; ki++) {
         const int k = ks[ki];
         RenderOpts o;
