@@ -2642,19 +2642,28 @@ class EngineImpl : public Engine {
 
   // the frame records and coordinate tables of a frame set, on the device: a single
   // frame's come with the kernel's arguments, several frames' through the pinned
-  // staging buffer
-  int make_tables(const std::vector<DevFrame>& df, const std::vector<FrameHp>& hp, int nr, int nc, bool series,
+  // staging buffer, kStageFrames at a time (a FrameHp is 2 KB, so that the buffer and
+  // its copy on the device stay at 8.6 MB each however many frames a set has)
+  static constexpr size_t kStageFrames = 4096;
+  int make_tables(const std::vector<DevFrame>& df, const std::vector<const FrameHp*>& hp, int nr, int nc, bool series,
                   const CoordTables& t) {
-    const size_t nf = df.size(), fbytes = (nf * sizeof(DevFrame) + 255) & ~(size_t)255;
+    const size_t nf = df.size(), batch = std::min(nf, kStageFrames);
+    const size_t fbytes = (batch * sizeof(DevFrame) + 255) & ~(size_t)255, bytes = fbytes + batch * sizeof(FrameHp);
     int st, limbs = 0;
-    for (const FrameHp& h : hp) limbs = std::max(limbs, h.limbs);
-    const bool one = nf == 1;
-    if (!one) {
-      // a call refused after its tables (a block size the kernels do not have) has
-      // not waited for the copies out of the buffer
+    for (const FrameHp* h : hp) limbs = std::max(limbs, h->limbs);
+    if (nf == 1) {
+      hipLaunchKernelGGL(k_put_frame, dim3(1), dim3(1), 0, stream, (DevFrame*)d_frames, df[0]);
+      NM_HIP(hipGetLastError());
+      if (coords_launch((void*)stream, hp[0], nullptr, 1, nr, nc, limbs, series, t))
+        return fail("k_coords launch", hipGetLastError());
+      return NM_OK;
+    }
+    if ((st = grow(&d_hp, &n_hp_bytes, batch * sizeof(FrameHp)))) return st;
+    for (size_t f = 0; f < nf; f += batch) {
+      const size_t n = std::min(batch, nf - f);
+      // the copies out of the buffer, the last batch's or those of a call that failed
+      // after its tables, are over
       NM_HIP(hipStreamSynchronize(stream));
-      const size_t bytes = fbytes + nf * sizeof(FrameHp);
-      if ((st = grow(&d_hp, &n_hp_bytes, nf * sizeof(FrameHp)))) return st;
       if (bytes > n_stage_bytes) {
         if (h_stage) NM_HIP(hipHostFree(h_stage));
         h_stage = nullptr;
@@ -2662,16 +2671,21 @@ class EngineImpl : public Engine {
         NM_HIP(hipHostMalloc(&h_stage, bytes, hipHostMallocDefault));
         n_stage_bytes = bytes;
       }
-      std::memcpy(h_stage, df.data(), nf * sizeof(DevFrame));
-      std::memcpy((char*)h_stage + fbytes, hp.data(), nf * sizeof(FrameHp));
-      NM_HIP(hipMemcpyAsync(d_frames, h_stage, nf * sizeof(DevFrame), hipMemcpyHostToDevice, stream));
-      NM_HIP(hipMemcpyAsync(d_hp, (char*)h_stage + fbytes, nf * sizeof(FrameHp), hipMemcpyHostToDevice, stream));
-    } else {
-      hipLaunchKernelGGL(k_put_frame, dim3(1), dim3(1), 0, stream, (DevFrame*)d_frames, df[0]);
-      NM_HIP(hipGetLastError());
+      FrameHp* stage = (FrameHp*)((char*)h_stage + fbytes);
+      std::memcpy(h_stage, df.data() + f, n * sizeof(DevFrame));
+      for (size_t k = 0; k < n; k++) stage[k] = *hp[f + k];
+      NM_HIP(hipMemcpyAsync((DevFrame*)d_frames + f, h_stage, n * sizeof(DevFrame), hipMemcpyHostToDevice, stream));
+      NM_HIP(hipMemcpyAsync(d_hp, stage, n * sizeof(FrameHp), hipMemcpyHostToDevice, stream));
+      CoordTables u = t;
+      u.chi += f * nc;
+      u.rhi += f * nr;
+      if (!series) {
+        u.clo += f * nc;
+        u.rlo += f * nr;
+      }
+      if (coords_launch((void*)stream, nullptr, (const FrameHp*)d_hp, (int)n, nr, nc, limbs, series, u))
+        return fail("k_coords launch", hipGetLastError());
     }
-    if (coords_launch((void*)stream, one ? &hp[0] : nullptr, (const FrameHp*)d_hp, (int)nf, nr, nc, limbs, series, t))
-      return fail("k_coords launch", hipGetLastError());
     return NM_OK;
   }
 
@@ -2874,8 +2888,8 @@ class EngineImpl : public Engine {
     if (upload) {
       // made again only when the device copy is stale: a repeated frame set reuses it
       tab_key.writing();
-      std::vector<FrameHp> hp;
-      for (auto* f : frames) hp.push_back(f->hp);
+      std::vector<const FrameHp*> hp;
+      for (auto* f : frames) hp.push_back(&f->hp);
       if ((st = make_tables(df, hp, frames[0]->nr, frames[0]->nc, false, {t, t + ncol, t + 2 * ncol, t + 2 * ncol + nrow})))
         return st;
       tab_key.written(opt.set_serial, opt.tile);
@@ -2985,7 +2999,7 @@ class EngineImpl : public Engine {
       // made again only when the device copy is stale: a repeated frame set reuses it
       std::vector<uint32_t> mask;
       std::vector<double> er, ei;
-      std::vector<FrameHp> hp;
+      std::vector<const FrameHp*> hp;
       UploadEnd end{stream, false};
       tab_key.writing();
       double emax = 0.0;
@@ -2997,7 +3011,7 @@ class EngineImpl : public Engine {
           er.insert(er.end(), f->epsre.begin(), f->epsre.end());
           ei.insert(ei.end(), f->epsim.begin(), f->epsim.end());
         } else {
-          hp.push_back(f->hp);
+          hp.push_back(&f->hp);
         }
       }
       end.pending = !mask.empty() || hp.empty();
