@@ -202,6 +202,9 @@ int render_hw_noalloc(const HwFrameHost& f, int N, double bailout, EscapeValue* 
 class Engine {
  public:
   static int instance(Engine** out);
+  // the engine if a call has started it, else null: a call that can do its work on the
+  // host neither starts the device nor moves the thread's current one
+  static Engine* running();
   virtual ~Engine() = default;
   // Make `ref` the device reference; `serial` identifies it so an unchanged
   // reference is not uploaded again.

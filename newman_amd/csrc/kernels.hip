@@ -3306,6 +3306,10 @@ int Engine::instance(Engine** out) {
   return g_engine_status;
 }
 
+Engine* Engine::running() {
+  std::lock_guard<std::mutex> lk(g_engine_mu);
+  return g_engine;
+}
 
 // ================================================ allocation-free plain render
 // render_hw_noalloc: the plain path (getIterationsHW, mandelbrot.cpp:231-254) of

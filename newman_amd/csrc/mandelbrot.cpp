@@ -288,12 +288,13 @@ void Mandelbrot::computeSeries() {
   if (!orbitTables(len, true, ref_)) series_chain(X.data(), len, hp_limbs_for_bits(hp_default_bits()), ref_);
 }
 
-// the device's work on X: r's orbit in doubles, and with `series` its coefficients
+// the device's work on X: r's orbit in doubles, and with `series` its coefficients.
+// Only on a device that is in use: precomputeAt and the host's probe search start none.
 bool Mandelbrot::orbitTables(int len, bool series, SaReferenceHost& r) {
   static_assert(sizeof(HPComplex) == 2 * sizeof(HpVal), "X is pairs of HpVal");
-  Engine* eng = nullptr;
+  Engine* eng = Engine::running();
   r.len = len;
-  if (Engine::instance(&eng) == NM_OK && X.size() == (size_t)len + 1 &&
+  if (eng && X.size() == (size_t)len + 1 &&
       eng->orbit_tables((const HpVal*)X.data(), len, hp_limbs_for_bits(hp_default_bits()), series, r))
     return true;
   r = SaReferenceHost();
