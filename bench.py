@@ -174,7 +174,7 @@ def roofline(config, flop, s, fxs=False):
                            else ("k_plain_iterate<%d,%s,%s>" % (K, fma2, grouped)),
                            "ms": s["ms_iterate"], "steps": exec_iter},
                "start": {"name": "k_series_start" if series else "k_plain_start",
-                         "instance": ("k_series_start<%s>" % ("true" if fxs else "false")) if series
+                         "instance": ("k_series_start<%s,true>" % ("true" if fxs else "false")) if series
                          else ("k_plain_start<%s,%s>" % (fma2, grouped)),
                          "ms": s["ms_start"], "steps": s["executed_start"]}}
     for k in kernels.values():

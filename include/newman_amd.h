@@ -51,7 +51,7 @@ typedef struct nm_render_stats {
   uint64_t n_iterated;   /* handed to the iteration kernel */
   uint64_t executed;     /* iteration steps executed (start and iteration kernels) */
   uint64_t skipped;      /* sum of series-skip start indices of iterated samples */
-  uint64_t n_rebased;    /* blocks of block_k steps in which a sample rebased its delta */
+  uint64_t n_rebased;    /* blocks of block_k steps in which a sample rebased its delta (and the start kernel's) */
   uint64_t credited;     /* sum of reported iterations over non-cardioid samples */
   double ms_start;       /* start kernel, ms (HIP events), mean over repeats */
   double ms_iterate;     /* iteration kernel, ms, mean over repeats */
@@ -60,13 +60,13 @@ typedef struct nm_render_stats {
   int32_t waves_per_simd; /* persistent waves per SIMD used (series path: at most 4) */
   uint64_t executed_start; /* of executed: steps run inside the start kernel */
   double ms_compact;     /* tile scan + scatter of the active list, ms */
-  double ms_finalize;    /* smoothing / output kernel, ms */
+  double ms_finalize;    /* tiled sample orders: results into the row-major grids, ms */
   int32_t graph;         /* 1: ms_total is the mean of HIP graph replays of the pass */
   int32_t tile;          /* sample order used: 0 row-major, T = T x T tiles */
   int32_t fma2;          /* plain path: 1 when y' = (2x) y + c ran as fma(x y, 2, c), bit-identical for frames
                             whose coordinates are 0 or at least 2^-200 in magnitude */
-  int32_t grouped;       /* plain path: 1 when the escape test ran once per group of four updates, the first
-                            escaping update found from the group's earlier |z|^2 (bailout radius 2 to 2^30 and
+  int32_t grouped;       /* plain path: 1 when the escape test ran once per group of 4 or 16 updates and the first
+                            escaping update was found in the group afterwards (bailout radius 2 to 2^30 and
                             every |c| <= 0.999 (R^2 - R): an escape at one update implies one at the next) */
   int32_t chunk_run;     /* the iterate kernel's chunk order used: 64 = 64 consecutive samples of the active
                             list per chunk, R < 64 = runs of R (nm_launch.chunk_run; the plain path: 1) */
@@ -174,7 +174,7 @@ int nm_get_reference(const nm_mandelbrot* h, double* X, double* A, double* B, do
 int nm_get_reference_tables(const nm_mandelbrot* h, double* Xlo, double* m, int32_t* e);
 /* render every row with explicit engine settings and `repeats` timed launches;
  * copy_back = 0 leaves the grid on the device (benchmarks).  block_k: 0 for the
- * default (plain 64; series FP64 64, FP32X 8), else plain 8/16/32/64, series
+ * default (plain 64; series FP64 32, on a floatexp series 64; FP32X 8), else plain 8/16/32/64, series
  * FP64 8/12/16/32/64, FP32X 8/12/16/32; other values give NM_ERR_ARG. */
 int nm_render(nm_mandelbrot* h, int block_k, int waves_per_simd, int repeats, int copy_back,
               nm_render_stats* stats);

@@ -181,12 +181,12 @@ struct RenderStats {
   double ms_start = 0;       // classification / series start kernel
   double ms_compact = 0;     // tile scan + scatter
   double ms_iterate = 0;     // iteration kernel
-  double ms_finalize = 0;    // smoothing / output kernel
+  double ms_finalize = 0;    // tiled sample orders: results into the row-major grids
   double ms_total = 0;       // all of one pass; every time is a mean over repeats
   int graph = 0;             // 1: ms_total is the mean of HIP graph replays
   int tile = 0;              // the sample order used
   int fma2 = 0;              // plain path: the folded update ran (plain_update)
-  int grouped = 0;           // plain path: updates were tested in groups of four (grouped_test_ok)
+  int grouped = 0;           // plain path: updates were tested in groups (grouped_test_ok)
   int chunk_run = 0;         // the iterate kernel's chunk order used: 64 consecutive samples, or runs of R
   int block_k = 0, waves_per_simd = 0;
 };

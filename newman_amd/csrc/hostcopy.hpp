@@ -34,14 +34,16 @@ namespace nm {
 class HostCopy {
  public:
   static constexpr size_t kRing = (size_t)32 << 20;
-  // Up to here the runtime's copy.  Whole calls that return 1.2 MB into memory in use
-  // or a fresh array: 153 and 403 us with it, 135 and 191 with the ring; 2.8 MB 233
-  // and 711, 178 and 319; 6.2 MB 425 and 930, 295 and 500.
+  // Up to here the runtime's copy.  Whole calls that return 0.5 MB into memory in use:
+  // 100 us with it, 106 with the ring; 0.75 MB 112 and 116; 1 MB 137 and 125.  1.2 MB
+  // into memory in use or a fresh array: 153 and 403, 135 and 191; 2.8 MB 233 and 711,
+  // 178 and 319; 6.2 MB 425 and 930, 295 and 500.
   static constexpr size_t kDirect = (size_t)1 << 20;
   static constexpr int kHelpers = 3;
   // What a thread takes at a time (128 KB of 512 KB chunks: 217 and 549 us); a large
   // result, whose fresh pages come 2 MB at a time, goes by whole chunks (41 MB: 1.80 ->
-  // 1.53 ms a call).
+  // 1.53 ms a call; into memory in use 48 MB 1.70 -> 1.41, 24 MB 0.90 -> 0.80, 16 MB
+  // 0.64 -> 0.57, 8 MB 0.37 either way, 4 MB 0.24 -> 0.27: the line could be lower).
   static constexpr size_t kPiece = (size_t)256 << 10;
 
   // dst[0, bytes) = src (device), after the stream's earlier work; returns when the

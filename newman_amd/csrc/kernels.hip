@@ -114,7 +114,7 @@ struct Common {
   const uint32_t* nactive;  // written by the scan
   unsigned long long* part;
   int N;
-  double b2, b2m, log_b;
+  double b2, log_b;
   double smooth_k;  // 0.5 ln 2 / ln(bailout), or 0 for a bailout below 2
 };
 
@@ -695,9 +695,13 @@ __global__ __launch_bounds__(kThreads) void k_plain_start(PlainArgs a) {
 // The plain pass of a small frame set in one launch, a wave per 64 consecutive samples:
 // up to kDirectSamples a SIMD has a wave or two, the pass takes as long as its longest
 // sample in any case, and handing samples on, compacting and refilling only add launches
-// to that.  Renders of 160x120 at N 256 / 1024 of the whole set 58 -> 47 / 70 -> 60 us,
-// N 2048 of the period-3 island 84 -> 76; 420x300 (two waves a SIMD) 57 -> 51, 70 -> 72
-// and 112 -> 100 us; at 640x480 the waves that wait for their longest sample cost more.
+// to that.  Whole calls with the usual kernels and with this one, at N 256 / 2048 / 8192:
+// 160x120 of the whole set 57 -> 43, 83 -> 72, 173 -> 170 us; 327x300 84 -> 71, 110 ->
+// 100, 201 -> 200 (of the valley 90 -> 74, 136 -> 120, 293 -> 280).  With two waves on
+// every SIMD a wave that is nearly done holds up another: 512x256 of the whole set 105 ->
+// 94, but 132 -> 142 and 223 -> 301 (of the valley 114 -> 95, 160 -> 143, 318 -> 303; of
+// the island 111 -> 95, 159 -> 142, 315 -> 302), so the line is there, where most views
+// still gain; at 640x480 the waves that wait for their longest sample cost more.
 constexpr uint32_t kDirectSamples = 1u << 17;
 template <bool FMA2, bool GROUPED>
 __global__ __launch_bounds__(64) void k_plain_direct(PlainArgs a) {
@@ -965,8 +969,8 @@ __device__ __forceinline__ void retire_push(const Common& c, RetireEntry* q, int
 
 // Chunk claims: persistent waves take chunks of the active list dynamically.
 // The chunks are split into kQueues equal ranges with one claim counter each
-// (each counter on its own 256-byte line; zeroed with the partial counters at
-// the start of a pass).  A wave claims from its home range (its workgroup's
+// (each counter on its own 256-byte line; the start launch's first workgroup clears
+// them).  A wave claims from its home range (its workgroup's
 // index mod kQueues: consecutive workgroups land on different XCDs) and, once
 // that is empty, from the others in turn.  Waves on a SIMD do not progress at
 // one rate (the issue arbiter prefers older waves), so with a static chunk list
@@ -1437,7 +1441,7 @@ __device__ __forceinline__ double2 sa_term_fx(const SeriesArgs& a, int i, double
 // index whose threshold T_j = log2(tol |B_j|^2 / |C_j|^2) lies more than kMarg
 // above log2 |e|^2 is stable (T_j = -inf where B_j = 0 and C_j != 0: unstable;
 // +inf where C_j = 0: stable); only the indices at or below that line are tested,
-// in order, found on the prefix minimum and then on the sparse table.
+// in order, found on the prefix minimum and then on the minimum tree.
 __device__ int sa_stop_index_fx(const SeriesArgs& a, double L, int2 br, const EpsFx& p) {
   const int last = a.len - 1;
   if (last < 1 || L == -INFINITY) return 0;  // e = 0: the test never fires
@@ -2578,7 +2582,9 @@ class EngineImpl : public Engine {
     if (off <= kRefStage) {
       // a short reference in one copy, by way of pinned memory: 16 copies of its tables
       // took some 10 us each (a 204x156 image of a view of length 2900 that alternates
-      // with another 368 -> 267 us, of length 20000 444 -> 337)
+      // with another 368 -> 267 us, of length 20000 444 -> 337).  The line is where the
+      // buffer is still small: of length 40000 (6.8 MB) one copy would be 355 us for
+      // 393, at 80000 (13.6 MB) it is behind, 2.7 ms for 2.6
       if (!h_ref) NM_HIP(hipHostMalloc((void**)&h_ref, kRefStage, hipHostMallocDefault));
       NM_HIP(hipStreamSynchronize(stream));  // an earlier copy out of it is over
       for (const Piece& p : pieces)
@@ -2716,7 +2722,6 @@ class EngineImpl : public Engine {
     c.part = d_part;
     c.N = opt.N;
     c.b2 = opt.bailout * opt.bailout;
-    c.b2m = c.b2 * (1.0 - 1.0 / 1099511627776.0);
     c.log_b = std::log(opt.bailout);
     c.smooth_k = opt.bailout >= 2.0 ? 0.5 * std::log(2.0) / c.log_b : 0.0;
     return NM_OK;
@@ -3315,7 +3320,7 @@ Engine* Engine::running() {
 // render_hw_noalloc: the plain path (getIterationsHW, mandelbrot.cpp:231-254) of
 // one frame with every device buffer carved from `scratch`, a file-scope device
 // array: coordinate tables, the frame record, per-sample results, hand-on words,
-// states, |z|^2, the active list, tile counts and the counters.  It calls no
+// states, the active list, tile counts and the counters.  It calls no
 // hipMalloc/hipFree, creates no stream or event (the null stream) and touches no
 // engine buffer, for callers that cannot allocate device memory.  Each device
 // holds its own copy of the array; its address comes from hipGetSymbolAddress
@@ -3336,7 +3341,7 @@ constexpr size_t na_bytes(uint64_t n, uint64_t nr, uint64_t nc) {
          na_align((size_t)kPartWords * sizeof(unsigned long long)) + na_align(4);
 }
 constexpr size_t kNoAllocScratchBytes =
-    na_bytes(kNoAllocMaxSamples, kNoAllocMaxSide, kNoAllocMaxSide);  // about 29 MiB
+    na_bytes(kNoAllocMaxSamples, kNoAllocMaxSide, kNoAllocMaxSide);  // about 23 MiB
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 
 struct NoAllocDevice {
@@ -3399,7 +3404,7 @@ int render_hw_noalloc(const HwFrameHost& f, int N, double bailout, EscapeValue* 
   NoAllocDevice* d = nullptr;
   int st = noalloc_setup(dev, &d, err);
   if (st != NM_OK) return st;
-  // the layout: tables, frame, out, r2, state, hand-on words, tile counts, active,
+  // the layout: tables, frame, out, state, hand-on words, tile counts, active,
   // counters, active count
   char* b = (char*)d->ptr;
   size_t off = 0;
@@ -3454,7 +3459,6 @@ int render_hw_noalloc(const HwFrameHost& f, int N, double bailout, EscapeValue* 
   c.part = part;
   c.N = N;
   c.b2 = bailout * bailout;
-  c.b2m = c.b2 * (1.0 - 1.0 / 1099511627776.0);
   c.log_b = std::log(bailout);
   c.smooth_k = bailout >= 2.0 ? 0.5 * std::log(2.0) / c.log_b : 0.0;
   a.pre_iter = kPreIterDefault;

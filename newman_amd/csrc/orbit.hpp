@@ -11,6 +11,8 @@ namespace nm {
 class OrbitTables {
  public:
   static constexpr int kMaxLimbs = 16;
+  // a precompute of length 512 takes 1.34 ms with the host's tables and 1.03 with these,
+  // 1024 2.69 and 1.43; 256 0.67 and 0.80 (4 limbs)
   static constexpr int kMinLen = 1024;
   // Zd and Xlo of r, and with `series` A .. Ce, for the orbit x (2 (len + 1) values of
   // L limbs, real and imaginary parts in turn).  False where the host has to make

@@ -90,7 +90,9 @@ constexpr int kCountsPerTile = kThreads / 64;
 __host__ __device__ inline uint32_t start_counts(uint32_t total) { return start_tiles(total) * kCountsPerTile; }
 __host__ __device__ inline uint32_t count_index(uint32_t tile, uint32_t wave) { return tile * kCountsPerTile + wave; }
 // up to this many tiles (1 M samples) the scatter's waves sum the earlier tiles'
-// counts themselves, and no scan is launched
+// counts themselves, and no scan is launched: with it 44, 51 and 54 us a pass at 300,
+// 1000 and 1500 tiles of the whole set, with the scan's launches 46, 51 and 53 (4096
+// tiles: 79 and 69)
 constexpr uint32_t kSelfScanTiles = 1024;
 // k_scatter: the active-list position of bit l of word k of a tile, given the
 // tile's offset (the exclusive scan of the tile counts) and the set bits of the
