@@ -57,7 +57,7 @@ typedef struct nm_render_stats {
   double ms_iterate;     /* iteration kernel, ms, mean over repeats */
   double ms_total;       /* all kernels of one pass, ms, mean over repeats */
   int32_t block_k;       /* iterations per block used */
-  int32_t waves_per_simd; /* persistent waves per SIMD used (series path: at most 4) */
+  int32_t waves_per_simd; /* persistent waves per SIMD used (series path: at most 4, or 6 for FP32X on many samples) */
   uint64_t executed_start; /* of executed: steps run inside the start kernel */
   double ms_compact;     /* tile scan + scatter of the active list, ms */
   double ms_finalize;    /* tiled sample orders: results into the row-major grids, ms */
@@ -186,7 +186,7 @@ int nm_render_frames(nm_mandelbrot* h, const char* const* widths, int nframes, i
                      int repeats, nm_escape_value* out, nm_render_stats* stats);
 /* extension: launch settings of later renders on h.  0 keeps the engine's
  * default; waves_per_simd above 4 is 4 on the series path, where one workgroup of 16
- * waves fills a CU; pre_iter must be 0 or 1..1024; tile = sample order (0 row-major, or T x T tiles of 8 x 8 blocks, T in
+ * waves fills a CU (6 for FP32X deltas on 4 M samples and more); pre_iter must be 0 or 1..1024; tile = sample order (0 row-major, or T x T tiles of 8 x 8 blocks, T in
  * 8..256, a power of two); graph = 1 replays repeated passes from one captured
  * HIP graph; ms = the kernel time the autotuner measured (output only). */
 typedef struct nm_launch {

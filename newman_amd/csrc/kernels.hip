@@ -81,17 +81,21 @@ constexpr int kHead = 64;               // orbit padding past its end (>= max K)
 // orbit windows each iterate workgroup keeps in LDS: the head (where rebased
 // lanes live) and the tail (where samples that have not rebased yet run out the
 // reference); lanes whose block fits a window read it from LDS, the others
-// gather from global memory, whose cache tag lookups bound the gathers
-constexpr int kLdsTail = 512, kLdsHead = 7648;
-// The series iterate kernel runs up to 16 waves per workgroup, all that a CU holds by
-// default (4 per SIMD), over one copy of the windows that fills its LDS: on the 1e-100
-// view 4.78 ms against 5.00 of two workgroups with 1024 + 3040 entries each (4.84 with
-// a tail of 1024, 4.83 of 2048), the 1e-30, 1e-40 and 1e-200 views the same.  More
-// waves over smaller windows: 6 per SIMD 1.88 against 2.00 ms at 1e-30, but 5.98 ms
-// at 1e-100.
-constexpr int kSeriesWaves = 4;  // per SIMD: all that such a workgroup holds
-constexpr int kSeriesIterThreads = 256 * kSeriesWaves;
-static_assert(kLdsTail >= 64 && kLdsHead >= 64, "a block of up to 64 steps reads inside one window");
+// gather from global memory, whose cache tag lookups bound the gathers.
+// WIDE: up to 16 waves per workgroup, all that a CU holds by default (4 per SIMD), over
+// one copy of the windows that fills its LDS: on the 1e-100 view 4.78 ms against 5.00
+// of two workgroups with 1024 + 3040 entries each (4.84 with a tail of 1024, 4.83 of
+// 2048), the 1e-30, 1e-40 and 1e-200 views the same.  More waves over smaller windows:
+// 6 per SIMD 1.88 against 2.00 ms at 1e-30, but 5.98 ms at 1e-100.
+// Not WIDE: three workgroups of 8 waves (6 per SIMD, as many as an FP32X lane's
+// registers allow) over smaller windows, for FP32X on many samples (kManySamples).
+template <bool WIDE>
+struct SeriesShape {
+  static constexpr int kWaves = WIDE ? 4 : 6;  // per SIMD: all that a CU holds
+  static constexpr int kThreads = WIDE ? 1024 : 512;
+  static constexpr int kTail = WIDE ? 512 : 256, kHead = WIDE ? 7648 : 2048;
+  static_assert(kTail >= 64 && kHead >= 64, "a block of up to 64 steps reads inside one window");
+};
 constexpr int kPartSlots = 6144;        // per-workgroup partial counter slots
 
 constexpr int kQueueStride = 64;  // u32 between claim counters (ChunkClaim): 256 bytes
@@ -170,6 +174,7 @@ struct SeriesArgs {
   const int2 *Ae, *Be, *Ce;
   int fxs;
   uint32_t run_shift;  // active-list chunks (ChunkMap): runs of 2^run_shift entries
+  int iter_threads;    // of an iterate workgroup at most (SeriesShape)
   int fx_runs;         // FP32X: blocks between refills (together at most 64 steps)
   double* safe;        // safe radius per orbit index (safe_radius); null: no coherent phase (FP32X deltas)
   double emax, radius;  // what the radii hold for: |e| of every sample, the bailout
@@ -2070,15 +2075,16 @@ __device__ __forceinline__ void pert_block_fx(float& wr, float& wi, int& ex, flo
 // base address is a literal (from a register it was one of 64 spilled ones, +18% time on
 // the 1e-30 view).  The head sits above 16 K positions so that a rebased lane's
 // base address (head - 16 j) stays non-negative.
+template <bool WIDE>
 struct SeriesLds {
-  RetireEntry retire[kSeriesIterThreads / 64][kRetireCap];
-  double2 tail[kLdsTail];
-  double2 head[kLdsHead];
+  RetireEntry retire[SeriesShape<WIDE>::kThreads / 64][kRetireCap];
+  double2 tail[SeriesShape<WIDE>::kTail];
+  double2 head[SeriesShape<WIDE>::kHead];
 };
-static_assert(sizeof(SeriesLds) + 256 <= 160 * 1024, "one workgroup per CU");
-template <int K, bool FX>
-__global__ __launch_bounds__(kSeriesIterThreads) __attribute__((amdgpu_waves_per_eu(4, 8)))
-void k_series_iterate(SeriesArgs a) {
+static_assert(sizeof(SeriesLds<true>) + 256 <= 160 * 1024, "one workgroup per CU");
+static_assert(3 * (sizeof(SeriesLds<false>) + 256) <= 160 * 1024, "three workgroups per CU");
+template <int K, bool FX, bool WIDE>
+__device__ __forceinline__ void series_iterate(const SeriesArgs& a) {
   const int runs = FX ? a.fx_runs : 1, KB = K * runs;  // the steps between refills
   const Common& c = a.c;
   const uint32_t total = *c.nactive;
@@ -2093,7 +2099,8 @@ void k_series_iterate(SeriesArgs a) {
     return;
   }
   // entries past Zd's allocation read 0
-  __shared__ SeriesLds lds;
+  constexpr int kLdsTail = SeriesShape<WIDE>::kTail, kLdsHead = SeriesShape<WIDE>::kHead;
+  __shared__ SeriesLds<WIDE> lds;
   RetireEntry* const rq = lds.retire[threadIdx.x >> 6];
   double2* const zlds = lds.tail;
   int rn = 0;
@@ -2252,6 +2259,18 @@ void k_series_iterate(SeriesArgs a) {
   const int idx[3] = {C_EXECUTED, C_REBASED, C_CREDITED};
   block_partial(c.part, kSlotIter + blockIdx.x, v, idx, 3);
 }
+template <int K, bool FX>
+__global__ __launch_bounds__(SeriesShape<true>::kThreads) __attribute__((amdgpu_waves_per_eu(4, 8)))
+void k_series_iterate(SeriesArgs a) {
+  series_iterate<K, FX, true>(a);
+}
+// FP32X on many samples: a lane's 28 instructions a step in chains of single precision
+// leave 4 waves a SIMD waiting for themselves, where most samples have few steps left.
+template <int K>
+__global__ __launch_bounds__(SeriesShape<false>::kThreads) __attribute__((amdgpu_waves_per_eu(6, 8)))
+void k_series_iterate_many(SeriesArgs a) {
+  series_iterate<K, true, false>(a);
+}
 
 // tiled sample order: results (sample order) -> the row-major grids
 __global__ __launch_bounds__(kThreads) void k_emit(Common c, EscapeValue* grid) {
@@ -2337,13 +2356,9 @@ __global__ void k_clear(double* p, int n) {
     if (e_ != hipSuccess) return fail(#expr, e_); \
   } while (0)
 
-// threads per workgroup of a path's iterate kernel
-// threads of an iterate workgroup; the series kernel's, one per CU, takes all of the
-// CU's waves
-template <class A>
-int iter_threads(int) { return kThreads; }
-template <>
-int iter_threads<SeriesArgs>(int waves) { return std::min(kSeriesIterThreads, 256 * std::max(1, waves)); }
+// threads of an iterate workgroup; the series kernel's large one takes all of a CU's waves
+static int iter_threads(const PlainArgs&, int) { return kThreads; }
+static int iter_threads(const SeriesArgs& a, int waves) { return std::min(a.iter_threads, 256 * std::max(1, waves)); }
 
 // workgroups of an iterate launch of `ti` threads: `waves` per SIMD
 static int iterate_grid(int num_cu, int waves, int ti) {
@@ -2380,7 +2395,7 @@ static hipError_t launch_pass_on(hipStream_t stream, int num_cu, unsigned long l
   const Common& c = args.c;
   const int gtile = tile_grid(c.total, num_cu);
   // waves = persistent waves per SIMD: 4 per CU for each 256 threads
-  const int ti = iter_threads<Args>(waves);
+  const int ti = iter_threads(args, waves);
   const int giter = iterate_grid(num_cu, waves, ti);
   hipError_t e;
 #define NM_LAUNCH_OK(expr)                   \
@@ -2697,6 +2712,8 @@ class EngineImpl : public Engine {
 
   // sample ids and the plain iterate kernel's chunk positions (ChunkMap) stay below 2^32
   static bool in_range(uint64_t total) { return total > 0 && total < 0xFFFFF000ull; }
+  static constexpr uint64_t kManySamples = (uint64_t)4 << 20;  // see render_sa
+  static constexpr int kManyOrbitMin = 4096, kManyOrbitMax = 65536;
   // the series kernels' block sizes (an FP32X mantissa is renormalised at block ends)
   static bool series_block(int K, bool fx) { return K == 8 || K == 12 || K == 16 || K == 32 || (K == 64 && !fx); }
 
@@ -2793,7 +2810,7 @@ class EngineImpl : public Engine {
     if (st == NM_OK) {
       hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(kReduceThreads), 0, stream, (const unsigned long long*)d_part,
                          dgrid ? dgrid : tile_grid(args.c.total, num_cu),
-                         dgrid ? 0 : iterate_grid(num_cu, waves, iter_threads<Args>(waves)),
+                         dgrid ? 0 : iterate_grid(num_cu, waves, iter_threads(args, waves)),
                          (const uint32_t*)d_nactive, h_totals);
       ce = hipGetLastError();
       if (ce == hipSuccess && host_out)
@@ -3064,19 +3081,32 @@ class EngineImpl : public Engine {
     // counts: 64 (5.27 -> 4.97 ms at 1e-100).  FP32X blocks renormalise their
     // mantissa at block ends, so they stay short
     const int K = opt.block_k > 0 ? opt.block_k : fx ? 8 : a.fxs ? 64 : 32;
+    // FP32X on many samples: see k_series_iterate_many.  Whole passes with one workgroup
+    // per CU and with three: 7680x4320 of the 1e-30 view 5.84 -> 5.15 ms (5.32 before the
+    // one workgroup), of 1e-40 7.58 -> 7.10, of 1e-200 17.3 -> 16.1; 3840x2160 of 1e-30
+    // 1.73 -> 1.59, of 1e-25 0.95 -> 0.94.  Fewer samples do not fill as many waves: at
+    // 2560x1440 1e-30 0.90 and 0.86, but 1e-25 0.46 and 0.48.  An orbit of 3000 entries is
+    // all in the large window, 7.0 and 7.4 ms at 7680x4320, and along one of 100,000 the
+    // samples run thousands of steps near its head, 20.1 and 20.8 at 3840x2160
+    const bool many = fx && total >= kManySamples && ref_len > kManyOrbitMin && ref_len <= kManyOrbitMax;
     // FP32X takes several of its short blocks between refills, as the refill and its
     // bookkeeping are 240 instructions: one / 32 steps / 64 steps of them 1.09 / 0.93 /
     // 0.89 ms on the 1279x719 frame of the 1e-200 view, 0.47 / 0.43 / 0.44 ms on
-    // 1600x900 of the 1e-30 view, 0.112 / 0.111 / 0.119 ms on 700x500 at 1e-25
-    a.fx_runs = fx ? std::max(1, (a.fxs ? 64 : 32) / K) : 1;
+    // 1600x900 of the 1e-30 view, 0.112 / 0.111 / 0.119 ms on 700x500 at 1e-25; on many
+    // samples 32 / 48 / 64 steps 5.09 / 5.04 / 5.33 ms at 1e-30, 7.28 / 7.04 / 6.73 at
+    // 1e-40, 16.1 / 15.7 / 15.6 at 1e-200
+    a.fx_runs = fx ? std::max(1, (many ? 48 : a.fxs ? 64 : 32) / K) : 1;
     // 4 persistent waves per SIMD: the workgroup whose queues and windows fill a CU's
     // LDS; fewer hide too little latency:
     // 2 waves 2.8-3.0 against 2.0 ms on the 1e-30 view, 1.29 against 0.91 ms on 16
     // frames of the 1e-40 video.  FP32X ran 8 with smaller windows: 1.18 -> 1.07 ms
     // on the 1279x719 frame of the 1e-200 view.  More waves would be workgroups that
     // hold their first chunks back until a CU is free (8 and 16 waves 1.34 and 2.06 ms
-    // a pass of that frame against 0.88), so a larger setting is taken as 4
-    const int waves = opt.waves_per_simd > 0 ? std::min(opt.waves_per_simd, kSeriesWaves) : kSeriesWaves;
+    // a pass of that frame against 0.88), so a larger setting is taken as the most that
+    // a CU holds
+    const int most = many ? SeriesShape<false>::kWaves : SeriesShape<true>::kWaves;
+    a.iter_threads = many ? SeriesShape<false>::kThreads : SeriesShape<true>::kThreads;
+    const int waves = opt.waves_per_simd > 0 ? std::min(opt.waves_per_simd, most) : most;
     if (stats) {
       stats->block_k = K;
       stats->waves_per_simd = waves;
@@ -3097,10 +3127,13 @@ class EngineImpl : public Engine {
                    : run(a, k_series_start<false, true>, iter, waves, opt, stats, nout, host_out, emit_to);
     };
     switch (K) {
-      case 8: return fx ? go(k_series_iterate<8, true>) : go(k_series_iterate<8, false>);
-      case 12: return fx ? go(k_series_iterate<12, true>) : go(k_series_iterate<12, false>);
-      case 16: return fx ? go(k_series_iterate<16, true>) : go(k_series_iterate<16, false>);
-      case 32: return fx ? go(k_series_iterate<32, true>) : go(k_series_iterate<32, false>);
+#define NM_SERIES(KK) \
+  return many ? go(k_series_iterate_many<KK>) : fx ? go(k_series_iterate<KK, true>) : go(k_series_iterate<KK, false>)
+      case 8: NM_SERIES(8);
+      case 12: NM_SERIES(12);
+      case 16: NM_SERIES(16);
+      case 32: NM_SERIES(32);
+#undef NM_SERIES
       default: return go(k_series_iterate<64, false>);  // 64: FP64 only (series_block)
     }
   }
