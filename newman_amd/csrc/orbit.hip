@@ -207,6 +207,13 @@ bool OrbitTables::go(void* stream, const HpVal* x, int len, int L, bool series, 
   if (!room(off)) return false;
   V* dx = (V*)(buf_ + ox);
   std::vector<V> hx(count + 2);
+  std::vector<uint16_t> run;
+  std::vector<int32_t> gap;
+  // also where a table's allocation throws: the copies out of and into them are over first
+  struct Wait {
+    hipStream_t s;
+    ~Wait() { (void)hipStreamSynchronize(s); }
+  } wait{s};
   for (size_t k = 0; k < count + 2; k++) hx[k] = hpd_load<ML>(x[k]);
   bool ok = hipMemcpyAsync(dx, hx.data(), hx.size() * sizeof(V), hipMemcpyHostToDevice, s) == hipSuccess;
   hipLaunchKernelGGL(k_orbit<ML>, dim3((unsigned)((count + 2 + 63) / 64)), dim3(64), 0, s, (const V*)dx, len, L,
@@ -242,8 +249,6 @@ bool OrbitTables::go(void* stream, const HpVal* x, int len, int L, bool series, 
   };
   fetch(r.Zd, oz, count + 4);
   fetch(r.Xlo, ol, count);
-  std::vector<uint16_t> run;
-  std::vector<int32_t> gap;
   if (series) {
     std::vector<double>*fd[3] = {&r.A, &r.B, &r.C}, *fm[3] = {&r.Am, &r.Bm, &r.Cm};
     std::vector<int32_t>* fe[3] = {&r.Ae, &r.Be, &r.Ce};
