@@ -14,9 +14,10 @@
 // bounds it is the latency of that arithmetic (carries run through a lane's limbs),
 // with a few waves in flight.  The orbit in doubles, a lane per value, took the host
 // another 5 ms each for the screening's orbit and the reference's.  precompute() with
-// the host's tables and with these (orbit lengths 2900, 8000, 20000, 100000 at 3, 4, 4
-// and 8 limbs): 13.5 -> 7.1, 38.3 -> 15.6, 89.5 -> 35.7, 598 -> 233 ms, most of what
-// is left the host's chain of the orbit itself.
+// the host's tables and with these (orbit lengths 3000, 8000, 20000, 100000 at 3, 4, 4
+// and 8 limbs): 13.1 -> 6.9, 35.5 -> 15.9, 86.1 -> 37.7, 598 -> 237 ms (0.1, 0.2, 0.5
+// and 2.8 ms of them the bound below), most of what is left the host's chain of the
+// orbit itself.
 //
 // A chunk's first value comes by another order of operations than the host's chain, so
 // its last bits differ (the first chunk's do not).  What is kept of a value is its

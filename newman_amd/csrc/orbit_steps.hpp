@@ -96,7 +96,7 @@ __host__ __device__ __forceinline__ uint16_t hpd_run(const hpd<ML>& v, int L) {
 // assumption about the orbit is left.  real: the orbit lies on the real axis and every
 // imaginary part is an exact zero.  Zd: the orbit as the kernels read it (Zd[i + 1] = x_i).
 // trace (a check's): 3 len values, D of every index as far as the bound does.
-// It is 0.2 ms of one host thread for a length of 8000.
+// It is 0.2 ms of one host thread for a length of 8000, 2.8 for 100,000.
 inline bool orbit_tables_hold(const double* Zd, int len, int L, int chunk, bool real, const int32_t* const (&ex)[3],
                               const uint16_t* const (&run)[3], const int32_t* const (&gap)[3],
                               double* trace = nullptr) {
